@@ -109,7 +109,7 @@ void k_batch(const FwdArgs *items,
                                               const int *modes,
                                               const int64_t *off,
                                               int64_t nitems, int64_t total) {
-  __shared__ FwdSmem<WG, CAP, false, TA, TI> sm;
+  __shared__ FwdSmem<WG, CAP, TA> sm;
   const int64_t per_xcd = (total + kXcds - 1) / kXcds;
   const int64_t xcd = blockIdx.x % kXcds;
   const int64_t lw = blockIdx.x / kXcds, nw = gridDim.x / kXcds;

@@ -229,10 +229,6 @@ __device__ __forceinline__ int64_t row_begin(const TI *rowptr, int64_t base,
   return nnz;
 }
 
-// Top bit of a column panel's row-map entry: the segment is its row's first
-// in panel order (row ids are non-negative, so the bit is free).
-template <typename TI> constexpr TI kFirstSeg = static_cast<TI>(TI(1) << (sizeof(TI) * 8 - 1));
-
 // Entries a block's window leaves free: a window of W entries holds at most
 // W - kWinSlack of the block's entries, so that lanes streaming groups of up
 // to kWinSlack consecutive entries from the group-aligned entry below the

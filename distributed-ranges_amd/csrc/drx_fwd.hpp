@@ -28,9 +28,8 @@
 namespace drx {
 
 // Kernel modes: plain CSR; vals read through a permutation (the transposed
-// structure of the adjoint); rows written through a row map and accumulated
-// (one column panel of a panel-layout plan).
-enum FwdMode { kPlain = 0, kPerm = 1, kRowMap = 2 };
+// structure of the adjoint).
+enum FwdMode { kPlain = 0, kPerm = 1 };
 
 struct FwdArgs {
   const void *rowptr;
@@ -40,7 +39,6 @@ struct FwdArgs {
   int64_t nblocks, per_xcd, grid;
   const void *colind, *vals, *x;
   const void *perm;    // kPerm: vals[perm[e]]
-  const void *rowmap;  // kRowMap: output row of share row r
   int64_t ldx;
   uint32_t xbytes;   // bytes of one x column (buffer gathers)
   void *y;
@@ -53,21 +51,6 @@ struct FwdArgs {
   const void *xr;  // k >= 2: x in row-major chunks of KP columns
   int64_t ncols;   // columns of the share (rows of one xr chunk)
 };
-
-// Row-map entries of column panels carry in their top bit whether the
-// segment is its row's first in panel order. That segment writes
-// y = beta * y + alpha * sum (y not read when beta is 0); the row's later
-// segments add alpha * sum to it.
-template <typename TI> __device__ __forceinline__ int64_t map_row(TI m) {
-  return static_cast<int64_t>(m & static_cast<TI>(~kFirstSeg<TI>));
-}
-// y of a segment's row before its sum is added.
-template <typename TA, typename TY, typename TI>
-__device__ __forceinline__ TA map_ypre(const TY *yj, TI m, TA beta) {
-  const int64_t row = map_row(m);
-  if ((m & kFirstSeg<TI>) == 0) return to_acc<TA>(yj[row]);
-  return beta == TA(0) ? TA(0) : beta * to_acc<TA>(yj[row]);
-}
 
 template <int WG, typename TA>
 __device__ __forceinline__ TA block_sum(TA v, TA *red) {
@@ -85,14 +68,12 @@ __device__ __forceinline__ TA block_sum(TA v, TA *red) {
 // Rows [0, nr) of the block (row r0 + i), products prod[0 .. n_s), row
 // offsets in rp_s (relative to e0) or, for blocks with more rows than the
 // LDS holds, read from rowptr.
-template <int WG, int G, int MODE, typename TA, typename TY, typename TI>
+template <int WG, int G, typename TA, typename TY, typename TI>
 __device__ __forceinline__ void reduce_rows(const TA *prod, const int *rp_s,
-                                            const TI *map_s, const TA *ypre,
                                             bool rows_lds, const FwdArgs &a,
                                             int64_t r0, int64_t e0, int64_t nr,
                                             TY *yj, TA alpha, TA beta) {
   const TI *rowptr = static_cast<const TI *>(a.rowptr);
-  const TI *rowmap = static_cast<const TI *>(a.rowmap);
   const int lane = threadIdx.x & (G - 1);
   constexpr int NG = WG / G;
   for (int64_t i = threadIdx.x / G; i < nr; i += NG) {
@@ -108,32 +89,22 @@ __device__ __forceinline__ void reduce_rows(const TA *prod, const int *rp_s,
     for (int q = s + lane; q < e; q += G) acc += prod[q];
     acc = group_sum<G>(acc);
     if (lane == 0) {
-      if constexpr (MODE == kRowMap) {
-        if (ypre != nullptr && rows_lds) {
-          yj[map_row(map_s[i])] = from_acc<TY>(ypre[i] + alpha * acc);
-        } else {
-          const TI m = rowmap[r0 + i];
-          yj[map_row(m)] = from_acc<TY>(map_ypre<TA>(yj, m, beta) + alpha * acc);
-        }
-      } else {
-        TA out = alpha * acc;
-        if (beta != TA(0)) out += beta * to_acc<TA>(yj[r0 + i]);
-        yj[r0 + i] = from_acc<TY>(out);
-      }
+      TA out = alpha * acc;
+      if (beta != TA(0)) out += beta * to_acc<TA>(yj[r0 + i]);
+      yj[r0 + i] = from_acc<TY>(out);
     }
   }
 }
 
-template <int WG, int MODE, typename TA, typename TY, typename TI>
+template <int WG, typename TA, typename TY, typename TI>
 __device__ __forceinline__ void reduce_rows_any(int n_s, const TA *prod,
-                                                const int *rp_s, const TI *map_s,
-                                                const TA *ypre, bool rows_lds,
+                                                const int *rp_s, bool rows_lds,
                                                 const FwdArgs &a, int64_t r0,
                                                 int64_t e0, int64_t nr, TY *yj,
                                                 TA alpha, TA beta) {
   if (nr <= 0) return;
   const int64_t avg = (n_s / nr) >> a.gshift;
-#define DRX_RR(G) reduce_rows<WG, G, MODE, TA, TY, TI>(prod, rp_s, map_s, ypre, rows_lds, a, r0, e0, nr, yj, alpha, beta)
+#define DRX_RR(G) reduce_rows<WG, G, TA, TY, TI>(prod, rp_s, rows_lds, a, r0, e0, nr, yj, alpha, beta)
   if (avg <= 3)
     DRX_RR(1);
   else if (avg <= 6)
@@ -304,19 +275,16 @@ __device__ __forceinline__ TV long_val(const TV *vals, const TI *perm,
     return ld_stream(vals + q);
 }
 
-// LDS of one workgroup of the forward kernels (row-map entries have the
-// index type; RG: the window's column indices for row-ordered gathers).
-template <int WG, int CAP, bool ROWMAP, typename TA, typename TI, bool RG = false>
+// LDS of one workgroup of the forward kernels (RG: the window's column
+// indices for row-ordered gathers).
+template <int WG, int CAP, typename TA, bool RG = false>
 struct FwdSmem {
   // rows of a block held in LDS (blocks with more read rowptr); row-ordered
   // gathers serve shares of at least four entries per row on average
   static constexpr int ROWCAP = RG ? CAP / 4 : CAP / 2;
-  static constexpr int MAPCAP = ROWMAP ? ROWCAP : 1;
   TA prod[CAP];
   uint32_t cs[RG ? CAP : 0];  // empty unless RG (the other kernels keep their LDS)
-  TA ypre[MAPCAP];        // kRowMap, k = 1: the current y of the block's rows
   TA red[WG / 64];
-  TI map_s[MAPCAP];       // kRowMap: output rows of the block
   int rp_s[ROWCAP + 1];
   uint32_t xmm[2 * (WG / 64)];  // per-wave column min / max (x staging)
 };
@@ -332,8 +300,8 @@ template <typename TV, typename U> __device__ __forceinline__ TV bits_to(U u) {
 // One row block `blk` of the share described by `a` (all lanes of the
 // workgroup call it together).
 //
-// VW = 2 or 4 (32-bit indices, plain or row-map mode, VW values in at most
-// 16 bytes): each lane streams groups of VW consecutive entries, one 4 VW-
+// VW = 2 or 4 (32-bit indices, plain mode, VW values in at most 16
+// bytes): each lane streams groups of VW consecutive entries, one 4 VW-
 // byte colind load and one VW * sizeof(TV)-byte vals load per group, from the
 // group-aligned entry ea below the block's first entry e0 (the caller
 // guarantees vals / colind pointers aligned to a group). Slot s of the LDS
@@ -346,19 +314,17 @@ template <int WG, int CAP, int MODE, bool BUFX, typename TV, typename TX,
           typename TY, typename TA, typename TI, int VW = 1, bool XS = false,
           bool RG = false>
 __device__ __forceinline__ void process_block(const FwdArgs &a, int64_t blk,
-                                              FwdSmem<WG, CAP, MODE == kRowMap, TA, TI, RG> &sm) {
+                                              FwdSmem<WG, CAP, TA, RG> &sm) {
   static_assert(VW == 1 || ((VW == 2 || VW == 4) && MODE != kPerm && sizeof(TI) == 4 &&
                             VW * sizeof(TV) <= 16 && VW <= kWinSlack),
-                "groups of entries: plain or row-map mode, 32-bit indices, at most 16 bytes "
+                "groups of entries: plain mode, 32-bit indices, at most 16 bytes "
                 "of values per group");
   static_assert(!XS || (MODE == kPlain && BUFX), "x staging: plain mode, buffer gathers");
   static_assert(!RG || (MODE == kPlain && BUFX && !XS), "row gathers: plain mode, buffer gathers");
   constexpr int T = CAP / WG;
-  constexpr int ROWCAP = FwdSmem<WG, CAP, MODE == kRowMap, TA, TI, RG>::ROWCAP;
+  constexpr int ROWCAP = FwdSmem<WG, CAP, TA, RG>::ROWCAP;
   TA *prod = sm.prod;
   int *rp_s = sm.rp_s;
-  TI *map_s = sm.map_s;
-  TA *ypre = sm.ypre;
   TA *red = sm.red;
   const int tid = threadIdx.x;
   const TI *rowptr = static_cast<const TI *>(a.rowptr);
@@ -385,63 +351,6 @@ __device__ __forceinline__ void process_block(const FwdArgs &a, int64_t blk,
       else
         return (tid + (u / VW) * WG) * VW + (u % VW);
     };
-
-    constexpr bool kRowsFirst = MODE == kRowMap && sizeof(TV) == 4;
-    if (kRowsFirst && rows_lds) {
-      // Column panels of 4-byte values: row offsets, output rows and their
-      // current y, before
-      // the window is streamed so that their registers are free again. Every
-      // load of a lane is issued before the first LDS write, with indices
-      // clamped to valid rows: a per-row predicate around load and use made
-      // each wave wait for one load at a time, three dependent round trips
-      // per row slot, and panel blocks hold up to ROWCAP short rows.
-      // nr < ROWCAP, so NI slots per lane cover rows 0..nr. Headline Zipf
-      // FP32 panels: 10.31 -> 9.91 ms per step. (Plain blocks hold few rows
-      // per lane and keep the simple loop below: batching spilled the
-      // 4096-entry kernel. 16-bit panels keep it too: with it, their pair
-      // unpacking waited on each streamed load, 9.2 -> 10.6 ms.)
-      constexpr int NI = (ROWCAP + WG - 1) / WG;
-      const TI *rowmap = static_cast<const TI *>(a.rowmap);
-      TI raw[NI], row[NI];
-      TA yv[NI];
-      // Slots k with k * WG > nr hold no row of the block (a block-uniform
-      // test): they load nothing.
-#pragma unroll
-      for (int k = 0; k < NI; k++) {
-        if (k * WG > nr) break;
-        const int64_t i = tid + k * WG;
-        const int64_t r = b.r0 + (i <= nr ? i : nr);
-        // row_begin without its branch: rowptr[nrows] exists only with a
-        // sentinel; otherwise that row begins at nnz.
-        raw[k] = rowptr[r < a.nrows || a.sent ? r : r - 1];
-        row[k] = nr > 0 ? rowmap[b.r0 + (i < nr ? i : nr - 1)] : TI(0);
-      }
-      if (a.k == 1 && nr > 0) {
-#pragma unroll
-        for (int k = 0; k < NI; k++) {
-          if (k * WG > nr) break;
-          yv[k] = map_ypre<TA>(y, row[k], beta);
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < NI; k++) {
-        if (k * WG > nr) break;
-        const int i = tid + k * WG;
-        if (i <= nr) {
-          const int64_t r = b.r0 + i;
-          int64_t v0 = a.nnz;
-          if (r < a.nrows || a.sent) {
-            v0 = static_cast<int64_t>(raw[k]) - a.base;
-            v0 = v0 < 0 ? 0 : (v0 > a.nnz ? a.nnz : v0);
-          }
-          rp_s[i] = static_cast<int>(v0 - b.e0);
-        }
-        if (i < nr) {
-          map_s[i] = row[k];
-          if (a.k == 1) ypre[i] = yv[k];
-        }
-      }
-    }
 
     // Stream the window (reads past n_s return 0 and touch no memory).
     TA v[T];
@@ -501,17 +410,10 @@ __device__ __forceinline__ void process_block(const FwdArgs &a, int64_t blk,
         }
       }
     }
-    if (!kRowsFirst && rows_lds) {
+    if (rows_lds) {
       for (int i = tid; i <= nr; i += WG) {
         rp_s[i] = static_cast<int>(
             row_begin(rowptr, a.base, a.nrows, a.nnz, a.sent, b.r0 + i) - b.e0);
-        if constexpr (MODE == kRowMap) {
-          if (i < nr) {
-            const TI row = static_cast<const TI *>(a.rowmap)[b.r0 + i];
-            map_s[i] = row;
-            if (a.k == 1) ypre[i] = map_ypre<TA>(y, row, beta);
-          }
-        }
       }
     }
 
@@ -622,10 +524,8 @@ __device__ __forceinline__ void process_block(const FwdArgs &a, int64_t blk,
         }
       }
       __syncthreads();
-      reduce_rows_any<WG, MODE, TA, TY, TI>(n_s, prod + sh, rp_s, map_s,
-                                            MODE == kRowMap && a.k == 1 ? ypre : nullptr,
-                                            rows_lds, a, b.r0, b.e0,
-                                      nr, y + j * a.ldy, alpha, beta);
+      reduce_rows_any<WG, TA, TY, TI>(n_s, prod + sh, rp_s, rows_lds, a, b.r0, b.e0, nr,
+                                      y + j * a.ldy, alpha, beta);
       __syncthreads();
     }
 
@@ -657,15 +557,9 @@ __device__ __forceinline__ void process_block(const FwdArgs &a, int64_t blk,
                   to_acc<TA>(xj[static_cast<int64_t>(ld_stream(colind + q))]);
         const TA s = block_sum<WG>(acc0 + acc1, red);
         if (tid == 0) {
-          if constexpr (MODE == kRowMap) {
-            const TI m = static_cast<const TI *>(a.rowmap)[last];
-            TY *yj = y + j * a.ldy;
-            yj[map_row(m)] = from_acc<TY>(map_ypre<TA>(yj, m, beta) + alpha * s);
-          } else {
-            TA out = alpha * s;
-            if (beta != TA(0)) out += beta * to_acc<TA>(y[last + j * a.ldy]);
-            y[last + j * a.ldy] = from_acc<TY>(out);
-          }
+          TA out = alpha * s;
+          if (beta != TA(0)) out += beta * to_acc<TA>(y[last + j * a.ldy]);
+          y[last + j * a.ldy] = from_acc<TY>(out);
         }
       }
     }
@@ -679,7 +573,7 @@ __device__ __forceinline__ void process_block(const FwdArgs &a, int64_t blk,
 // workgroup spilled registers and lost 30 %.
 template <int WG, int CAP, int MODE, typename TA, typename TI, bool RG = false>
 constexpr int fwd_waves() {
-  constexpr int lds = static_cast<int>(sizeof(FwdSmem<WG, CAP, MODE == kRowMap, TA, TI, RG>));
+  constexpr int lds = static_cast<int>(sizeof(FwdSmem<WG, CAP, TA, RG>));
   constexpr int wgs = (160 * 1024) / lds;
   constexpr int w = wgs * (WG / 256);
   return w > 8 ? 8 : (w < 1 ? 1 : w);
@@ -698,14 +592,13 @@ template <int WG, int CAP, int MODE, bool BUFX, typename TV, typename TX,
 __global__ __launch_bounds__(WG)
 // (16-bit values in plain mode take one wave fewer: at the LDS-bound count
 // their pair unpacking spilled registers; 3-D Laplacian BF16 390 -> 371 us.
-// The panel kernel's LDS already holds it at 7 waves, where it does not.
 // Permuted values take one wave fewer too: their T unconditional value
 // loads spilled at 8; band +-16 FP32 adjoint 563 -> 471 us.)
 // (FP64 sums with 8 or more entries per lane run at most 6 waves: their
 // gathers in halves of four need the registers.)
 __attribute__((amdgpu_waves_per_eu(fwd_kernel_waves<WG, CAP, MODE, TV, TA, TI, RG>(), 8)))
 void k_spmv_fwd(FwdArgs a) {
-  __shared__ FwdSmem<WG, CAP, MODE == kRowMap, TA, TI, RG> sm;
+  __shared__ FwdSmem<WG, CAP, TA, RG> sm;
   for (int64_t wi = blockIdx.x; wi < a.per_xcd * kXcds; wi += a.grid) {
     const int64_t blk = map_block(wi, a.per_xcd);
     if (blk >= a.nblocks) continue;
@@ -1288,7 +1181,6 @@ template <int WG, int CAP, int KP, int MODE, typename TV, typename TX,
 __device__ __forceinline__ void process_block_mrhs(const FwdArgs &a,
                                                    int64_t blk,
                                                    MrhsSmem<WG, CAP, TA> &sm) {
-  static_assert(MODE == kPlain || MODE == kPerm, "row maps use k = 1 panels");
   constexpr int T = CAP / WG;
   constexpr int ROWCAP = CAP / 2;
   constexpr int NW = WG / 64;

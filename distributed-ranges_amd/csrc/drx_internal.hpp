@@ -105,6 +105,12 @@ int tuned_rowgather();
 // Stream-ordered scratch from the library's per-device pool.
 void *scratch_alloc(size_t bytes, hipStream_t s);
 void scratch_free(void *p, hipStream_t s);
+// An object whose products take `bytes` of scratch at once: scratch_reserve
+// brings the pool to that size (so that its first product does not pay for
+// it) until scratch_unreserve, which gives the pool's unused memory back down
+// to the largest reserve left.
+void scratch_reserve(int dev, size_t bytes, hipStream_t s);
+void scratch_unreserve(int dev, size_t bytes);
 
 // Row-major chunks of x for k >= 2 right-hand sides: chunk width KP and the
 // bytes of all chunks; the copy kernel.
@@ -149,13 +155,6 @@ void run_spmv_panels(const Plan &p, int vtype, const void *colind,
                      const void *vals, int xtype, const void *x, int64_t ldx,
                      int ytype, void *y, int64_t ldy, int64_t k, double alpha,
                      double beta, hipStream_t s);
-// One column panel: its segments add alpha * sum into y[row]; a row's first
-// segment (row-map top bit) writes beta * y + alpha * sum instead.
-void run_spmv_rowmap(const Plan &p, int vtype, const void *colind,
-                     const void *vals, const void *rowmap, int xtype,
-                     const void *x, int64_t ldx, int ytype, void *y,
-                     int64_t ldy, int64_t k, double alpha, double beta,
-                     hipStream_t s);
 void free_panels(PanelSet *ps);
 // A plan with panels is called with the colind/vals it was built from (or
 // last updated to); throws otherwise.

@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <set>
 
 #include "drx_common.hpp"
 #include "drx_fwd.hpp"
@@ -31,6 +32,7 @@ namespace drx {
 constexpr int kMaxDevices = 64;
 static std::mutex g_pool_mu;
 static hipMemPool_t g_pools[kMaxDevices];
+static std::multiset<size_t> g_reserved[kMaxDevices];
 
 static hipMemPool_t pool_for(int dev) {
   std::lock_guard<std::mutex> lk(g_pool_mu);
@@ -60,6 +62,23 @@ void *scratch_alloc(size_t bytes, hipStream_t s) {
 
 void scratch_free(void *p, hipStream_t s) {
   if (p) (void)hipFreeAsync(p, s);
+}
+
+void scratch_reserve(int dev, size_t bytes, hipStream_t s) {
+  void *p = scratch_alloc(bytes, s);
+  scratch_free(p, s);
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  g_reserved[dev].insert(bytes);
+}
+
+void scratch_unreserve(int dev, size_t bytes) {
+  constexpr size_t kKeep = size_t(256) << 20;  // small products' scratch
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  auto &r = g_reserved[dev];
+  const auto at = r.find(bytes);
+  if (at != r.end()) r.erase(at);
+  if (g_pools[dev])
+    (void)hipMemPoolTrimTo(g_pools[dev], std::max(kKeep, r.empty() ? size_t(0) : *r.rbegin()));
 }
 
 // Samples up to 4096 row blocks: the span between the first and the last

@@ -104,8 +104,7 @@ static bool launch_fwd_rg(int64_t cap, const FwdArgs &a, hipStream_t s) {
 // most 4 bytes, single entries for FP64; 1 single entries; 2 pairs; 4
 // groups of four, wherever eligible (else single entries). Measured with
 // every gather in flight (us per call): 3-D Laplacian 256^3 FP32 271 -> 222,
-// BF16 / FP16 234 / 260 -> 199, headline Zipf column panels 8.44 -> 8.12 ms
-// per step; band +-16 FP32 211 -> 212 (its gathers, coalesced across lanes
+// BF16 / FP16 234 / 260 -> 199; band +-16 FP32 211 -> 212 (its gathers, coalesced across lanes
 // with one entry per lane, spread over four times the lines with groups);
 // FP64 pairs (3-D Laplacian 403 -> 420) spill.
 template <int MODE, bool BUFX, typename TV, typename TX, typename TY,
@@ -235,14 +234,7 @@ static void launch_fwd(const Plan &p, FwdArgs a, hipStream_t s) {
 template <int MODE, typename TV, typename TX, typename TY, typename TA>
 static void launch_fwd_t(const Plan &p, const FwdArgs &a, bool bufx,
                          hipStream_t s) {
-  if constexpr (MODE == kRowMap) {
-    // panels exist only when x fits a buffer resource
-    if (p.itype == DRX_I32)
-      launch_fwd<MODE, true, TV, TX, TY, TA, int32_t>(p, a, s);
-    else
-      launch_fwd<MODE, true, TV, TX, TY, TA, int64_t>(p, a, s);
-    (void)bufx;
-  } else if (p.itype == DRX_I32) {
+  if (p.itype == DRX_I32) {
     if (bufx)
       launch_fwd<MODE, true, TV, TX, TY, TA, int32_t>(p, a, s);
     else
@@ -258,7 +250,7 @@ static void launch_fwd_t(const Plan &p, const FwdArgs &a, bool bufx,
 template <int MODE>
 static void run_spmv_impl(const Plan &p, int vtype, const void *colind,
                           const void *vals, const void *perm,
-                          const void *rowmap, int xtype,
+                          int xtype,
                           const void *x, int64_t ldx, int ytype, void *y,
                           int64_t ldy, int64_t k, double alpha, double beta,
                           hipStream_t s) {
@@ -283,7 +275,6 @@ static void run_spmv_impl(const Plan &p, int vtype, const void *colind,
   a.colind = colind;
   a.vals = vals;
   a.perm = perm;
-  a.rowmap = rowmap;
   a.x = x;
   a.ldx = ldx;
   a.y = y;
@@ -301,20 +292,18 @@ static void run_spmv_impl(const Plan &p, int vtype, const void *colind,
   // an empty range.
   a.xbytes = bufx && p.nnz > 0 ? static_cast<uint32_t>(xb) : 0;
   a.ncols = p.ncols;
-  if constexpr (MODE != kRowMap) {
-    // Row-major chunks of x for k >= 2, except up to 4 right-hand sides over
-    // short rows with local columns (stencils): their column gathers are
-    // already coalesced and the copy of x is large next to the matrix
-    // (2-D Laplacian FP64, k = 2 / 3 / 4: 3009 / 2891 / 2811 GB/s through
-    // column gathers vs 2151 / 2245 / 2572 through chunks; a +-16 band, 33
-    // entries per row, is faster through chunks at every k).
-    const int mr = p.no_scratch ? 0 : tuned_mrhs();
-    const bool stencil = k <= 4 && p.nnz <= 8 * p.nrows;
-    if (k >= 2 && mr != 0 &&
-        (mr == 2 || !stencil || (column_locality(p, colind, s) & 1) == 0)) {
-      run_mrhs(p, a, MODE, vtype, xtype, ytype, s);
-      return;
-    }
+  // Row-major chunks of x for k >= 2, except up to 4 right-hand sides over
+  // short rows with local columns (stencils): their column gathers are
+  // already coalesced and the copy of x is large next to the matrix
+  // (2-D Laplacian FP64, k = 2 / 3 / 4: 3009 / 2891 / 2811 GB/s through
+  // column gathers vs 2151 / 2245 / 2572 through chunks; a +-16 band, 33
+  // entries per row, is faster through chunks at every k).
+  const int mr = p.no_scratch ? 0 : tuned_mrhs();
+  const bool stencil = k <= 4 && p.nnz <= 8 * p.nrows;
+  if (k >= 2 && mr != 0 &&
+      (mr == 2 || !stencil || (column_locality(p, colind, s) & 1) == 0)) {
+    run_mrhs(p, a, MODE, vtype, xtype, ytype, s);
+    return;
   }
   // Staging each block's x window in LDS (one right-hand side) only when
   // the knob forces it: with all of a lane's gathers in flight, per-entry
@@ -370,26 +359,17 @@ void run_spmv(const Plan &p, int vtype, const void *colind, const void *vals,
               int xtype, const void *x, int64_t ldx, int ytype, void *y,
               int64_t ldy, int64_t k, double alpha, double beta,
               hipStream_t s) {
-  // Column panels serve k = 1; with k >= 2 the row-major x chunks are KP
-  // times wider than a panel's L2-sized slice, and the product runs over
-  // the share's own arrays.
+  // Column panels serve k = 1 (one column after another where row-major
+  // chunks of x are off); with k >= 2 the product runs over the share's own
+  // arrays.
   if (p.panels && (k == 1 || tuned_mrhs() == 0)) {
     run_spmv_panels(p, vtype, colind, vals, xtype, x, ldx, ytype, y, ldy, k,
                     alpha, beta, s);
     return;
   }
   if (p.panels) check_panel_operands(p, vtype, colind, vals);
-  run_spmv_impl<kPlain>(p, vtype, colind, vals, nullptr, nullptr, xtype, x,
+  run_spmv_impl<kPlain>(p, vtype, colind, vals, nullptr, xtype, x,
                         ldx, ytype, y, ldy, k, alpha, beta, s);
-}
-
-void run_spmv_rowmap(const Plan &p, int vtype, const void *colind,
-                     const void *vals, const void *rowmap, int xtype,
-                     const void *x, int64_t ldx, int ytype, void *y,
-                     int64_t ldy, int64_t k, double alpha, double beta,
-                     hipStream_t s) {
-  run_spmv_impl<kRowMap>(p, vtype, colind, vals, nullptr, rowmap, xtype, x,
-                         ldx, ytype, y, ldy, k, alpha, beta, s);
 }
 
 void run_spmv_perm(const Plan &p, int vtype, const void *colind,
@@ -397,7 +377,7 @@ void run_spmv_perm(const Plan &p, int vtype, const void *colind,
                    const void *x, int64_t ldx, int ytype, void *y,
                    int64_t ldy, int64_t k, double alpha, double beta,
                    hipStream_t s) {
-  run_spmv_impl<kPerm>(p, vtype, colind, vals, perm, nullptr, xtype, x, ldx,
+  run_spmv_impl<kPerm>(p, vtype, colind, vals, perm, xtype, x, ldx,
                        ytype, y, ldy, k, alpha, beta, s);
 }
 

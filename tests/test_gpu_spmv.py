@@ -463,6 +463,106 @@ def test_panel_layout_zipf(orc):
     assert componentwise_err(y.cpu().numpy(), ystar, absy) < 1e-5
 
 
+def _sliced_rows(rng, n):
+    """Row lengths that put segment ends everywhere: empty rows, single
+    entries, rows of a few entries, rows whose segments run over lanes, steps
+    and the ranges of waves, and one row that holds every column."""
+    lens = ([0, 0, 1, n, 0, 1, 1, 20000, 3, 0] + list(rng.integers(0, 12, 30000)) +
+            [513, 5000, 0, 40000] + list(rng.integers(0, 3, 9000)) + [n // 2, 0, 0])
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    ci = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens if L]).astype(np.int64)
+    return rp, ci
+
+
+@pytest.mark.parametrize("vdt,xdt", [(torch.float64, torch.float64), (torch.float32, torch.float32),
+                                     (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)])
+@pytest.mark.parametrize("panel_cols", [0, 7001, 50000])
+def test_panel_slices(orc, vdt, xdt, panel_cols):
+    """Column slices (x in LDS) of 131075 columns: slices cut from a wide
+    panel, narrow panels that share a slice, a last slice of three columns;
+    alpha / beta, infinities that only some rows meet, and new values."""
+    rng = np.random.default_rng(17 + panel_cols)
+    n = 131075
+    rp, ci = _sliced_rows(rng, n)
+    m = rp.size - 1
+    wide = np.float64 if vdt == torch.float64 else np.float32
+    Ad = upload(rp, ci, rng.uniform(-1, 1, ci.size).astype(wide), (m, n))
+    Aq = drx.CsrMatrix(Ad.rowptr, Ad.colind, Ad.vals.to(vdt), Ad.shape)
+    Aq.set_panels(panel_cols)
+    x = torch.as_tensor(rng.uniform(-1, 1, n).astype(wide)).to(DEV).to(xdt)
+    y0 = torch.rand(m, dtype=torch.float64 if vdt == torch.float64 else torch.float32, device=DEV)
+    y = Aq.matvec(x, y=y0.clone(), alpha=2.0, beta=0.5)
+    torch.cuda.synchronize()
+    v = Aq.vals.double().cpu().numpy()
+    ys, absy = orc.spmv(rp, ci, v, x.double().cpu().numpy())
+    y0h = y0.double().cpu().numpy()
+    tol = 1e-12 if vdt == torch.float64 else 1e-5
+    err = np.abs(y.double().cpu().numpy() - (2.0 * ys + 0.5 * y0h))
+    assert (err <= tol * (2.0 * absy + 0.5 * y0h) + 1e-300).all()
+    # the same bits every time, and new values through the permutation
+    assert torch.equal(Aq.matvec(x, y=y0.clone(), alpha=2.0, beta=0.5), y)
+    Aq.update_values(-Aq.vals)
+    assert torch.equal(Aq.matvec(x, y=-y0, alpha=2.0, beta=0.5), -y)
+    # an infinite x reaches the rows that hold its column and no others
+    c = int(ci[rp[8]])
+    x[c] = float("inf")
+    y2 = Aq.matvec(x).cpu().numpy()
+    rows = np.repeat(np.arange(m), np.diff(rp))[ci == c]
+    assert np.array_equal(np.flatnonzero(~np.isfinite(y2)), np.unique(rows))
+    Aq.close()
+    Ad.close()
+
+
+def test_panel_slices_captured(orc):
+    """A panel product captured in a graph (its segment sums allocated on the
+    captured stream) and replayed with new x, eager products between."""
+    rng = np.random.default_rng(5)
+    rp, ci = _sliced_rows(rng, 131075)
+    v = rng.uniform(-1, 1, ci.size).astype(np.float32)
+    A = upload(rp, ci, v, (rp.size - 1, 131075))
+    A.set_panels()
+    x = drx.gen.uniform(131075, torch.float32, -1, 1, seed=1)
+    y = torch.empty(rp.size - 1, dtype=torch.float32, device=DEV)
+    A.matvec(x, y=y)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        A.matvec(x, y=y)
+    for i in range(4):
+        x.copy_(drx.gen.uniform(131075, torch.float32, -1, 1, seed=10 + i))
+        eager = A.matvec(x)
+        y.zero_()
+        g.replay()
+        other = A.matvec(2 * x)
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager) and torch.equal(other, 2 * y)
+    ys, absy = orc.spmv(rp, ci, v, x.cpu().numpy())
+    assert componentwise_err(y.cpu().numpy(), ys, absy) < 1e-5
+    del g
+    A.close()
+
+
+@pytest.mark.parametrize("vdt", [torch.float64, torch.float32])
+def test_panel_slices_sparse_rows(orc, vdt):
+    """So few entries over 25M rows and 4M columns that the table of row
+    groups would outgrow them: groups owned by whole workgroups."""
+    rng = np.random.default_rng(23)
+    m, n, nnz = 25_000_000, 4_000_000, 1_000_000
+    rows = np.sort(rng.integers(0, m, nnz))
+    rp = np.zeros(m + 1, np.int64)
+    np.cumsum(np.bincount(rows, minlength=m), out=rp[1:])
+    ci = rng.integers(0, n, nnz)
+    v = rng.uniform(-1, 1, nnz).astype(np.float64 if vdt == torch.float64 else np.float32)
+    A = upload(rp, ci, v, (m, n))
+    A.set_panels()
+    x = drx.gen.uniform(n, vdt, -1, 1, seed=2)
+    y = A.matvec(x)
+    torch.cuda.synchronize()
+    ys, absy = orc.spmv(rp, ci, v, x.cpu().numpy())
+    assert componentwise_err(y.cpu().numpy(), ys, absy) < (1e-12 if vdt == torch.float64 else 1e-5)
+    A.close()
+
+
 def _batch_mats(nmat, seed, rows=(500, 4000), lens=(3, 64)):
     rng = np.random.default_rng(seed)
     mats = []
