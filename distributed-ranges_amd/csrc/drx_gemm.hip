@@ -76,6 +76,82 @@ struct GemmCfg {
 // that XCD's L2.
 constexpr int kGroupM = 8;
 
+// Which part of the product a workgroup computes. The first `main` tiles
+// (a multiple of the CUs) are computed whole. The rest would leave most CUs
+// idle for the time of a whole tile, so each of them is cut into `parts`
+// ranges of k stages: a workgroup writes its range's sums to slot u of a
+// workspace (BM x BN elements each), and k_gemm_reduce adds the parts in
+// order. FP32, whole tiles only -> cut (us): 2000^3 262 -> 164, 1000^3 144 -> 41,
+// 203 x 295 x 4502 703 -> 36, 96 x 5000 x 5000 653 -> 78; FP64 540 -> 287, 292 ->
+// 61, 1375 -> 44, 1280 -> 131.
+struct GemmGrid {
+  int64_t tiles_m, tiles_n;
+  int64_t main, main_xcd;  // whole tiles; per XCD
+  int64_t tail_xcd;        // parts of the other tiles per XCD
+  int parts;
+};
+struct GemmPart {
+  int64_t m0, n0;     // first row and column of the tile
+  int64_t kt0, kt1;   // stages
+  int64_t slot;       // workspace slot, -1: the whole tile goes to C
+};
+template <int BM, int BN>
+__device__ __forceinline__ void gemm_tile_at(const GemmGrid &g, int64_t tile, int64_t &m0,
+                                             int64_t &n0) {
+  const int64_t per_group = int64_t(kGroupM) * g.tiles_n;
+  const int64_t first = tile / per_group * kGroupM;
+  const int64_t gsz = g.tiles_m - first < kGroupM ? g.tiles_m - first : kGroupM;
+  const int64_t in_g = tile % per_group;
+  m0 = (first + in_g % gsz) * BM;
+  n0 = (in_g / gsz) * BN;
+}
+// false: nothing to do (the whole workgroup leaves together).
+template <int BM, int BN>
+__device__ __forceinline__ bool gemm_part(const GemmGrid &g, int64_t nk, GemmPart &p) {
+  const int64_t whole = g.main_xcd * kXcds;
+  int64_t tile;
+  if (blockIdx.x < whole) {
+    tile = map_block(blockIdx.x, g.main_xcd);
+    if (tile >= g.main) return false;
+    p.kt0 = 0;
+    p.kt1 = nk;
+    p.slot = -1;
+  } else {
+    p.slot = map_block(blockIdx.x - whole, g.tail_xcd);
+    tile = g.main + p.slot / g.parts;
+    if (tile >= g.tiles_m * g.tiles_n) return false;
+    const int64_t part = p.slot % g.parts;
+    p.kt0 = nk * part / g.parts;
+    p.kt1 = nk * (part + 1) / g.parts;
+  }
+  gemm_tile_at<BM, BN>(g, tile, p.m0, p.n0);
+  return true;
+}
+
+// C of the tiles that were cut: the parts' sums in order, then alpha and beta
+// as in the kernels' own epilogue. A wave reads 64 consecutive elements of a
+// tile row.
+template <typename T, int BM, int BN>
+__global__ void k_gemm_reduce(int64_t m, int64_t n, T alpha, T beta, T *__restrict__ C,
+                              int64_t ldc, GemmGrid g, const T *__restrict__ ws) {
+  const int64_t tiles = g.tiles_m * g.tiles_n - g.main;
+  const int64_t total = tiles * BM * BN;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int64_t t = i / (BM * BN), e = i % (BM * BN);
+    int64_t m0, n0;
+    gemm_tile_at<BM, BN>(g, g.main + t, m0, n0);
+    const int64_t gi = m0 + e / BN, gj = n0 + e % BN;
+    if (gi >= m || gj >= n) continue;
+    const T *p = ws + t * g.parts * (BM * BN) + e;
+    T sum = p[0];
+    for (int q = 1; q < g.parts; q++) sum += p[static_cast<int64_t>(q) * (BM * BN)];
+    T &c = C[gi * ldc + gj];
+    const T prod = alpha * sum;
+    c = beta == T(0) ? prod : prod + beta * c;
+  }
+}
+
 // Waves per SIMD the register budget is held to, from the accumulator
 // registers per lane: 64 -> 4 waves with eight-wave workgroups, 3 with
 // four-wave ones (their lanes carry more of each stage's loads; 4 would
@@ -90,85 +166,98 @@ __global__ void __launch_bounds__(64 * WM * WN)
         gemm_waves<GemmCfg<T, BM, BN, BK, WM, WN>::ACC_REGS, 64 * WM * WN>())))
     k_gemm(int64_t m, int64_t n, int64_t K, T alpha, const T *__restrict__ A,
            int64_t lda, const T *__restrict__ B, int64_t ldb, T beta,
-           T *__restrict__ C, int64_t ldc, int64_t tiles_m, int64_t tiles_n,
-           int64_t per_xcd, int vec_ok) {
+           T *__restrict__ C, int64_t ldc, GemmGrid grid, T *__restrict__ ws) {
   using Cfg = GemmCfg<T, BM, BN, BK, WM, WN>;
   using vec_t = T __attribute__((ext_vector_type(Cfg::V)));
+  // Rows of A and B start anywhere (any leading dimension): 16-byte loads at
+  // element alignment, which global memory serves. Loading rows that are not
+  // 16-byte aligned element by element ran 4099 x 3001 x 2050 FP32 at 53
+  // TFLOP/s.
+  typedef vec_t mem_t __attribute__((aligned(sizeof(T))));
   using acc_t = typename Mfma<T>::acc_t;
   __shared__ __attribute__((aligned(16))) T smem[2 * Cfg::STAGE];
 
-  const int64_t logical = map_block(blockIdx.x, per_xcd);
-  if (logical >= tiles_m * tiles_n) return;  // whole workgroup leaves together
-  const int64_t per_group = int64_t(kGroupM) * tiles_n;
-  const int64_t first = logical / per_group * kGroupM;
-  const int64_t gsz = tiles_m - first < kGroupM ? tiles_m - first : kGroupM;
-  const int64_t in_g = logical % per_group;
-  const int64_t m0 = (first + in_g % gsz) * BM;
-  const int64_t n0 = (in_g / gsz) * BN;
+  const int64_t nk = (K + BK - 1) / BK;
+  GemmPart part;
+  if (!gemm_part<BM, BN>(grid, nk, part)) return;
+  const int64_t m0 = part.m0, n0 = part.n0;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, r = lane & 15;
   const int wm = wave / WN, wn = wave % WN;
-  const bool inner_mn = vec_ok && m0 + BM <= m && n0 + BN <= n;
-
+  // Full stages load 16 bytes per slot wherever the tile lies: rows of A past
+  // m read row m - 1, slots of B past n the row's last whole slot (their
+  // products are never stored), and a slot across column n reads on into the
+  // next row -- so not in the stage that holds B's last row, which like a
+  // partial last stage is loaded with a check per slot. (With a check per
+  // slot in every stage of the edge tiles 4100 x 3004 x 2052 FP32 took 585 us
+  // where 4096 x 3072 x 2048 took 425; now 446.)
+  const bool n_inner = n0 + BN <= n;
+  const T *a_src[Cfg::A_VECS], *b_src[Cfg::B_VECS];
+#pragma unroll
+  for (int p = 0; p < Cfg::A_VECS; ++p) {
+    const int q = tid + p * Cfg::kThreads;
+    const int64_t gi = m0 + q / Cfg::A_TPR;
+    a_src[p] = A + (gi < m ? gi : m - 1) * lda + (q % Cfg::A_TPR) * Cfg::V;
+  }
+#pragma unroll
+  for (int p = 0; p < Cfg::B_VECS; ++p) {
+    const int q = tid + p * Cfg::kThreads;
+    const int64_t gj = n0 + (q % Cfg::B_TPR) * Cfg::V;
+    b_src[p] = B + (q / Cfg::B_TPR) * ldb + (gj < n ? gj : n - Cfg::V);
+  }
+  // stages [0, nwhole) load whole slots
+  const int64_t nwhole = n < Cfg::V ? 0 : n_inner ? K / BK : (K - 1) / BK;
   vec_t ra[Cfg::A_VECS], rb[Cfg::B_VECS];
   auto load = [&](int64_t k0) {
-    if (inner_mn && k0 + BK <= K) {
 #pragma unroll
-      for (int p = 0; p < Cfg::A_VECS; ++p) {
-        const int q = tid + p * Cfg::kThreads;
-        const int row = q / Cfg::A_TPR, kv = q % Cfg::A_TPR;
-        ra[p] = *reinterpret_cast<const vec_t *>(A + (m0 + row) * lda + k0 + kv * Cfg::V);
-      }
+    for (int p = 0; p < Cfg::A_VECS; ++p)
+      ra[p] = *reinterpret_cast<const mem_t *>(a_src[p] + k0);
 #pragma unroll
-      for (int p = 0; p < Cfg::B_VECS; ++p) {
-        const int q = tid + p * Cfg::kThreads;
-        const int kr = q / Cfg::B_TPR, jv = q % Cfg::B_TPR;
-        rb[p] = *reinterpret_cast<const vec_t *>(B + (k0 + kr) * ldb + n0 + jv * Cfg::V);
-      }
-    } else {  // edge tile, partial last stage or unaligned rows: per 16-byte slot
-#pragma unroll
-      for (int p = 0; p < Cfg::A_VECS; ++p) {
-        const int q = tid + p * Cfg::kThreads;
-        const int row = q / Cfg::A_TPR, kv = q % Cfg::A_TPR;
-        const int64_t gi = m0 + row, gk = k0 + kv * Cfg::V;
-        if (vec_ok && gi < m && gk + Cfg::V <= K) {
-          ra[p] = *reinterpret_cast<const vec_t *>(A + gi * lda + gk);
-        } else {
-#pragma unroll
-          for (int e = 0; e < Cfg::V; ++e)
-            ra[p][e] = (gi < m && gk + e < K) ? A[gi * lda + gk + e] : T(0);
-        }
-      }
-#pragma unroll
-      for (int p = 0; p < Cfg::B_VECS; ++p) {
-        const int q = tid + p * Cfg::kThreads;
-        const int kr = q / Cfg::B_TPR, jv = q % Cfg::B_TPR;
-        const int64_t gk = k0 + kr, gj = n0 + jv * Cfg::V;
-        if (vec_ok && gk < K && gj + Cfg::V <= n) {
-          rb[p] = *reinterpret_cast<const vec_t *>(B + gk * ldb + gj);
-        } else {
-#pragma unroll
-          for (int e = 0; e < Cfg::V; ++e)
-            rb[p][e] = (gk < K && gj + e < n) ? B[gk * ldb + gj + e] : T(0);
-        }
-      }
-    }
+    for (int p = 0; p < Cfg::B_VECS; ++p)
+      rb[p] = *reinterpret_cast<const mem_t *>(b_src[p] + k0 * ldb);
+  };
+  auto a_at = [&](T *st, int q) {
+    return reinterpret_cast<vec_t *>(st + (q / Cfg::A_TPR) * Cfg::LDA_S + (q % Cfg::A_TPR) * Cfg::V);
+  };
+  auto b_at = [&](T *st, int q) {
+    return reinterpret_cast<vec_t *>(st + BM * Cfg::LDA_S + (q / Cfg::B_TPR) * Cfg::LDB_S +
+                                     (q % Cfg::B_TPR) * Cfg::V);
   };
   auto store = [&](T *st) {
-    T *As = st, *Bs = st + BM * Cfg::LDA_S;
+#pragma unroll
+    for (int p = 0; p < Cfg::A_VECS; ++p) *a_at(st, tid + p * Cfg::kThreads) = ra[p];
+#pragma unroll
+    for (int p = 0; p < Cfg::B_VECS; ++p) *b_at(st, tid + p * Cfg::kThreads) = rb[p];
+  };
+  // A stage with a check per slot, straight to LDS.
+  auto load_checked = [&](int64_t k0, T *st) {
 #pragma unroll
     for (int p = 0; p < Cfg::A_VECS; ++p) {
       const int q = tid + p * Cfg::kThreads;
-      *reinterpret_cast<vec_t *>(As + (q / Cfg::A_TPR) * Cfg::LDA_S +
-                                 (q % Cfg::A_TPR) * Cfg::V) = ra[p];
+      const int64_t gi = m0 + q / Cfg::A_TPR, gk = k0 + (q % Cfg::A_TPR) * Cfg::V;
+      vec_t v;
+      if (gi < m && gk + Cfg::V <= K) {
+        v = *reinterpret_cast<const mem_t *>(A + gi * lda + gk);
+      } else {
+#pragma unroll
+        for (int e = 0; e < Cfg::V; ++e) v[e] = (gi < m && gk + e < K) ? A[gi * lda + gk + e] : T(0);
+      }
+      *a_at(st, q) = v;
     }
 #pragma unroll
     for (int p = 0; p < Cfg::B_VECS; ++p) {
       const int q = tid + p * Cfg::kThreads;
-      *reinterpret_cast<vec_t *>(Bs + (q / Cfg::B_TPR) * Cfg::LDB_S +
-                                 (q % Cfg::B_TPR) * Cfg::V) = rb[p];
+      const int64_t gk = k0 + q / Cfg::B_TPR, gj = n0 + (q % Cfg::B_TPR) * Cfg::V;
+      vec_t v;
+      if (gk < K && gj + Cfg::V <= n) {
+        v = *reinterpret_cast<const mem_t *>(B + gk * ldb + gj);
+      } else {
+#pragma unroll
+        for (int e = 0; e < Cfg::V; ++e) v[e] = (gk < K && gj + e < n) ? B[gk * ldb + gj + e] : T(0);
+      }
+      *b_at(st, q) = v;
     }
   };
 
@@ -178,16 +267,19 @@ __global__ void __launch_bounds__(64 * WM * WN)
 #pragma unroll
     for (int j = 0; j < Cfg::FN; ++j) acc[i][j] = acc_t{};
 
-  const int64_t nk = (K + BK - 1) / BK;
-  if (nk > 0) {
-    load(0);
-    store(smem);
+  if (part.kt0 < part.kt1) {
+    T *st = smem + (part.kt0 & 1) * Cfg::STAGE;
+    if (part.kt0 < nwhole) {
+      load(part.kt0 * BK);
+      store(st);
+    } else {
+      load_checked(part.kt0 * BK, st);
+    }
   }
   __syncthreads();
-  for (int64_t kt = 0; kt < nk; ++kt) {
+  auto products = [&](int64_t kt) {
     const T *As = smem + (kt & 1) * Cfg::STAGE;
     const T *Bs = As + BM * Cfg::LDA_S;
-    if (kt + 1 < nk) load((kt + 1) * BK);
 #pragma unroll
     for (int s = 0; s < BK / Cfg::SK; ++s) {
       vec_t a[Cfg::FM];
@@ -209,10 +301,38 @@ __global__ void __launch_bounds__(64 * WM * WN)
           for (int j = 0; j < Cfg::FN; ++j)
             acc[i][j] = Mfma<T>::op(a[i][kk], b[j][kk], acc[i][j]);
     }
-    if (kt + 1 < nk) store(smem + ((kt + 1) & 1) * Cfg::STAGE);
+  };
+  // The stages whose successor loads whole slots, then the rest: with the
+  // checked loads in the same loop, every stage waited for its loads before
+  // its products (4096^3: FP32 1161 -> 1042 us, FP64 2234 -> 2081).
+  int64_t kt = part.kt0;
+  for (; kt + 1 < (part.kt1 < nwhole ? part.kt1 : nwhole); ++kt) {
+    load((kt + 1) * BK);
+    products(kt);
+    store(smem + ((kt + 1) & 1) * Cfg::STAGE);
+    __syncthreads();
+  }
+  for (; kt < part.kt1; ++kt) {
+    products(kt);
+    if (kt + 1 < part.kt1) load_checked((kt + 1) * BK, smem + ((kt + 1) & 1) * Cfg::STAGE);
     __syncthreads();
   }
 
+  // Epilogue: element v of the lane holds D[Mfma<T>::row(g, v)][r] of each
+  // MFMA tile. beta == 0 does not read C (so C may hold anything, NaN
+  // included), as in BLAS.
+  if (part.slot >= 0) {
+    T *p = ws + part.slot * (BM * BN);
+#pragma unroll
+    for (int i = 0; i < Cfg::FM; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int j = 0; j < Cfg::FN; ++j)
+          p[(wm * Cfg::TM + i * 16 + Mfma<T>::row(g, v)) * BN + wn * Cfg::TN + j * 16 + r] =
+              acc[i][j][v];
+    return;
+  }
   // Epilogue: element v of the lane holds D[Mfma<T>::row(g, v)][r] of each
   // MFMA tile. beta == 0 does not read C (so C may hold anything, NaN
   // included), as in BLAS.
@@ -259,8 +379,8 @@ template <int BM, int WM, int WN>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(3)))
     k_gemm_dl(int64_t m, int64_t n, int64_t K, float alpha, const float *__restrict__ A,
               int64_t lda, const float *__restrict__ B, int64_t ldb, float beta,
-              float *__restrict__ C, int64_t ldc, int64_t tiles_m, int64_t tiles_n,
-              int64_t per_xcd, int vec_ok) {
+              float *__restrict__ C, int64_t ldc, GemmGrid grid, float *__restrict__ ws,
+              int vec_ok) {
   constexpr int BN = 128, BK = 16, NW = WM * WN;
   constexpr int A_BYTES = BM * BK * 4, B_BYTES = BK * BN * 4, STAGE = A_BYTES + B_BYTES;
   constexpr int A_INSTR = A_BYTES / 1024 / NW, B_INSTR = B_BYTES / 1024 / NW;
@@ -270,20 +390,20 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
   static_assert(TM % 16 == 0 && TN % 16 == 0, "wave tile must be whole MFMA tiles");
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
 
-  const int64_t logical = map_block(blockIdx.x, per_xcd);
-  if (logical >= tiles_m * tiles_n) return;  // whole workgroup leaves together
-  const int64_t per_group = int64_t(kGroupM) * tiles_n;
-  const int64_t first = logical / per_group * kGroupM;
-  const int64_t gsz = tiles_m - first < kGroupM ? tiles_m - first : kGroupM;
-  const int64_t in_g = logical % per_group;
-  const int64_t m0 = (first + in_g % gsz) * BM;
-  const int64_t n0 = (in_g / gsz) * BN;
+  const int64_t nk = (K + BK - 1) / BK;
+  GemmPart part;
+  if (!gemm_part<BM, BN>(grid, nk, part)) return;
+  const int64_t m0 = part.m0, n0 = part.n0;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, r = lane & 15;
   const int wm = wave / WN, wn = wave % WN;
-  const bool n_inner = vec_ok && n0 + BN <= n;
+  const bool n_inner = n0 + BN <= n;
+  // stage kt straight into LDS (which slots may not: see k_gemm)
+  auto direct_ok = [&](int64_t kt) {
+    return vec_ok && n >= 4 && ((kt + 1) * BK < K || (n_inner && (kt + 1) * BK == K));
+  };
 
   // The (row, slot) each lane moves: A block p * NW + wave, row block*16 +
   // lane/4, slot (lane%4) ^ fa(lane/4); B block p * NW + wave, row
@@ -300,7 +420,10 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
     a_src[p] = A + gi * lda + a_col(p);
   }
 #pragma unroll
-  for (int p = 0; p < B_INSTR; ++p) b_src[p] = B + b_row(p) * ldb + n0 + b_col(p);
+  for (int p = 0; p < B_INSTR; ++p) {
+    const int64_t gj = n0 + b_col(p);
+    b_src[p] = B + b_row(p) * ldb + (gj < n ? gj : (n - 4) / 4 * 4);
+  }
 
   auto issue_direct = [&](int64_t k0, char *st) {
 #pragma unroll
@@ -360,22 +483,22 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{};
 
-  const int64_t nk = (K + BK - 1) / BK;
-  if (nk > 0) {
-    if (n_inner && BK <= K) {
-      issue_direct(0, smem);
+  if (part.kt0 < part.kt1) {
+    char *st = smem + (part.kt0 & 1) * STAGE;
+    if (direct_ok(part.kt0)) {
+      issue_direct(part.kt0 * BK, st);
     } else {
-      load_regs(0);
-      store_regs(smem);
+      load_regs(part.kt0 * BK);
+      store_regs(st);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  for (int64_t kt = 0; kt < nk; ++kt) {
+  for (int64_t kt = part.kt0; kt < part.kt1; ++kt) {
     const char *cur = smem + (kt & 1) * STAGE;
     char *nxt = smem + ((kt + 1) & 1) * STAGE;
-    const bool more = kt + 1 < nk;
-    const bool direct = more && n_inner && (kt + 2) * BK <= K;
+    const bool more = kt + 1 < part.kt1;
+    const bool direct = more && direct_ok(kt + 1);
     if (direct) issue_direct((kt + 1) * BK, nxt);
     f32x4 a[FM];
 #pragma unroll
@@ -398,6 +521,18 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
     __syncthreads();
   }
 
+  if (part.slot >= 0) {
+    float *p = ws + part.slot * (BM * BN);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          p[(wm * TM + i * 16 + Mfma<float>::row(g, v)) * BN + wn * TN + j * 16 + r] =
+              acc[i][j][v];
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
 #pragma unroll
@@ -429,8 +564,8 @@ template <int BM, int WM, int WN>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2)))
     k_gemm_dl64(int64_t m, int64_t n, int64_t K, double alpha, const double *__restrict__ A,
                 int64_t lda, const double *__restrict__ B, int64_t ldb, double beta,
-                double *__restrict__ C, int64_t ldc, int64_t tiles_m, int64_t tiles_n,
-                int64_t per_xcd, int vec_ok) {
+                double *__restrict__ C, int64_t ldc, GemmGrid grid, double *__restrict__ ws,
+                int vec_ok) {
   typedef double f64x2 __attribute__((ext_vector_type(2)));
   constexpr int BN = 128, BK = 16, NW = WM * WN;
   constexpr int A_BYTES = BM * BK * 8, B_BYTES = BK * BN * 8, STAGE = A_BYTES + B_BYTES;
@@ -441,20 +576,20 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
   static_assert(TM % 16 == 0 && TN % 16 == 0, "wave tile must be whole MFMA tiles");
   __shared__ __attribute__((aligned(1024))) char smem[2 * STAGE];
 
-  const int64_t logical = map_block(blockIdx.x, per_xcd);
-  if (logical >= tiles_m * tiles_n) return;  // whole workgroup leaves together
-  const int64_t per_group = int64_t(kGroupM) * tiles_n;
-  const int64_t first = logical / per_group * kGroupM;
-  const int64_t gsz = tiles_m - first < kGroupM ? tiles_m - first : kGroupM;
-  const int64_t in_g = logical % per_group;
-  const int64_t m0 = (first + in_g % gsz) * BM;
-  const int64_t n0 = (in_g / gsz) * BN;
+  const int64_t nk = (K + BK - 1) / BK;
+  GemmPart part;
+  if (!gemm_part<BM, BN>(grid, nk, part)) return;
+  const int64_t m0 = part.m0, n0 = part.n0;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, r = lane & 15;
   const int wm = wave / WN, wn = wave % WN;
-  const bool n_inner = vec_ok && n0 + BN <= n;
+  const bool n_inner = n0 + BN <= n;
+  // stage kt straight into LDS (which slots may not: see k_gemm)
+  auto direct_ok = [&](int64_t kt) {
+    return vec_ok && n >= 2 && ((kt + 1) * BK < K || (n_inner && (kt + 1) * BK == K));
+  };
 
   // A block p * NW + wave: rows block*8 + lane/8, slot (lane%8) ^ fa64(row);
   // B block p * NW + wave: row = block, slot lane ^ hb64(row).
@@ -470,7 +605,10 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
     a_src[p] = A + gi * lda + a_col(p);
   }
 #pragma unroll
-  for (int p = 0; p < B_INSTR; ++p) b_src[p] = B + b_row(p) * ldb + n0 + b_col(p);
+  for (int p = 0; p < B_INSTR; ++p) {
+    const int64_t gj = n0 + b_col(p);
+    b_src[p] = B + b_row(p) * ldb + (gj < n ? gj : (n - 2) / 2 * 2);
+  }
 
   auto issue_direct = [&](int64_t k0, char *st) {
 #pragma unroll
@@ -526,20 +664,20 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f64x4{};
 
-  const int64_t nk = (K + BK - 1) / BK;
-  if (nk > 0) {
-    if (n_inner && BK <= K)
-      issue_direct(0, smem);
+  if (part.kt0 < part.kt1) {
+    char *st = smem + (part.kt0 & 1) * STAGE;
+    if (direct_ok(part.kt0))
+      issue_direct(part.kt0 * BK, st);
     else
-      load_store_regs(0, smem);
+      load_store_regs(part.kt0 * BK, st);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  for (int64_t kt = 0; kt < nk; ++kt) {
+  for (int64_t kt = part.kt0; kt < part.kt1; ++kt) {
     const char *cur = smem + (kt & 1) * STAGE;
     char *nxt = smem + ((kt + 1) & 1) * STAGE;
-    const bool more = kt + 1 < nk;
-    const bool direct = more && n_inner && (kt + 2) * BK <= K;
+    const bool more = kt + 1 < part.kt1;
+    const bool direct = more && direct_ok(kt + 1);
     if (direct) issue_direct((kt + 1) * BK, nxt);
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
@@ -564,6 +702,18 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
     __syncthreads();
   }
 
+  if (part.slot >= 0) {
+    double *p = ws + part.slot * (BM * BN);
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          p[(wm * TM + i * 16 + Mfma<double>::row(g, v)) * BN + wn * TN + j * 16 + r] =
+              acc[i][j][v];
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
 #pragma unroll
@@ -582,50 +732,134 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
   }
 }
 
+// Tiles whole and in parts: the parts of the tiles beyond the last full round
+// of resident workgroups that cost least by this model. A CU works its tiles
+// off at one rate, less while few waves share a SIMD (measured: 2000^3, one
+// four-wave workgroup per CU, 0.45 of the rate of three), and the cut tiles'
+// sums are written and read once more.
+constexpr int64_t kLeastStages = 4;
+struct GemmCost {
+  int waves;     // per SIMD and workgroup
+  int resident;  // workgroups per CU
+  double rate;   // of a busy CU, Tflop/s
+};
+inline double gemm_time_us(int64_t units, int64_t parts, double tile_us, int64_t cus,
+                           const GemmCost &c) {
+  constexpr double kEff[5] = {0.45, 0.45, 0.75, 0.95, 1.0};
+  const int64_t per_cu = (units + cus - 1) / cus;
+  const int64_t waves = std::min<int64_t>(4, std::min<int64_t>(per_cu, c.resident) * c.waves);
+  return static_cast<double>(per_cu) / static_cast<double>(parts) * tile_us / kEff[waves];
+}
+inline GemmGrid gemm_grid(int64_t m, int64_t n, int64_t k, int bm, int bn, int bk, size_t esz,
+                          int64_t cus, const GemmCost &c, double *cost_us = nullptr) {
+  GemmGrid g{};
+  g.tiles_m = (m + bm - 1) / bm;
+  g.tiles_n = (n + bn - 1) / bn;
+  const int64_t tiles = g.tiles_m * g.tiles_n, nk = (k + bk - 1) / bk;
+  const int64_t whole = tiles / (c.resident * cus) * (c.resident * cus), rest = tiles - whole;
+  const double tile_us = 2e-6 * bm * bn * static_cast<double>(nk * bk) / c.rate;
+  g.main = tiles;
+  g.parts = 1;
+  double best = gemm_time_us(tiles, 1, tile_us, cus, c);
+  const double before = static_cast<double>(whole) / static_cast<double>(cus) * tile_us;
+  for (int64_t p = 2; rest > 0 && p <= std::min<int64_t>(64, nk / kLeastStages); p++) {
+    const double bytes = 2.0 * static_cast<double>(rest * p) * bm * bn * static_cast<double>(esz);
+    const double t = before + gemm_time_us(rest * p, p, tile_us, cus, c) + 6.0 + bytes / 4e6;
+    if (t < best) {
+      best = t;
+      g.main = whole;
+      g.parts = static_cast<int>(p);
+    }
+  }
+  if (cost_us) *cost_us = best;
+  g.main_xcd = (g.main + kXcds - 1) / kXcds;
+  g.tail_xcd = ((tiles - g.main) * g.parts + kXcds - 1) / kXcds;
+  DRX_REQUIRE((g.main_xcd + g.tail_xcd) * kXcds <= int64_t(0xffffffff),
+              "product too large for one launch");
+  return g;
+}
+
+// Resident workgroups follow from the register budgets (gemm_waves) and the
+// 512 registers of a SIMD lane.
+template <typename T> constexpr double gemm_rate() { return sizeof(T) == 8 ? 0.26 : 0.52; }
+template <typename T, int BM, int BN, int WM, int WN> constexpr GemmCost gemm_cost() {
+  constexpr int acc = BM / WM * (BN / WN) / 64 * static_cast<int>(sizeof(T)) / 4;
+  constexpr int waves = gemm_waves<acc, 64 * WM * WN>();
+  return GemmCost{WM * WN / 4, waves * 4 / (WM * WN) > 0 ? waves * 4 / (WM * WN) : 1,
+                  gemm_rate<T>()};
+}
+
+inline int gemm_cus() {
+  int dev = 0, cus = 0;
+  DRX_HIP(hipGetDevice(&dev));
+  DRX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  return std::max(cus, 1);
+}
+
+// Launches `kernel(grid, threads, g, ws)` over the tiles, then the reduction of
+// those that were cut.
+template <typename T, int BM, int BN, int BK, typename Launch>
+void launch_tiles(int64_t m, int64_t n, int64_t k, T alpha, T beta, T *c, int64_t ldc,
+                  const GemmCost &cost, hipStream_t s, Launch &&kernel) {
+  const GemmGrid g = gemm_grid(m, n, k, BM, BN, BK, sizeof(T), gemm_cus(), cost);
+  const dim3 grid(static_cast<unsigned>((g.main_xcd + g.tail_xcd) * kXcds));
+  const int64_t cut = g.tiles_m * g.tiles_n - g.main;
+  if (cut == 0) {
+    kernel(grid, g, static_cast<T *>(nullptr));
+    DRX_HIP(hipGetLastError());
+    return;
+  }
+  T *ws = static_cast<T *>(scratch_alloc(static_cast<size_t>(cut) * g.parts * BM * BN * sizeof(T), s));
+  try {
+    kernel(grid, g, ws);
+    const int64_t blocks = std::min<int64_t>(cut * (BM * BN / 256), 8192);
+    hipLaunchKernelGGL((k_gemm_reduce<T, BM, BN>), dim3(static_cast<unsigned>(blocks)), dim3(256),
+                       0, s, m, n, alpha, beta, c, ldc, g, ws);
+    DRX_HIP(hipGetLastError());
+  } catch (...) {
+    scratch_free(ws, s);
+    throw;
+  }
+  scratch_free(ws, s);
+}
+
 inline void launch_gemm_dl64(int64_t m, int64_t n, int64_t k, double alpha, const double *a,
                              int64_t lda, const double *b, int64_t ldb, double beta, double *c,
                              int64_t ldc, hipStream_t s) {
-  const int64_t tiles_m = (m + 127) / 128, tiles_n = (n + 127) / 128;
-  const int64_t per_xcd = (tiles_m * tiles_n + kXcds - 1) / kXcds;
-  DRX_REQUIRE(per_xcd * kXcds <= int64_t(0xffffffff), "product too large for one launch");
   const bool aligned = reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(b) % 16 == 0 && lda % 2 == 0 && ldb % 2 == 0;
-  hipLaunchKernelGGL((k_gemm_dl64<128, 2, 2>), dim3(static_cast<unsigned>(per_xcd * kXcds)),
-                     dim3(256), 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tiles_m,
-                     tiles_n, per_xcd, aligned ? 1 : 0);
-  DRX_HIP(hipGetLastError());
+  launch_tiles<double, 128, 128, 16>(
+      m, n, k, alpha, beta, c, ldc, GemmCost{1, 2, gemm_rate<double>()}, s,
+      [&](dim3 grid, const GemmGrid &g, double *ws) {
+        hipLaunchKernelGGL((k_gemm_dl64<128, 2, 2>), grid, dim3(256), 0, s, m, n, k, alpha, a, lda,
+                           b, ldb, beta, c, ldc, g, ws, aligned ? 1 : 0);
+      });
 }
 
 template <int BM, int WM, int WN>
 void launch_gemm_dl(int64_t m, int64_t n, int64_t k, float alpha, const float *a, int64_t lda,
                     const float *b, int64_t ldb, float beta, float *c, int64_t ldc,
                     hipStream_t s) {
-  const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (n + 127) / 128;
-  const int64_t per_xcd = (tiles_m * tiles_n + kXcds - 1) / kXcds;
-  DRX_REQUIRE(per_xcd * kXcds <= int64_t(0xffffffff), "product too large for one launch");
   const bool aligned = reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(b) % 16 == 0 && lda % 4 == 0 && ldb % 4 == 0;
-  hipLaunchKernelGGL((k_gemm_dl<BM, WM, WN>), dim3(static_cast<unsigned>(per_xcd * kXcds)),
-                     dim3(64 * WM * WN), 0, s, m, n, k, alpha, a, lda, b, ldb, beta, c, ldc,
-                     tiles_m, tiles_n, per_xcd, aligned ? 1 : 0);
-  DRX_HIP(hipGetLastError());
+  launch_tiles<float, BM, 128, 16>(
+      m, n, k, alpha, beta, c, ldc, GemmCost{WM * WN / 4, 12 / (WM * WN), gemm_rate<float>()}, s,
+      [&](dim3 grid, const GemmGrid &g, float *ws) {
+        hipLaunchKernelGGL((k_gemm_dl<BM, WM, WN>), grid, dim3(64 * WM * WN), 0, s, m, n, k, alpha,
+                           a, lda, b, ldb, beta, c, ldc, g, ws, aligned ? 1 : 0);
+      });
 }
 
 template <typename T, int BM, int BN, int BK, int WM, int WN>
 void launch_gemm(int64_t m, int64_t n, int64_t k, T alpha, const T *a, int64_t lda,
                  const T *b, int64_t ldb, T beta, T *c, int64_t ldc, hipStream_t s) {
-  using Cfg = GemmCfg<T, BM, BN, BK, WM, WN>;
-  const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
-  const int64_t per_xcd = (tiles_m * tiles_n + kXcds - 1) / kXcds;
-  DRX_REQUIRE(per_xcd * kXcds <= int64_t(0xffffffff), "product too large for one launch");
-  const bool aligned = reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
-                       reinterpret_cast<uintptr_t>(b) % 16 == 0 &&
-                       lda % Cfg::V == 0 && ldb % Cfg::V == 0;
-  hipLaunchKernelGGL((k_gemm<T, BM, BN, BK, WM, WN>),
-                     dim3(static_cast<unsigned>(per_xcd * kXcds)), dim3(Cfg::kThreads), 0, s,
-                     m, n, k, alpha, a, lda, b, ldb, beta, c, ldc, tiles_m, tiles_n,
-                     per_xcd, aligned ? 1 : 0);
-  DRX_HIP(hipGetLastError());
+  launch_tiles<T, BM, BN, BK>(
+      m, n, k, alpha, beta, c, ldc, gemm_cost<T, BM, BN, WM, WN>(), s,
+      [&](dim3 grid, const GemmGrid &g, T *ws) {
+        hipLaunchKernelGGL((k_gemm<T, BM, BN, BK, WM, WN>), grid,
+                           dim3(GemmCfg<T, BM, BN, BK, WM, WN>::kThreads), 0, s, m, n, k, alpha, a,
+                           lda, b, ldb, beta, c, ldc, g, ws);
+      });
 }
 
 // Workgroup tiles (gemm_tile knob):
@@ -635,14 +869,13 @@ void launch_gemm(int64_t m, int64_t n, int64_t k, T alpha, const T *a, int64_t l
 //   5: 256 x 256, eight waves of 64 x 128 (FP32 only; FP64 takes 4)
 //   6, 7: 128 x 128 and 256 x 128 loading stages straight into LDS (FP32;
 //      FP64 has the 128 x 128 one, BK 16, and takes 4 for 7)
-// 0 picks by type and size (measured on 4096^3 .. 16384^3): FP64 takes 6
-// (its direct-to-LDS kernel: 64-68 TFLOP/s against 57-65 for 3); FP32 takes
-// 6 once C holds 4096 tiles of 128 x 128 (about 8192^2), 5 while it holds at
-// least 256 of 256 x 256 (about 4096^2), else 1.
+// 0 picks by type and size (us for n^3, tiles 1 / 2 / 6): FP64 takes 1 (4096:
+// 2081 / 2118 / 2105, 999: 62 / 62 / 78); FP32 takes 2 once C holds 4096 tiles
+// of 128 x 128 (8192: 8064 / 7935 / 8373), else 1 (5000: 2000 / 2022 / 2063,
+// 999: 40.3 / 40.7 / 48.5; rows that are not 16-byte aligned load element by
+// element in 6).
 inline int default_gemm_tile(bool fp64, int64_t m, int64_t n) {
-  if (fp64) return 6;
-  if (((m + 127) / 128) * ((n + 127) / 128) >= 4096) return 6;
-  return ((m + 255) / 256) * ((n + 255) / 256) >= 256 ? 5 : 1;
+  return !fp64 && ((m + 127) / 128) * ((n + 127) / 128) >= 4096 ? 2 : 1;
 }
 
 template <typename T>

@@ -157,3 +157,47 @@ def test_gemm_large_against_fp64_torch(dtype):
     torch.cuda.synchronize()
     err = float(((c.double() - ref).abs() / absref).max())
     assert err <= _bound(n, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("tile", [0, 1, 2, 6])
+@pytest.mark.parametrize("m,n,k", [(1, 3, 4000), (3, 2, 65), (128, 129, 64), (203, 295, 4502),
+                                   (385, 131, 1030), (1000, 999, 97), (257, 256, 2048)])
+def test_gemm_tiles_in_parts_exact(orc, dtype, tile, m, n, k):
+    """Products of fewer tiles than the chip holds: their tiles are cut along
+    k and the parts added (alpha and beta by the reduction), over rows that
+    start at any element, fewer columns than a 16-byte slot, partial last
+    stages, and a last column slot that reaches into the next row (NaN there
+    must not reach C)."""
+    rng = np.random.default_rng(m + 7 * n + k)
+    a = rng.integers(-3, 4, (m, k)).astype(NP[dtype])
+    b = rng.integers(-3, 4, (k, n)).astype(NP[dtype])
+    c = rng.integers(-5, 6, (m, n)).astype(NP[dtype])
+    ref, _ = orc.gemm(a, b, c, alpha=2.0, beta=-1.0)
+    for off in (0, 1):
+        Bd = torch.full((k, n + 2 * off), float("nan"), dtype=dtype, device=DEV)
+        Bd[:, off:off + n] = _dev(b, dtype)
+        cd = _dev(c, dtype)
+        with drx.tuned(gemm_tile=tile):
+            drx.gemm(_dev(a, dtype), Bd[:, off:off + n], cd, alpha=2.0, beta=-1.0)
+        torch.cuda.synchronize()
+        assert np.array_equal(cd.double().cpu().numpy(), ref)
+
+
+def test_gemm_in_parts_captured():
+    """A product whose tiles are cut, captured in a graph (its workspace
+    allocated on the captured stream) and replayed with new inputs."""
+    a = torch.randn(200, 3000, device=DEV)
+    b = torch.randn(3000, 190, device=DEV)
+    c = drx.gemm(a, b)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        drx.gemm(a, b, c, beta=0.0)
+    for i in range(4):
+        a.normal_()
+        eager = drx.gemm(a, b)
+        g.replay()
+        other = drx.gemm(-a, b)
+        torch.cuda.synchronize()
+        assert torch.equal(c, eager) and torch.equal(other, -c)
