@@ -10,26 +10,78 @@
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
+#include <vector>
+
 #include "drx_common.hpp"
 #include "drx_internal.hpp"
 
 namespace drx {
 
+// Row of every entry. A workgroup's kRowIds entries lie in the rows between the
+// first one's and the last one's (found by search); each of these rows marks
+// its first entry in LDS, and a running maximum over the marks gives every
+// entry's row. Searching all rows for each entry took 88-150 us for 20M entries
+// of 600K rows, this 37 us.
+constexpr int kRowIds = 4096;
 template <typename TI>
-__global__ void k_row_ids(const TI *rowptr, int64_t base, int64_t nrows,
-                          int64_t nnz, int sent, TI *rowid) {
-  int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= nnz) return;
-  // last row r with row_begin(r) <= e
-  int64_t lo = 0, hi = nrows - 1;
-  while (lo < hi) {
-    int64_t mid = lo + (hi - lo + 1) / 2;
-    if (row_begin(rowptr, base, nrows, nnz, sent, mid) <= e)
-      lo = mid;
-    else
-      hi = mid - 1;
+__global__ __launch_bounds__(256) void k_row_ids(const TI *rowptr, int64_t base, int64_t nrows,
+                                                 int64_t nnz, int sent, TI *rowid) {
+  __shared__ int64_t bound[2];
+  __shared__ int mark[kRowIds + kRowIds / 16];  // (a lane's 16 marks, padded against bank conflicts)
+  auto at_mark = [](int e) { return e + e / 16; };
+  __shared__ int top[4];
+  constexpr int PER = kRowIds / 256;
+  const int tid = threadIdx.x;
+  const int64_t e0 = static_cast<int64_t>(blockIdx.x) * kRowIds;
+  const int64_t e1 = e0 + kRowIds < nnz ? e0 + kRowIds : nnz;
+  if ((tid & 63) == 0 && tid < 128) {
+    const int64_t e = tid == 0 ? e0 : e1 - 1;
+    int64_t lo = 0, hi = nrows - 1;  // last row r with row_begin(r) <= e
+    while (lo < hi) {
+      const int64_t mid = lo + (hi - lo + 1) / 2;
+      if (row_begin(rowptr, base, nrows, nnz, sent, mid) <= e)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    bound[tid >> 6] = lo;
   }
-  rowid[e] = static_cast<TI>(lo);
+#pragma unroll
+  for (int k = 0; k < PER; k++) mark[at_mark(tid + 256 * k)] = 0;
+  __syncthreads();
+  const int64_t lo = bound[0], hi = bound[1];
+  // (of rows that start together, the last one holds the entry)
+  for (int64_t r = lo + 1 + tid; r <= hi; r += 256) {
+    const int64_t at = row_begin(rowptr, base, nrows, nnz, sent, r) - e0;
+    if (at >= 0 && at < kRowIds) atomicMax(&mark[at_mark(static_cast<int>(at))], static_cast<int>(r - lo));
+  }
+  __syncthreads();
+  int run = 0;
+#pragma unroll
+  for (int k = 0; k < PER; k++) run = max(run, mark[at_mark(tid * PER + k)]);
+  const int lane = tid & 63;
+#pragma unroll
+  for (int o = 1; o < 64; o *= 2) {
+    const int t = __shfl_up(run, o, 64);
+    if (lane >= o) run = max(run, t);
+  }
+  if (lane == 63) top[tid >> 6] = run;
+  int before = __shfl_up(run, 1, 64);
+  if (lane == 0) before = 0;
+  __syncthreads();
+  for (int w = 0; w < (tid >> 6); w++) before = max(before, top[w]);
+  // the lane's running maxima back to LDS, then stored in entry order
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    before = max(before, mark[at_mark(tid * PER + k)]);
+    mark[at_mark(tid * PER + k)] = before;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    const int64_t e = e0 + tid + 256 * k;
+    if (e < e1) rowid[e] = static_cast<TI>(lo + mark[at_mark(tid + 256 * k)]);
+  }
 }
 
 template <typename TI>
@@ -79,60 +131,66 @@ static void build_transpose(Transpose &t, const Plan &p, const TI *colind,
   const int64_t nnz = p.nnz, ncols = p.ncols;
   const int tpb = 256;
   const size_t isz = sizeof(TI);
-  DRX_HIP(hipMalloc(&t.colptr, (ncols + 1) * isz));
-  DRX_HIP(hipMalloc(&t.rowind, std::max<int64_t>(nnz, 1) * isz));
-  DRX_HIP(hipMalloc(&t.perm, std::max<int64_t>(nnz, 1) * isz));
+  DRX_HIP(hipGetDevice(&t.device));
+  t.colptr = block_alloc((ncols + 1) * isz);
+  t.rowind = block_alloc(nnz * isz);
+  t.perm = block_alloc(nnz * isz);
+  std::vector<void *> tmp;
   if (nnz > 0) {
-    TI *rowid = nullptr, *keys_out = nullptr, *iota = nullptr;
-    DRX_HIP(hipMalloc(&rowid, nnz * isz));
-    DRX_HIP(hipMalloc(&keys_out, nnz * isz));
-    DRX_HIP(hipMalloc(&iota, nnz * isz));
-    hipLaunchKernelGGL(k_row_ids<TI>, dim3(blocks_for(nnz, tpb)), dim3(tpb), 0,
-                       s, static_cast<const TI *>(p.rowptr), p.base, p.nrows,
-                       nnz, p.has_sentinel, rowid);
-    hipLaunchKernelGGL(k_iota<TI>, dim3(blocks_for(nnz, tpb)), dim3(tpb), 0, s,
-                       iota, nnz);
-    int end_bit = 1;
-    while (end_bit < static_cast<int>(8 * isz) &&
-           (int64_t(1) << end_bit) < std::max<int64_t>(ncols, 2))
-      end_bit++;
-    size_t temp_bytes = 0;
-    DRX_HIP(hipcub::DeviceRadixSort::SortPairs(
-        nullptr, temp_bytes, colind, keys_out, iota, static_cast<TI *>(t.perm),
-        static_cast<int>(nnz), 0, end_bit, s));
-    void *temp = nullptr;
-    DRX_HIP(hipMalloc(&temp, std::max<size_t>(temp_bytes, 1)));
-    DRX_HIP(hipcub::DeviceRadixSort::SortPairs(
-        temp, temp_bytes, colind, keys_out, iota, static_cast<TI *>(t.perm),
-        static_cast<int>(nnz), 0, end_bit, s));
-    hipLaunchKernelGGL(k_colptr<TI>, dim3(blocks_for(ncols + 1, tpb)),
-                       dim3(tpb), 0, s, keys_out, nnz, ncols,
-                       static_cast<TI *>(t.colptr));
-    hipLaunchKernelGGL(k_gather_rows<TI>, dim3(blocks_for(nnz, tpb)), dim3(tpb),
-                       0, s, rowid, static_cast<const TI *>(t.perm), nnz,
-                       static_cast<TI *>(t.rowind));
-    DRX_HIP(hipGetLastError());
-    DRX_HIP(hipStreamSynchronize(s));
-    (void)hipFree(temp);
-    (void)hipFree(rowid);
-    (void)hipFree(keys_out);
-    (void)hipFree(iota);
+    auto temp = [&](size_t bytes) {
+      void *q = block_alloc(bytes);
+      tmp.push_back(q);
+      return q;
+    };
+    try {
+      TI *rowid = static_cast<TI *>(temp(nnz * isz));
+      TI *keys_out = static_cast<TI *>(temp(nnz * isz));
+      TI *iota = static_cast<TI *>(temp(nnz * isz));
+      hipLaunchKernelGGL(k_row_ids<TI>, dim3(blocks_for(nnz, kRowIds)), dim3(tpb), 0, s,
+                         static_cast<const TI *>(p.rowptr), p.base, p.nrows, nnz, p.has_sentinel,
+                         rowid);
+      hipLaunchKernelGGL(k_iota<TI>, dim3(blocks_for(nnz, tpb)), dim3(tpb), 0, s, iota, nnz);
+      int end_bit = 1;
+      while (end_bit < static_cast<int>(8 * isz) &&
+             (int64_t(1) << end_bit) < std::max<int64_t>(ncols, 2))
+        end_bit++;
+      size_t temp_bytes = 0;
+      DRX_HIP(hipcub::DeviceRadixSort::SortPairs(
+          nullptr, temp_bytes, colind, keys_out, iota, static_cast<TI *>(t.perm),
+          static_cast<int>(nnz), 0, end_bit, s));
+      void *work = temp(std::max<size_t>(temp_bytes, 1));
+      DRX_HIP(hipcub::DeviceRadixSort::SortPairs(
+          work, temp_bytes, colind, keys_out, iota, static_cast<TI *>(t.perm),
+          static_cast<int>(nnz), 0, end_bit, s));
+      hipLaunchKernelGGL(k_colptr<TI>, dim3(blocks_for(ncols + 1, tpb)), dim3(tpb), 0, s, keys_out,
+                         nnz, ncols, static_cast<TI *>(t.colptr));
+      hipLaunchKernelGGL(k_gather_rows<TI>, dim3(blocks_for(nnz, tpb)), dim3(tpb), 0, s, rowid,
+                         static_cast<const TI *>(t.perm), nnz, static_cast<TI *>(t.rowind));
+      DRX_HIP(hipGetLastError());
+    } catch (...) {
+      (void)hipStreamSynchronize(s);
+      for (void *q : tmp) block_free(t.device, q);
+      throw;
+    }
   } else {
     DRX_HIP(hipMemsetAsync(t.colptr, 0, (ncols + 1) * isz, s));
-    DRX_HIP(hipStreamSynchronize(s));
   }
-  t.plan = make_plan(p.itype, t.colptr, 0, ncols, p.nrows, nnz, 1, 0, s,
-                     false, false, true);
-  DRX_HIP(hipStreamSynchronize(s));
+  try {
+    t.plan = make_plan(p.itype, t.colptr, 0, ncols, p.nrows, nnz, 1, 0, s,
+                       false, false, true);
+    DRX_HIP(hipStreamSynchronize(s));
+  } catch (...) {
+    (void)hipStreamSynchronize(s);
+    for (void *q : tmp) block_free(t.device, q);
+    throw;
+  }
+  for (void *q : tmp) block_free(t.device, q);
 }
 
 static void free_transpose(Transpose *t) {
   if (!t) return;
   if (t->plan) free_plan(t->plan, nullptr);
-  if (t->colptr) (void)hipFree(t->colptr);
-  if (t->rowind) (void)hipFree(t->rowind);
-  if (t->perm) (void)hipFree(t->perm);
-  if (t->tvals) (void)hipFree(t->tvals);
+  owned_free(t->device, {t->colptr, t->rowind, t->perm, t->tvals});
   delete t;
 }
 
@@ -191,9 +249,9 @@ int drx_transpose_set_values(drx_transpose t, int vtype, const void *vals,
     DRX_REQUIRE(vtype >= DRX_F64 && vtype <= DRX_F16, "bad vtype");
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (tt->tvals == nullptr || tt->tvtype != vtype) {
-      if (tt->tvals) (void)hipFree(tt->tvals);
+      owned_free(tt->device, {tt->tvals});
       tt->tvals = nullptr;
-      DRX_HIP(hipMalloc(&tt->tvals, std::max<int64_t>(nnz, 1) * dtype_size(vtype)));
+      tt->tvals = block_alloc(nnz * dtype_size(vtype));
       tt->tvtype = vtype;
     }
     if (nnz == 0) return;

@@ -5,6 +5,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <initializer_list>
 
 namespace drx {
 
@@ -35,6 +36,9 @@ struct Plan {
   int64_t nblocks_wide = 0;
   // Longest row of the share (-1: not measured); sets the block pitch.
   int64_t lmax = -1;
+  // What holds the records: a block, or (owns_async) memory of one call that
+  // is freed on its stream; null where the caller's buffer does.
+  void *rec_mem = nullptr;
   bool owns_async = false;
   int device = 0;
   PanelSet *panels = nullptr;  // column-panel layout (drx_plan_set_panels)
@@ -69,6 +73,7 @@ struct Transpose {
   void *tvals = nullptr;   // nnz, values in CSC order (drx_transpose_set_values)
   int tvtype = -1;         // dtype of tvals
   int itype = 0;
+  int device = 0;
 };
 
 int64_t tuned_block_nnz();
@@ -102,7 +107,8 @@ int tuned_fwd_cap();
 // lengths and column locality, 2 always.
 int tuned_rowgather();
 
-// Stream-ordered scratch from the library's per-device pool.
+// Stream-ordered scratch from the library's per-device pool, which keeps up to
+// kPoolKeep bytes (and the reserves below) of unused memory.
 void *scratch_alloc(size_t bytes, hipStream_t s);
 void scratch_free(void *p, hipStream_t s);
 // An object whose products take `bytes` of scratch at once: scratch_reserve
@@ -111,6 +117,14 @@ void scratch_free(void *p, hipStream_t s);
 // to the largest reserve left.
 void scratch_reserve(int dev, size_t bytes, hipStream_t s);
 void scratch_unreserve(int dev, size_t bytes);
+// Device memory of objects (plans, transposes, panels) and of their building.
+// A block may be given back only when no work that uses it is left on the GPU,
+// so a kept block serves any stream at once. At most kBlocksKeep bytes are kept
+// per device; a failed allocation gives all of them back and tries again.
+void *block_alloc(size_t bytes);
+void block_free(int dev, void *p);
+// Blocks that any stream may have used: waits for the device, as hipFree does.
+void owned_free(int dev, std::initializer_list<void *> ptrs);
 
 // Row-major chunks of x for k >= 2 right-hand sides: chunk width KP and the
 // bytes of all chunks; the copy kernel.

@@ -14,8 +14,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <list>
+#include <map>
 #include <mutex>
 #include <set>
+#include <unordered_map>
 
 #include "drx_common.hpp"
 #include "drx_fwd.hpp"
@@ -24,12 +27,14 @@
 namespace drx {
 
 // ---------------------------------------------------------------------------
-// Scratch: one memory pool per device, created on first use, that keeps its
-// memory across calls (release threshold = max), so that steady-state calls
-// reuse it without reaching the driver's allocator. Allocation and release
+// Scratch: one memory pool per device, created on first use, that keeps up to
+// kPoolKeep bytes across calls (plus the largest reserve), so that steady-state
+// calls reuse it without reaching the driver's allocator. Allocation and release
 // are ordered on the caller's stream.
 // ---------------------------------------------------------------------------
 constexpr int kMaxDevices = 64;
+constexpr size_t kPoolKeep = size_t(8) << 30;
+constexpr size_t kBlocksKeep = size_t(4) << 30;
 static std::mutex g_pool_mu;
 static hipMemPool_t g_pools[kMaxDevices];
 static std::multiset<size_t> g_reserved[kMaxDevices];
@@ -45,7 +50,7 @@ static hipMemPool_t pool_for(int dev) {
     props.location.id = dev;
     hipMemPool_t pool = nullptr;
     DRX_HIP(hipMemPoolCreate(&pool, &props));
-    uint64_t keep = UINT64_MAX;
+    uint64_t keep = kPoolKeep;
     DRX_HIP(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
     g_pools[dev] = pool;
   }
@@ -64,21 +69,107 @@ void scratch_free(void *p, hipStream_t s) {
   if (p) (void)hipFreeAsync(p, s);
 }
 
+// What device dev's pool keeps when it releases memory (with g_pool_mu held).
+static size_t set_keep(int dev) {
+  const auto &r = g_reserved[dev];
+  uint64_t keep = kPoolKeep + (r.empty() ? size_t(0) : *r.rbegin());
+  if (g_pools[dev])
+    (void)hipMemPoolSetAttribute(g_pools[dev], hipMemPoolAttrReleaseThreshold, &keep);
+  return static_cast<size_t>(keep);
+}
+
 void scratch_reserve(int dev, size_t bytes, hipStream_t s) {
-  void *p = scratch_alloc(bytes, s);
-  scratch_free(p, s);
+  scratch_free(scratch_alloc(bytes, s), s);
   std::lock_guard<std::mutex> lk(g_pool_mu);
   g_reserved[dev].insert(bytes);
+  set_keep(dev);
 }
 
 void scratch_unreserve(int dev, size_t bytes) {
-  constexpr size_t kKeep = size_t(256) << 20;  // small products' scratch
   std::lock_guard<std::mutex> lk(g_pool_mu);
   auto &r = g_reserved[dev];
   const auto at = r.find(bytes);
   if (at != r.end()) r.erase(at);
-  if (g_pools[dev])
-    (void)hipMemPoolTrimTo(g_pools[dev], std::max(kKeep, r.empty() ? size_t(0) : *r.rbegin()));
+  if (g_pools[dev]) (void)hipMemPoolTrimTo(g_pools[dev], set_keep(dev));
+}
+
+// ---------------------------------------------------------------------------
+// Blocks (block_alloc): mapping and unmapping the 0.5 GB that the plan and the
+// transpose of 20M entries take cost 14 ms beside 1.2 ms of kernels, and the
+// pool above unmaps freed memory whenever it holds more of it than is in use.
+// ---------------------------------------------------------------------------
+struct Blocks {
+  std::mutex mu;
+  std::unordered_map<void *, size_t> size;      // every block handed out or kept
+  std::multimap<size_t, void *> kept;           // by size
+  std::list<void *> order;                      // kept ones, oldest first
+  size_t total = 0;                             // bytes kept
+  void drop(void *p) {  // a kept block goes back to the driver
+    const size_t n = size[p];
+    for (auto it = kept.lower_bound(n); it != kept.end() && it->first == n; ++it)
+      if (it->second == p) {
+        kept.erase(it);
+        break;
+      }
+    order.remove(p);
+    total -= n;
+    size.erase(p);
+    (void)hipFree(p);
+  }
+};
+static Blocks g_blocks[kMaxDevices];
+
+void *block_alloc(size_t bytes) {
+  int dev = 0;
+  DRX_HIP(hipGetDevice(&dev));
+  DRX_REQUIRE(dev >= 0 && dev < kMaxDevices, "device ordinal out of range");
+  bytes = (std::max<size_t>(bytes, 1) + 4095) & ~size_t(4095);
+  Blocks &b = g_blocks[dev];
+  std::lock_guard<std::mutex> lk(b.mu);
+  // a kept block of at most a quarter (small ones: 64 KB) more
+  const auto it = b.kept.lower_bound(bytes);
+  if (it != b.kept.end() && it->first <= bytes + std::max<size_t>(bytes / 4, 65536)) {
+    void *p = it->second;
+    b.total -= it->first;
+    b.kept.erase(it);
+    b.order.remove(p);
+    return p;
+  }
+  void *p = nullptr;
+  hipError_t e = hipMalloc(&p, bytes);
+  if (e == hipErrorOutOfMemory && b.total > 0) {
+    (void)hipGetLastError();
+    while (!b.order.empty()) b.drop(b.order.front());
+    e = hipMalloc(&p, bytes);
+  }
+  DRX_HIP(e);
+  b.size[p] = bytes;
+  return p;
+}
+
+void block_free(int dev, void *p) {
+  if (p == nullptr || dev < 0 || dev >= kMaxDevices) return;
+  Blocks &b = g_blocks[dev];
+  std::lock_guard<std::mutex> lk(b.mu);
+  const auto at = b.size.find(p);
+  if (at == b.size.end()) return;
+  const size_t n = at->second;
+  b.kept.emplace(n, p);
+  b.order.push_back(p);
+  b.total += n;
+  while (b.total > kBlocksKeep) b.drop(b.order.front());
+}
+
+void owned_free(int dev, std::initializer_list<void *> ptrs) {
+  bool any = false;
+  for (void *p : ptrs) any = any || p != nullptr;
+  if (!any) return;
+  int cur = dev;
+  (void)hipGetDevice(&cur);
+  if (cur != dev) (void)hipSetDevice(dev);
+  (void)hipDeviceSynchronize();
+  for (void *p : ptrs) block_free(dev, p);
+  if (cur != dev) (void)hipSetDevice(cur);
 }
 
 // Samples up to 4096 row blocks: the span between the first and the last

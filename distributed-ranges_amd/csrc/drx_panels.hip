@@ -78,10 +78,8 @@ struct PanelSet {
 
 void free_panels(PanelSet *ps) {
   if (!ps) return;
-  for (void *ptr : {(void *)ps->pcol, ps->pval, ps->perm, (void *)ps->seg_row,
-                    (void *)ps->seg_at, (void *)ps->wg_tile, (void *)ps->tile_slice,
-                    (void *)ps->tile_e, (void *)ps->tile_s})
-    if (ptr) (void)hipFree(ptr);
+  owned_free(ps->device, {ps->pcol, ps->pval, ps->perm, ps->seg_row, ps->seg_at, ps->wg_tile,
+                          ps->tile_slice, ps->tile_e, ps->tile_s});
   if (ps->scratch > 0) scratch_unreserve(ps->device, ps->scratch);
   delete ps;
 }
@@ -563,9 +561,7 @@ void run_spmv_panels(const Plan &p, int vtype, const void *colind,
 // Building the layout
 // ---------------------------------------------------------------------------
 template <typename T> static T *dmalloc(int64_t n) {
-  T *p = nullptr;
-  DRX_HIP(hipMalloc(reinterpret_cast<void **>(&p), static_cast<size_t>(std::max<int64_t>(n, 1)) * sizeof(T)));
-  return p;
+  return static_cast<T *>(block_alloc(static_cast<size_t>(n) * sizeof(T)));
 }
 
 // Slice of every entry.
@@ -753,7 +749,7 @@ static void build_panels(Plan &p, PanelSet &ps, const TI *colind, const TV *vals
     tmp.push_back(ptr);
   };
   auto release = [&](void *ptr) {
-    (void)hipFree(ptr);
+    block_free(ps.device, ptr);
     tmp.erase(std::find(tmp.begin(), tmp.end(), ptr));
   };
   try {
@@ -877,10 +873,10 @@ static void build_panels(Plan &p, PanelSet &ps, const TI *colind, const TV *vals
     DRX_HIP(hipStreamSynchronize(s));
   } catch (...) {
     (void)hipStreamSynchronize(s);
-    for (void *q : tmp) (void)hipFree(q);
+    for (void *q : tmp) block_free(ps.device, q);
     throw;
   }
-  for (void *q : tmp) (void)hipFree(q);
+  for (void *q : tmp) block_free(ps.device, q);
 }
 
 // Builds the panel layout of p (drx_plan_set_panels).

@@ -36,16 +36,26 @@ __device__ int64_t first_row_at(const TI *rowptr, int64_t base, int64_t nrows,
   return lo;
 }
 
+// One set of records: blocks starting every `pitch` entries, windows of `cap`.
+struct RecordSet {
+  int64_t pitch, cap, nblocks;
+  BlockRec *rec;
+};
+
+// The records of both sets in one launch (each is a chain of dependent reads:
+// 14 us however few there are).
 template <typename TI>
 __global__ void k_plan_records(const TI *rowptr, int64_t base, int64_t nrows,
-                               int64_t nnz, int sent, int64_t nb_nnz,
-                               int64_t cap, int64_t nblocks, BlockRec *rec) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (c > nblocks) return;
+                               int64_t nnz, int sent, RecordSet a, RecordSet b) {
+  int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const bool second = c > a.nblocks;
+  if (second) c -= a.nblocks + 1;
+  const RecordSet &set = second ? b : a;
+  if (set.rec == nullptr || c > set.nblocks) return;
   auto r_of = [&](int64_t cc) -> int64_t {
     if (cc == 0) return 0;
-    if (cc >= nblocks) return nrows;
-    return first_row_at(rowptr, base, nrows, nnz, sent, cc * nb_nnz);
+    if (cc >= set.nblocks) return nrows;
+    return first_row_at(rowptr, base, nrows, nnz, sent, cc * set.pitch);
   };
   const int64_t r0 = r_of(c);
   const int64_t e0 = row_begin(rowptr, base, nrows, nnz, sent, r0);
@@ -54,24 +64,28 @@ __global__ void k_plan_records(const TI *rowptr, int64_t base, int64_t nrows,
   out.e0 = e0;
   out.es = e0;
   out.pad = 0;
-  if (c < nblocks) {
+  if (c < set.nblocks) {
     const int64_t r1 = r_of(c + 1);
     const int64_t e1 = row_begin(rowptr, base, nrows, nnz, sent, r1);
-    if (r1 > r0 && e1 - e0 > cap - kWinSlack)
+    if (r1 > r0 && e1 - e0 > set.cap - kWinSlack)
       out.es = row_begin(rowptr, base, nrows, nnz, sent, r1 - 1);
     else
       out.es = e1;
   }
-  rec[c] = out;
+  set.rec[c] = out;
 }
 
-// Longest row of the share (clamped to it): one partial maximum per
-// workgroup, then one atomic.
+// Analysis of a share: out = {longest row (clamped to the share), first row
+// offset, last row offset}, one partial maximum per workgroup, then one atomic.
 template <typename TI>
-__global__ void k_max_rowlen(const TI *rowptr, int64_t base, int64_t nrows,
-                             int64_t nnz, int sent, unsigned long long *out) {
+__global__ void k_share_info(const TI *rowptr, int64_t base, int64_t nrows, int64_t nnz, int sent,
+                             unsigned long long *out) {
   __shared__ unsigned long long red[4];
   unsigned long long m = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    out[1] = static_cast<unsigned long long>(static_cast<int64_t>(rowptr[0]));
+    out[2] = static_cast<unsigned long long>(static_cast<int64_t>(rowptr[sent ? nrows : nrows - 1]));
+  }
   for (int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; r < nrows;
        r += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     const int64_t len = row_begin(rowptr, base, nrows, nnz, sent, r + 1) -
@@ -112,74 +126,72 @@ int64_t default_block_nnz(int itype) {
   return 1024;
 }
 
-// Records of blocks starting every `nb` entries with windows of `cap`
-// entries into a new array, or into `into` (caller-owned, at least
-// nblocks + 1 records) when it is given.
-static BlockRec *make_records(const Plan &p, int64_t nb, int64_t cap, int64_t *nblocks,
-                              hipStream_t s, bool async_alloc, BlockRec *into = nullptr) {
-  *nblocks = p.nnz / nb + 1;
-  const size_t bytes = static_cast<size_t>(*nblocks + 1) * sizeof(BlockRec);
-  BlockRec *rec = into;
-  if (rec != nullptr) {
-  } else if (async_alloc)
-    DRX_HIP(hipMallocAsync(reinterpret_cast<void **>(&rec), bytes, s));
-  else
-    DRX_HIP(hipMalloc(reinterpret_cast<void **>(&rec), bytes));
-  const int tpb = 256;
-  const int64_t n = *nblocks + 1;
-  const dim3 grid(static_cast<unsigned>((n + tpb - 1) / tpb));
-  if (p.itype == DRX_I32)
-    hipLaunchKernelGGL(k_plan_records<int32_t>, grid, dim3(tpb), 0, s,
-                       static_cast<const int32_t *>(p.rowptr), p.base, p.nrows,
-                       p.nnz, p.has_sentinel, nb, cap, *nblocks, rec);
-  else
-    hipLaunchKernelGGL(k_plan_records<int64_t>, grid, dim3(tpb), 0, s,
-                       static_cast<const int64_t *>(p.rowptr), p.base, p.nrows,
-                       p.nnz, p.has_sentinel, nb, cap, *nblocks, rec);
-  DRX_HIP(hipGetLastError());
-  return rec;
-}
-
-// The plan's records, and the records of twice as large blocks (window
-// 4096) that the forward kernel uses for 4-byte values when the plan's
-// block is 1024 entries.
 // The plan's records (windows of 2 block_nnz entries), and for the default
 // 1024-entry blocks the records of windows of 4096 that the forward kernel
-// uses for 4-byte values.
-static void build_records(Plan &p, hipStream_t s, bool async_alloc) {
+// uses for 4-byte values, one set after the other from `at` on.
+static void make_records(Plan &p, BlockRec *at, hipStream_t s) {
   p.cap = 2 * p.block_nnz;
-  p.owns_async = async_alloc;
-  p.rec = make_records(p, block_pitch(p, p.cap), p.cap, &p.nblocks, s, async_alloc);
-  if (p.block_nnz == 1024)
-    p.rec_wide = make_records(p, block_pitch(p, 4096), 4096, &p.nblocks_wide, s, async_alloc);
+  RecordSet a{block_pitch(p, p.cap), p.cap, 0, at}, b{1, 4096, -1, nullptr};
+  a.nblocks = p.nnz / a.pitch + 1;
+  p.rec = at;
+  p.nblocks = a.nblocks;
+  if (p.block_nnz == 1024) {
+    b.pitch = block_pitch(p, 4096);
+    b.nblocks = p.nnz / b.pitch + 1;
+    b.rec = at + a.nblocks + 1;
+    p.rec_wide = b.rec;
+    p.nblocks_wide = b.nblocks;
+  }
+  const int64_t n = a.nblocks + 1 + b.nblocks + 1;
+  const dim3 grid(static_cast<unsigned>((n + 63) / 64));
+  if (p.itype == DRX_I32)
+    hipLaunchKernelGGL(k_plan_records<int32_t>, grid, dim3(64), 0, s,
+                       static_cast<const int32_t *>(p.rowptr), p.base, p.nrows, p.nnz,
+                       p.has_sentinel, a, b);
+  else
+    hipLaunchKernelGGL(k_plan_records<int64_t>, grid, dim3(64), 0, s,
+                       static_cast<const int64_t *>(p.rowptr), p.base, p.nrows, p.nnz,
+                       p.has_sentinel, a, b);
+  DRX_HIP(hipGetLastError());
 }
 
-// Longest row of p's share (waits for the stream).
-static int64_t max_row_len(const Plan &p, hipStream_t s) {
-  if (p.nrows == 0) return 0;
-  unsigned long long *d = static_cast<unsigned long long *>(
-      scratch_alloc(sizeof(unsigned long long), s));
-  unsigned long long h = 0;
+// Longest row of p's share (waits for the stream); with `validate` its first
+// and last row offsets must bracket the share.
+static int64_t analyse(const Plan &p, bool validate, hipStream_t s) {
+  if (p.nrows == 0) {
+    DRX_HIP(hipStreamSynchronize(s));
+    return 0;
+  }
+  unsigned long long *d =
+      static_cast<unsigned long long *>(block_alloc(3 * sizeof(unsigned long long)));
+  unsigned long long h[3] = {0, 0, 0};
   try {
     DRX_HIP(hipMemsetAsync(d, 0, sizeof(unsigned long long), s));
-    const int64_t nb = std::min<int64_t>((p.nrows + 255) / 256, 4096);
+    const int64_t nb = std::min<int64_t>((p.nrows + 255) / 256, 512);
     if (p.itype == DRX_I32)
-      hipLaunchKernelGGL(k_max_rowlen<int32_t>, dim3(static_cast<unsigned>(nb)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_share_info<int32_t>, dim3(static_cast<unsigned>(nb)), dim3(256), 0, s,
                          static_cast<const int32_t *>(p.rowptr), p.base, p.nrows, p.nnz,
                          p.has_sentinel, d);
     else
-      hipLaunchKernelGGL(k_max_rowlen<int64_t>, dim3(static_cast<unsigned>(nb)), dim3(256), 0, s,
+      hipLaunchKernelGGL(k_share_info<int64_t>, dim3(static_cast<unsigned>(nb)), dim3(256), 0, s,
                          static_cast<const int64_t *>(p.rowptr), p.base, p.nrows, p.nnz,
                          p.has_sentinel, d);
     DRX_HIP(hipGetLastError());
-    DRX_HIP(hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, s));
+    DRX_HIP(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
     DRX_HIP(hipStreamSynchronize(s));
   } catch (...) {
-    scratch_free(d, s);
+    owned_free(p.device, {d});
     throw;
   }
-  scratch_free(d, s);
-  return static_cast<int64_t>(h);
+  block_free(p.device, d);
+  if (validate) {
+    const int64_t first = static_cast<int64_t>(h[1]), last = static_cast<int64_t>(h[2]);
+    DRX_REQUIRE(first - p.base <= p.nnz && last >= first,
+                "rowptr does not bracket the share (check rowptr_base/nnz)");
+    if (p.has_sentinel)
+      DRX_REQUIRE(last - p.base <= p.nnz, "rowptr[nrows] - rowptr_base exceeds nnz");
+  }
+  return static_cast<int64_t>(h[0]);
 }
 
 int64_t records_needed(int64_t nnz, int64_t block_nnz) {
@@ -219,35 +231,21 @@ Plan *make_plan(int itype, const void *rowptr, int64_t base, int64_t nrows,
   p->block_nnz = block_nnz > 0 ? block_nnz : default_block_nnz(itype);
   try {
     DRX_HIP(hipGetDevice(&p->device));
-    if (validate && nrows > 0) {
-      // The first and last row offsets must bracket the share.
-      const size_t isz = itype == DRX_I32 ? 4 : 8;
-      const int64_t lastidx = sent ? nrows : nrows - 1;
-      unsigned char buf[16] = {0};
-      DRX_HIP(hipMemcpyAsync(buf, rowptr, isz, hipMemcpyDeviceToHost, s));
-      DRX_HIP(hipMemcpyAsync(buf + 8,
-                             static_cast<const char *>(rowptr) + lastidx * isz,
-                             isz, hipMemcpyDeviceToHost, s));
-      DRX_HIP(hipStreamSynchronize(s));
-      int64_t first = 0, lastv = 0;
-      if (isz == 4) {
-        int32_t a, b;
-        std::memcpy(&a, buf, 4);
-        std::memcpy(&b, buf + 8, 4);
-        first = a;
-        lastv = b;
-      } else {
-        std::memcpy(&first, buf, 8);
-        std::memcpy(&lastv, buf + 8, 8);
-      }
-      DRX_REQUIRE(first - base <= nnz && lastv >= first,
-                  "rowptr does not bracket the share (check rowptr_base/nnz)");
-      if (sent)
-        DRX_REQUIRE(lastv - base <= nnz,
-                    "rowptr[nrows] - rowptr_base exceeds nnz");
+    if (!async_alloc) {
+      // room for the most records the share can need: the pitch of filled
+      // windows is at least kWinSlack below half a window
+      const int64_t most = nnz / (p->block_nnz - kWinSlack) + 2 + nnz / (2048 - kWinSlack) + 2;
+      p->rec_mem = block_alloc(static_cast<size_t>(most) * sizeof(BlockRec));
+      const int64_t lmax = analyse(*p, validate, s);
+      if (fill) p->lmax = lmax;
+    } else {
+      DRX_HIP(hipMallocAsync(&p->rec_mem,
+                             static_cast<size_t>(records_needed(nnz, p->block_nnz)) *
+                                 sizeof(BlockRec),
+                             s));
+      p->owns_async = true;
     }
-    if (fill) p->lmax = max_row_len(*p, s);
-    build_records(*p, s, async_alloc);
+    make_records(*p, static_cast<BlockRec *>(p->rec_mem), s);
   } catch (...) {
     free_plan(p, s);
     throw;
@@ -272,20 +270,16 @@ void init_plan_in(Plan &p, int itype, const void *rowptr, int64_t base, int64_t 
   DRX_REQUIRE(records_needed(nnz, p.block_nnz) <= buf_records,
               "the share needs more plan records than the buffer holds");
   DRX_HIP(hipGetDevice(&p.device));
-  p.rec = make_records(p, p.block_nnz, p.cap, &p.nblocks, s, false, buf);
-  p.rec_wide = make_records(p, 2048, 4096, &p.nblocks_wide, s, false, buf + p.nblocks + 1);
+  make_records(p, buf, s);
 }
 
 void free_plan(Plan *p, hipStream_t s) {
   if (!p) return;
   if (p->panels) free_panels(p->panels);
-  for (BlockRec *r : {p->rec, p->rec_wide}) {
-    if (!r) continue;
-    if (p->owns_async)
-      (void)hipFreeAsync(r, s);
-    else
-      (void)hipFree(r);
-  }
+  if (!p->owns_async)
+    owned_free(p->device, {p->rec_mem});
+  else if (p->rec_mem)
+    (void)hipFreeAsync(p->rec_mem, s);
   delete p;
 }
 

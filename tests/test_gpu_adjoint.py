@@ -40,6 +40,58 @@ def test_transpose_structure_bitexact(orc, itype):
     assert np.array_equal(pm.cpu().numpy(), opm)
 
 
+@pytest.mark.parametrize("itype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("base", [0, 7])
+def test_transpose_of_rows_around_chunks(orc, itype, base):
+    """Rows of the transposed structure's row ids: rows that end at and around
+    multiples of 4096 entries, one over several such chunks, runs of empty
+    rows longer than a chunk, and a share that starts at an offset."""
+    rng = np.random.default_rng(11)
+    lens = ([0] * 5000 + [4095, 1, 4096, 1, 0, 4097, 0, 9000, 2] + [0] * 9000 + [1] * 3000 +
+            list(rng.integers(0, 4, 6000)) + [4096, 0, 0, 3])
+    n = 10007
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    ci = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens if L])
+    ocp, ori, opm = orc.transpose(rp, ci, n)
+    rpd = torch.as_tensor(rp + base).to(itype).to(DEV)
+    cid = torch.as_tensor(ci).to(itype).to(DEV)
+    A = drx.CsrMatrix(rpd, cid, torch.ones(ci.size, device=DEV), (len(lens), n), base=base)
+    for got, want in zip(A.transpose().arrays(), (ocp, ori, opm)):
+        assert np.array_equal(got.cpu().numpy(), want)
+    A.close()
+
+
+def test_new_matrices_reuse_memory(orc):
+    """Matrices made, used and closed one after another on alternating
+    streams take over each other's memory (plan records, transposes), sizes
+    up and down, two alive at a time; their products stay right."""
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    alive = []
+    for i, m in enumerate([4000, 200, 9000, 8800, 300, 9100, 50]):
+        A = rand_csr(m, m // 2 + 7, 0.01, i)
+        v = A.data.astype(np.float32)
+        x = np.random.default_rng(i).uniform(-1, 1, A.shape[1]).astype(np.float32)
+        dy = np.random.default_rng(i + 50).uniform(-1, 1, m).astype(np.float32)
+        with torch.cuda.stream(streams[i % 2]):
+            Ad = drx.from_host(A.indptr, A.indices, v, A.shape)
+            y = Ad.matvec(torch.as_tensor(x).to(DEV))
+            dx = Ad.rmatvec(torch.as_tensor(dy).to(DEV))
+            Ad.set_transposed_values()
+            dx2 = Ad.rmatvec(torch.as_tensor(dy).to(DEV))
+        alive.append((Ad, A, v, x, dy, y, dx, dx2))
+        if len(alive) == 3:
+            alive.pop(0)[0].close()  # (its work may still be queued)
+        torch.cuda.synchronize()
+        for _, B, w, xb, dyb, yb, dxb, dxb2 in alive:
+            ys, absy = orc.spmv(B.indptr, B.indices, w, xb)
+            assert componentwise_err(yb.cpu().numpy(), ys, absy) < 1e-5
+            ref, absr = orc.spmv_t(B.indptr, B.indices, w, dyb, B.shape[1])
+            assert componentwise_err(dxb.cpu().numpy(), ref, absr) < 1e-5
+            assert torch.equal(dxb, dxb2)
+    for a in alive:
+        a[0].close()
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("k", [1, 4, 11])
 def test_adjoint_matches_oracle(orc, dtype, k):
