@@ -163,7 +163,7 @@ void k_batch_mrhs(const FwdArgs *items,
                                                    const int *modes,
                                                    const int64_t *off,
                                                    int64_t nitems, int64_t total) {
-  __shared__ MrhsSmem<WG, CAP, TA> sm;
+  __shared__ MrhsSmem<WG, CAP, KP, TA> sm;
   const int64_t per_xcd = (total + kXcds - 1) / kXcds;
   const int64_t xcd = blockIdx.x % kXcds;
   const int64_t lw = blockIdx.x / kXcds, nw = gridDim.x / kXcds;
@@ -526,6 +526,7 @@ int drx_batch_create(drx_batch *out, int64_t nitems, const drx_batch_item *items
       b->ytype = ytype;
       b->k = k;
       b->mrhs = k >= 2 && tuned_mrhs() != 0;
+      b->gshift = b->mrhs ? tuned_mrhs_gshift() : 0;
       b->kp = b->mrhs ? mrhs_kp(k, xtype, tuned_mrhs_kp_max() == 8) : 0;
       b->alpha = alpha;
       b->beta = beta;

@@ -845,11 +845,18 @@ void k_spmv_rows(FwdArgs a) {
 // ---------------------------------------------------------------------------
 namespace drx {
 
-template <int WG, int CAP, typename TA> struct MrhsSmem {
+// Sums of rows that a block stages in LDS before it writes them: sixteen 4-byte
+// sums per row, 8 KB (five workgroups per CU, as the registers allow).
+template <int KP, typename TA> constexpr int mrhs_staged() {
+  return KP == 16 && sizeof(TA) == 4 ? 2048 : 0;
+}
+
+template <int WG, int CAP, int KP, typename TA> struct MrhsSmem {
   TA v[CAP];
   uint32_t c[CAP];
   int rp_s[CAP / 2 + 1];
   TA red[16 * (WG / 64)];
+  TA yb[mrhs_staged<KP, TA>()];  // rows of KP sums, padded by one
 };
 
 // KP consecutive x values (one xr row) converted to the accumulator type.
@@ -912,8 +919,7 @@ __device__ __forceinline__ void reduce_rows_mrhs(
       const TA v0 = v_s[q], v1 = v_s[q + G];
 #pragma unroll
       for (int jj = 0; jj < KP; jj++) {
-        acc[jj] += v0 * x0[jj];
-        acc[jj] += v1 * x1[jj];
+        acc[jj] += v0 * x0[jj] + v1 * x1[jj];
       }
     }
     if (q < e) {
@@ -946,12 +952,13 @@ __device__ __forceinline__ void reduce_rows_mrhs(
 // lane shuffles (stride S). Holding the whole KP-vector per lane (16 sums
 // and 16 values per entry in flight for FP32 k = 16) limited the batched
 // kernel to two waves per SIMD with two entries in flight per lane.
-template <int WG, int G, int KP, typename TX, typename TY, typename TA,
+// STAGE: the sums of row i go to yb[i * (KP + 1) + column] instead of y.
+template <int WG, int G, int KP, bool STAGE, typename TX, typename TY, typename TA,
           typename TI>
 __device__ __forceinline__ void reduce_rows_mrhs_split(
     const TA *v_s, const uint32_t *c_s, const int *rp_s, bool rows_lds,
-    const FwdArgs &a, int64_t r0, int64_t e0, int64_t nr, const TX *xrc,
-    int64_t j0, int kk, TA alpha, TA beta, int tid) {
+    const FwdArgs &a, int64_t r0, int64_t e0, std::conditional_t<STAGE, int, int64_t> nr, const TX *xrc,
+    int64_t j0, int kk, TA alpha, TA beta, TA *yb, int tid) {
   constexpr int KL = 16 / static_cast<int>(sizeof(TX));
   constexpr int S = KP / KL;
   constexpr int GS = G * S;
@@ -960,7 +967,7 @@ __device__ __forceinline__ void reduce_rows_mrhs_split(
   TY *y = static_cast<TY *>(a.y);
   const int lg = tid & (GS - 1);
   const int sub = lg % S, el = lg / S;
-  for (int64_t i = tid / GS; i < nr; i += WG / GS) {
+  for (std::conditional_t<STAGE, int, int64_t> i = tid / GS; i < nr; i += WG / GS) {
     int s, e;
     if (rows_lds) {
       s = rp_s[i];
@@ -983,25 +990,36 @@ __device__ __forceinline__ void reduce_rows_mrhs_split(
       const TA v0 = v_s[q], v1 = v_s[q + G], v2 = v_s[q + 2 * G], v3 = v_s[q + 3 * G];
 #pragma unroll
       for (int j = 0; j < KL; j++) {
-        acc[j] += v0 * x0[j];
-        acc[j] += v1 * x1[j];
-        acc[j] += v2 * x2[j];
-        acc[j] += v3 * x3[j];
+        // (pairwise: a lane that takes more of a row's entries one after
+        // another would round more often)
+        acc[j] += (v0 * x0[j] + v1 * x1[j]) + (v2 * x2[j] + v3 * x3[j]);
       }
     }
-    for (; q < e; q += G) {
-      TA x0[KL];
-      load_xrow<KL>(xs + static_cast<size_t>(c_s[q]) * KP, x0);
-      const TA v0 = v_s[q];
+    if (q < e) {
+      TA rest[KL];
 #pragma unroll
-      for (int j = 0; j < KL; j++) acc[j] += v0 * x0[j];
+      for (int j = 0; j < KL; j++) rest[j] = 0;
+      for (; q < e; q += G) {
+        TA x0[KL];
+        load_xrow<KL>(xs + static_cast<size_t>(c_s[q]) * KP, x0);
+        const TA v0 = v_s[q];
+#pragma unroll
+        for (int j = 0; j < KL; j++) rest[j] += v0 * x0[j];
+      }
+#pragma unroll
+      for (int j = 0; j < KL; j++) acc[j] += rest[j];
     }
 #pragma unroll
     for (int o = S; o < GS; o *= 2) {
 #pragma unroll
       for (int j = 0; j < KL; j++) acc[j] += __shfl_xor(acc[j], o, 64);
     }
-    if (el == 0) {
+    if (STAGE) {
+      if (el == 0) {
+#pragma unroll
+        for (int j = 0; j < KL; j++) yb[i * (KP + 1) + sub * KL + j] = acc[j];
+      }
+    } else if (el == 0) {
       const int64_t row = r0 + i;
 #pragma unroll
       for (int j = 0; j < KL; j++) {
@@ -1127,9 +1145,16 @@ template <int WG, int KP, typename TX, typename TY, typename TA, typename TI>
 __device__ __forceinline__ void reduce_rows_mrhs_any(
     int n_s, const TA *v_s, const uint32_t *c_s, const int *rp_s,
     bool rows_lds, const FwdArgs &a, int64_t r0, int64_t e0, int64_t nr,
-    const TX *xrc, int64_t j0, int kk, TA alpha, TA beta, TA *red, int tid) {
+    const TX *xrc, int64_t j0, int kk, TA alpha, TA beta, TA *red, TA *yb, int tid) {
   if (nr <= 0) return;
-  const int64_t avg = (n_s / nr) >> a.gshift;
+  // Few lanes per row, each with several entries in flight, use the gathers'
+  // slots best. us, thresholds as written / halved / quartered: 64 matrices of
+  // up to 200K rows of 3..64 entries, k = 16, 7408 / 5753 / 5185; band +-16, 2M
+  // rows, k = 8, FP32 399 / 261 / 224, FP64 752 / 495 / 423. gshift 1 is the
+  // default. (More entries in flight by masked or repeated ones in the last
+  // round lose: the gathers are bound by the misses that a CU's L1 keeps in
+  // flight, about 95, each 240 cycles from L2 and 900 from beyond.)
+  const int64_t avg = (n_s / nr) >> (a.gshift + 1);
   if (nr < WG / 64 && n_s / nr > 96) {
     reduce_rows_mrhs_wg<WG, KP, TX, TY, TA, TI>(v_s, c_s, rp_s, rows_lds, a, r0, e0, nr, xrc, j0,
                                                kk, alpha, beta, red, tid);
@@ -1142,7 +1167,40 @@ __device__ __forceinline__ void reduce_rows_mrhs_any(
     constexpr int GMAX = 64 / (KP / KL);
     constexpr int G2 = 2 < GMAX ? 2 : GMAX, G4 = 4 < GMAX ? 4 : GMAX;
     constexpr int G8 = 8 < GMAX ? 8 : GMAX, G16 = 16 < GMAX ? 16 : GMAX;
-#define DRX_RS(G) reduce_rows_mrhs_split<WG, G, KP, TX, TY, TA, TI>(v_s, c_s, rp_s, rows_lds, a, r0, e0, nr, xrc, j0, kk, alpha, beta, tid)
+    // Sixteen sums of long rows are staged in LDS, for as many rows as fit, and
+    // written column by column, consecutive rows from consecutive lanes: written
+    // from the lanes that hold them they went to 16 lines per row, a third of
+    // the kernel's L2 requests (the matrices above, k = 16: 5185 -> 4850 us;
+    // fewer sums or shorter rows lose by the barriers).
+    if constexpr (mrhs_staged<KP, TA>() > 0) {
+      if (avg > 6) {
+        constexpr int NB = mrhs_staged<KP, TA>() / (KP + 1);
+        TY *y = static_cast<TY *>(a.y);
+        for (int64_t i0 = 0; i0 < nr; i0 += NB) {
+          const int nb = static_cast<int>(nr - i0 < NB ? nr - i0 : NB);
+#define DRX_RS(G) reduce_rows_mrhs_split<WG, G, KP, true, TX, TY, TA, TI>(v_s, c_s, rp_s + i0, rows_lds, a, r0 + i0, e0, nb, xrc, j0, kk, alpha, beta, yb, tid)
+          if (avg <= 12)
+            DRX_RS(G4);
+          else if (avg <= 24)
+            DRX_RS(G8);
+          else
+            DRX_RS(G16);
+#undef DRX_RS
+          __syncthreads();
+          for (int j = tid >> 6; j < kk; j += WG / 64) {
+            TY *yp = y + (j0 + j) * a.ldy + r0 + i0;
+            for (int i = tid & 63; i < nb; i += 64) {
+              TA out = alpha * yb[i * (KP + 1) + j];
+              if (beta != TA(0)) out += beta * to_acc<TA>(yp[i]);
+              __builtin_nontemporal_store(from_acc<TY>(out), yp + i);
+            }
+          }
+          __syncthreads();
+        }
+        return;
+      }
+    }
+#define DRX_RS(G) reduce_rows_mrhs_split<WG, G, KP, false, TX, TY, TA, TI>(v_s, c_s, rp_s, rows_lds, a, r0, e0, nr, xrc, j0, kk, alpha, beta, yb, tid)
     if (avg <= 3)
       DRX_RS(1);
     else if (avg <= 6)
@@ -1180,7 +1238,7 @@ template <int WG, int CAP, int KP, int MODE, typename TV, typename TX,
           typename TY, typename TA, typename TI>
 __device__ __forceinline__ void process_block_mrhs(const FwdArgs &a,
                                                    int64_t blk,
-                                                   MrhsSmem<WG, CAP, TA> &sm) {
+                                                   MrhsSmem<WG, CAP, KP, TA> &sm) {
   constexpr int T = CAP / WG;
   constexpr int ROWCAP = CAP / 2;
   constexpr int NW = WG / 64;
@@ -1248,7 +1306,7 @@ __device__ __forceinline__ void process_block_mrhs(const FwdArgs &a,
     const int kk = static_cast<int>(a.k - jc * KP < KP ? a.k - jc * KP : KP);
     reduce_rows_mrhs_any<WG, KP, TX, TY, TA, TI>(
         n_s, sm.v, sm.c, sm.rp_s, rows_lds, a, b.r0, b.e0, nr,
-        xr + jc * a.ncols * KP, jc * KP, kk, alpha, beta, sm.red, tid);
+        xr + jc * a.ncols * KP, jc * KP, kk, alpha, beta, sm.red, sm.yb, tid);
   }
 
   if (b.es < e1) {
@@ -1278,7 +1336,7 @@ __device__ __forceinline__ void process_block_mrhs(const FwdArgs &a,
 // to 16 bytes per lane (73-78 VGPRs), 5 for wider ones taken in 16-byte
 // pieces (95), 4 for 16-bit x in wide chunks (whole chunks per lane).
 template <int WG, int CAP, int KP, typename TX, typename TA> constexpr int mrhs_waves() {
-  constexpr int lds = static_cast<int>(sizeof(MrhsSmem<WG, CAP, TA>));
+  constexpr int lds = static_cast<int>(sizeof(MrhsSmem<WG, CAP, KP, TA>));
   constexpr int w = (160 * 1024) / lds * (WG / 256);
   constexpr int most = KP * sizeof(TA) <= 16 ? 6 : (sizeof(TX) == 2 ? 4 : 5);
   return w > most ? most : (w < 1 ? 1 : w);
@@ -1289,7 +1347,7 @@ template <int WG, int CAP, int KP, int MODE, typename TV, typename TX,
 __global__ __launch_bounds__(WG)
 __attribute__((amdgpu_waves_per_eu(mrhs_waves<WG, CAP, KP, TX, TA>(), 8)))
 void k_spmv_mrhs(FwdArgs a) {
-  __shared__ MrhsSmem<WG, CAP, TA> sm;
+  __shared__ MrhsSmem<WG, CAP, KP, TA> sm;
   for (int64_t wi = blockIdx.x; wi < a.per_xcd * kXcds; wi += a.grid) {
     const int64_t blk = map_block(wi, a.per_xcd);
     if (blk >= a.nblocks) continue;

@@ -217,6 +217,35 @@ def test_low_precision_multi_rhs(orc, vdt, xdt_same):
         assert componentwise_err(y.cpu().numpy(), ystar, absy) < 1e-5
 
 
+@pytest.mark.parametrize("vdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [9, 16, 33])
+def test_multi_rhs_staged_sums(orc, vdt, k):
+    """Sixteen sums per row staged in LDS: blocks of fewer and more rows than
+    are staged at once (rows around 13..60 entries, then short and empty rows),
+    the last chunk of right-hand sides partly filled, beta, padded ldy."""
+    rng = np.random.default_rng(k)
+    lens = ([13] * 700 + list(rng.integers(14, 61, 400)) + [700, 0, 0, 1] +
+            list(rng.integers(0, 9, 3000)) + [30] * 150)
+    n = 6000
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    ci = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens if L])
+    v = rng.uniform(-1, 1, ci.size).astype(np.float32)
+    Ad = upload(rp, ci, v, (len(lens), n))
+    vq = Ad.vals.to(vdt)
+    x = torch.as_tensor(rng.uniform(-1, 1, (k, n)).astype(np.float32)).to(DEV).to(vdt)
+    y0 = torch.rand(k, len(lens) + 5, device=DEV)
+    y = y0.clone()
+    Ad.matvec(x, y=y, vals=vq, alpha=2.0, beta=-0.5)
+    torch.cuda.synchronize()
+    ys, absy = orc.spmv(rp, ci, vq.double().cpu().numpy(), x.double().cpu().numpy())
+    got, was = y.double().cpu().numpy(), y0.double().cpu().numpy()
+    m = len(lens)
+    want, den = 2.0 * ys - 0.5 * was[:, :m], 2.0 * absy + 0.5 * was[:, :m]
+    assert (np.abs(got[:, :m] - want) <= 1e-5 * den + 1e-300).all()
+    assert np.array_equal(got[:, m:], was[:, m:])
+    Ad.close()
+
+
 def test_multi_rhs_on_panel_plan(orc):
     """A plan with column panels serves k >= 2 from the share's own arrays
     (same operand contract: the pointers the layout was built from)."""
