@@ -44,7 +44,8 @@ struct Plan {
   PanelSet *panels = nullptr;  // column-panel layout (drx_plan_set_panels)
   // Cached column locality of the share for one colind pointer (k >= 2
   // path choice): -1 unknown, else bit 0 = tight (row blocks span about as
-  // many columns as entries), bit 1 = loose (within ncols / 16).
+  // many columns as entries), bit 1 = loose (within ncols / 16), bit 2 =
+  // shared (neighbouring rows hold the same columns).
   // Atomics: calls sharing the plan from several threads read and write the
   // cache without a lock. A torn read only picks the other, equally correct,
   // k >= 2 path once.
@@ -134,9 +135,10 @@ void owned_free(int dev, std::initializer_list<void *> ptrs);
 int mrhs_kp(int64_t k, int xtype, bool loose_local = false);
 // Column locality of the share: bit 0 when most row blocks' windows span few
 // more columns than entries (banded, 2-D stencils), bit 1 when they span at
-// most ncols / 16 (3-D stencils too). Measured once per colind pointer (one
-// small kernel and a wait), cached in the plan; 0 while the stream is being
-// captured.
+// most ncols / 16 (3-D stencils too), bit 2 when eight neighbouring rows hold
+// each column of their span twice or more (wide bands). Measured once per
+// colind pointer (one small kernel and a wait), cached in the plan; 0 while the
+// stream is being captured.
 int column_locality(const Plan &p, const void *colind, hipStream_t s);
 size_t mrhs_xr_bytes(int64_t ncols, int64_t k, int kp, int xtype);
 void launch_x_rowmajor(int xtype, const void *x, int64_t ldx, int64_t ncols,

@@ -174,15 +174,21 @@ void owned_free(int dev, std::initializer_list<void *> ptrs) {
 
 // Samples up to 4096 row blocks: the span between the first and the last
 // column index of each window, against its entry count (tight: at most
-// 4 n + 64) and against ncols / 16 (loose). out = {tight, loose, sampled}.
+// 4 n + 64) and against ncols / 16 (loose); and the columns that the eight rows
+// from the block's first on span together, against the entries they hold
+// (shared: at most half as many columns). out = {tight, loose, sampled,
+// shared}. One workgroup, bound by the chain record, row start, column: as many
+// lanes as it can have, a sample's loads all in flight.
 template <typename TI>
-__global__ void k_col_local(const BlockRec *rec, int64_t nblocks, int64_t ncols,
-                            const TI *colind, int *out) {
-  __shared__ int cnt[3];
-  if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
+__global__ __launch_bounds__(1024) void k_col_local(const BlockRec *rec, int64_t nblocks,
+                                                    int64_t ncols, const TI *colind,
+                                                    const TI *rowptr, int64_t base, int64_t nrows,
+                                                    int64_t nnz, int sent, int *out) {
+  __shared__ int cnt[4];
+  if (threadIdx.x < 4) cnt[threadIdx.x] = 0;
   __syncthreads();
   const int64_t S = nblocks < 4096 ? nblocks : 4096;
-  int tight = 0, loose = 0, seen = 0;
+  int tight = 0, loose = 0, seen = 0, shared = 0;
   for (int64_t i = threadIdx.x; i < S; i += blockDim.x) {
     const BlockRec b = rec[i * nblocks / S];
     const int64_t n = b.es - b.e0;
@@ -193,17 +199,34 @@ __global__ void k_col_local(const BlockRec *rec, int64_t nblocks, int64_t ncols,
       seen++;
       if (span <= 4 * n + 64) tight++;
       if (span <= 4 * n + 64 || span <= ncols / 16) loose++;
+      int64_t at[9], c0[8], c1[8];
+#pragma unroll
+      for (int q = 0; q < 9; q++) {
+        const int64_t r = b.r0 + q < nrows ? b.r0 + q : nrows;
+        at[q] = row_begin(rowptr, base, nrows, nnz, sent, r);
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++) {  // (n >= 2, so nnz is no smaller)
+        c0[q] = static_cast<int64_t>(colind[at[q] < nnz ? at[q] : nnz - 1]);
+        c1[q] = static_cast<int64_t>(colind[at[q + 1] > 0 ? at[q + 1] - 1 : 0]);
+      }
+      const int64_t held = at[8] - at[0];
+      int64_t first = ncols, last = 0;
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        if (at[q] >= at[q + 1]) continue;
+        first = c0[q] < first ? c0[q] : first;
+        last = c1[q] > last ? c1[q] : last;
+      }
+      if (2 * (last - first) <= held) shared++;
     }
   }
   atomicAdd(&cnt[0], tight);
   atomicAdd(&cnt[1], loose);
   atomicAdd(&cnt[2], seen);
+  atomicAdd(&cnt[3], shared);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    out[0] = cnt[0];
-    out[1] = cnt[1];
-    out[2] = cnt[2];
-  }
+  if (threadIdx.x < 4) out[threadIdx.x] = cnt[threadIdx.x];
 }
 
 int column_locality(const Plan &p, const void *colind, hipStream_t s) {
@@ -215,15 +238,19 @@ int column_locality(const Plan &p, const void *colind, hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   DRX_HIP(hipStreamIsCapturing(s, &st));
   if (st != hipStreamCaptureStatusNone) return 0;
-  int *d = static_cast<int *>(scratch_alloc(3 * sizeof(int), s));
-  int h[3] = {0, 0, 0};
+  int *d = static_cast<int *>(scratch_alloc(4 * sizeof(int), s));
+  int h[4] = {0, 0, 0, 0};
   try {
     if (p.itype == DRX_I32)
-      hipLaunchKernelGGL(k_col_local<int32_t>, dim3(1), dim3(256), 0, s, p.rec, p.nblocks,
-                         p.ncols, static_cast<const int32_t *>(colind), d);
+      hipLaunchKernelGGL(k_col_local<int32_t>, dim3(1), dim3(1024), 0, s, p.rec, p.nblocks,
+                         p.ncols, static_cast<const int32_t *>(colind),
+                         static_cast<const int32_t *>(p.rowptr), p.base, p.nrows, p.nnz,
+                         p.has_sentinel, d);
     else
-      hipLaunchKernelGGL(k_col_local<int64_t>, dim3(1), dim3(256), 0, s, p.rec, p.nblocks,
-                         p.ncols, static_cast<const int64_t *>(colind), d);
+      hipLaunchKernelGGL(k_col_local<int64_t>, dim3(1), dim3(1024), 0, s, p.rec, p.nblocks,
+                         p.ncols, static_cast<const int64_t *>(colind),
+                         static_cast<const int64_t *>(p.rowptr), p.base, p.nrows, p.nnz,
+                         p.has_sentinel, d);
     DRX_HIP(hipGetLastError());
     DRX_HIP(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
     DRX_HIP(hipStreamSynchronize(s));
@@ -235,11 +262,248 @@ int column_locality(const Plan &p, const void *colind, hipStream_t s) {
   int loc = 0;
   if (h[2] > 0 && 10 * h[0] >= 9 * h[2]) loc |= 1;
   if (h[2] > 0 && 10 * h[1] >= 9 * h[2]) loc |= 2;
+  if (h[2] > 0 && 10 * h[3] >= 9 * h[2]) loc |= 4;
   // Invalidate, then publish pointer and value.
   p.loc_local.store(-1, std::memory_order_release);
   p.loc_colind.store(colind, std::memory_order_release);
   p.loc_local.store(loc, std::memory_order_release);
   return loc;
+}
+
+// ---------------------------------------------------------------------------
+// k >= 2 over long rows whose neighbours hold neighbouring columns (wide
+// bands). Gathered one row at a time, each entry reads its x row (KP values)
+// from L2, 64 bytes per 16 of the matrix in FP64 and k = 8: that bounds the
+// row-block kernel, though eight neighbouring rows read almost the same x.
+// Here a workgroup takes eight rows and copies the columns that they span into
+// LDS piece by piece, straight from x as the caller holds it (no row-major copy,
+// no scratch, one launch). A wave sums two rows, a lane every 64th entry; a row's
+// next U * 64 entries wait in registers until the piece with their columns is
+// there (so their loads are in flight while x is copied, and no entry is read
+// twice), and are summed from memory where columns are out of order.
+// Bound by the matrix stream: 50000 rows of 2001 entries, k = 8, FP64 values and
+// 64-bit columns 315 us (5.1 TB/s; with its launch in a loop 345, the row-block
+// kernel 518; entries read again
+// in the next piece instead of kept: 390), FP32 and 32-bit columns 201 (325).
+// U: FP64 2 / 4 / 8 batches 362 / 345 / 457 us, FP32 260 / 223 / 201.
+// ---------------------------------------------------------------------------
+constexpr int kBandRows = 8;                 // rows of a workgroup, two per wave
+constexpr int kBandLds = 38 * 1024;          // x of one piece (four workgroups per CU)
+
+// Bytes between the x rows of neighbouring columns in LDS: rows of more than 16
+// bytes are padded by 16, so that 16 lanes' 16-byte reads of neighbouring
+// columns fall into different banks.
+template <int KP, typename TX> constexpr int band_stride() {
+  constexpr int b = KP * static_cast<int>(sizeof(TX));
+  return b <= 16 ? b : b + 16;
+}
+
+// x of column c (KP columns from j0 on, kk of them there) in storage type;
+// zeros past the last column.
+template <int KP, typename TX>
+__device__ __forceinline__ void band_xcol(const TX *x, int64_t ldx, int64_t ncols, int64_t j0,
+                                          int kk, int64_t c, TX (&t)[KP]) {
+  if (static_cast<uint64_t>(c) >= static_cast<uint64_t>(ncols)) kk = 0;
+#pragma unroll
+  for (int j = 0; j < KP; j++) t[j] = j < kk ? x[(j0 + j) * ldx + c] : TX{};
+}
+
+template <int KP, typename TV, typename TX, typename TY, typename TA, typename TI>
+__global__ __launch_bounds__(256) void k_spmv_band(FwdArgs a, int64_t j0) {
+  constexpr int STRIDE = band_stride<KP, TX>(), PC = kBandLds / STRIDE / 64 * 64;
+  constexpr int ALIGN = STRIDE < 16 ? STRIDE : 16;
+  constexpr int RW = kBandRows / 4, U = sizeof(TA) == 4 ? 8 : 4;
+  constexpr uint32_t kDone = 0xffffffffu;
+  __shared__ __attribute__((aligned(16))) char xs[PC * STRIDE];
+  __shared__ int64_t row_at[kBandRows + 1];
+  __shared__ uint32_t range[2];
+  __shared__ TA ys[kBandRows * (KP + 1)];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t blk = map_block(blockIdx.x, a.per_xcd);
+  if (blk >= a.nblocks) return;  // the whole workgroup
+  const int64_t r0 = blk * kBandRows;
+  const TI *rowptr = static_cast<const TI *>(a.rowptr);
+  const TI *colind = static_cast<const TI *>(a.colind);
+  const TV *vals = static_cast<const TV *>(a.vals);
+  const TX *x = static_cast<const TX *>(a.x);
+  const int kk = a.k - j0 < KP ? static_cast<int>(a.k - j0) : KP;
+  if (tid <= kBandRows) {
+    const int64_t r = r0 + tid < a.nrows ? r0 + tid : a.nrows;
+    row_at[tid] = row_begin(rowptr, a.base, a.nrows, a.nnz, a.sent, r);
+  }
+  if (tid == 0) {
+    range[0] = kDone;
+    range[1] = 0;
+  }
+  __syncthreads();
+  int64_t at[RW], end[RW];
+  uint32_t c[RW][U];
+  TV w[RW][U];
+  TA acc[RW][KP];
+  // The next U * 64 entries of a row of the wave; lanes past its end are done.
+  auto load = [&](int r) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int64_t e = at[r] + u * 64 + lane;
+      const int64_t ee = e < end[r] ? e : end[r] - 1;
+      c[r][u] = col32(ld_stream(colind + ee));
+      w[r][u] = ld_stream(vals + ee);
+      if (e >= end[r]) c[r][u] = kDone;
+    }
+    at[r] += U * 64;
+  };
+#pragma unroll
+  for (int r = 0; r < RW; r++) {
+    at[r] = row_at[wave * RW + r];
+    end[r] = row_at[wave * RW + r + 1];
+#pragma unroll
+    for (int j = 0; j < KP; j++) acc[r][j] = 0;
+    if (at[r] < end[r]) {
+      load(r);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        c[r][u] = kDone;
+        w[r][u] = TV{};
+      }
+    }
+  }
+  if (tid < kBandRows && row_at[tid] < row_at[tid + 1]) {
+    atomicMin(&range[0], col32(colind[row_at[tid]]));
+    atomicMax(&range[1], col32(colind[row_at[tid + 1] - 1]));
+  }
+  __syncthreads();
+  const uint32_t lo = range[0], ncols = static_cast<uint32_t>(a.ncols);
+  const uint32_t past = range[1] < ncols ? range[1] + 1 : ncols;
+  const int64_t held = row_at[kBandRows] - row_at[0];
+  // The entries held of the wave's rows with columns below p1: x from LDS from
+  // column p0 on, from memory below.
+  auto sum_below = [&](uint32_t p0, uint32_t p1) {
+#pragma unroll
+    for (int r = 0; r < RW; r++) {
+      for (;;) {
+        bool rest = false;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          if (c[r][u] < p1) {
+            TX t[KP];
+            if (c[r][u] >= p0)
+              __builtin_memcpy(t, __builtin_assume_aligned(xs + (c[r][u] - p0) * STRIDE, ALIGN),
+                               sizeof(t));
+            else
+              band_xcol<KP>(x, a.ldx, a.ncols, j0, kk, c[r][u], t);
+            const TA v = to_acc<TA>(w[r][u]);
+#pragma unroll
+            for (int j = 0; j < KP; j++) acc[r][j] += v * to_acc<TA>(t[j]);
+            c[r][u] = kDone;
+          }
+          rest |= c[r][u] != kDone;
+        }
+        if (__ballot(rest) != 0 || at[r] >= end[r]) break;
+        load(r);
+      }
+    }
+  };
+  // Pieces of the columns that the rows span, unless they span far more than
+  // the rows hold.
+  if (lo < past && past - lo < 2 * held + PC) {
+    for (uint32_t p0 = lo; p0 < past; p0 += PC) {
+      const uint32_t p1 = past - p0 > PC ? p0 + PC : past;
+      __syncthreads();
+      for (uint32_t i = tid; i < p1 - p0; i += 256) {
+        TX t[KP];
+        band_xcol<KP>(x, a.ldx, a.ncols, j0, kk, p0 + i, t);
+        __builtin_memcpy(__builtin_assume_aligned(xs + i * STRIDE, ALIGN), t, sizeof(t));
+      }
+      __syncthreads();
+      sum_below(p0, p1);
+    }
+  }
+  // What is left (columns out of order, or no pieces).
+  sum_below(kDone, kDone);
+#pragma unroll
+  for (int r = 0; r < RW; r++) {
+#pragma unroll
+    for (int j = 0; j < KP; j++) {
+      const TA sum = group_sum<64>(acc[r][j]);
+      if (lane == 0) ys[(wave * RW + r) * (KP + 1) + j] = sum;
+    }
+  }
+  __syncthreads();
+  TY *y = static_cast<TY *>(a.y);
+  const TA alpha = static_cast<TA>(a.alpha), beta = static_cast<TA>(a.beta);
+  for (int t = tid; t < kBandRows * kk; t += 256) {
+    const int j = t / kBandRows, i = t % kBandRows;
+    if (r0 + i >= a.nrows) continue;
+    TY *yp = y + (j0 + j) * a.ldy + r0 + i;
+    TA out = alpha * ys[i * (KP + 1) + j];
+    if (beta != TA(0)) out += beta * to_acc<TA>(*yp);
+    *yp = from_acc<TY>(out);
+  }
+}
+
+template <int KP, typename TV, typename TX, typename TY, typename TA>
+static void launch_band(const Plan &p, const FwdArgs &a, int64_t j0, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(a.grid));
+  if (p.itype == DRX_I32)
+    hipLaunchKernelGGL((k_spmv_band<KP, TV, TX, TY, TA, int32_t>), grid, dim3(256), 0, s, a, j0);
+  else
+    hipLaunchKernelGGL((k_spmv_band<KP, TV, TX, TY, TA, int64_t>), grid, dim3(256), 0, s, a, j0);
+}
+
+template <typename TV, typename TX, typename TY, typename TA>
+static void launch_band_t(const Plan &p, const FwdArgs &a, hipStream_t s) {
+  // Up to 16 right-hand sides per pass over the matrix (FP64, rows of 600, 16
+  // of them: 183 us, in two passes of 8 228).
+  for (int64_t j0 = 0; j0 < a.k; j0 += 16) {
+    const int64_t left = a.k - j0;
+    if (left <= 2)
+      launch_band<2, TV, TX, TY, TA>(p, a, j0, s);
+    else if (left <= 4)
+      launch_band<4, TV, TX, TY, TA>(p, a, j0, s);
+    else if (left <= 8)
+      launch_band<8, TV, TX, TY, TA>(p, a, j0, s);
+    else
+      launch_band<16, TV, TX, TY, TA>(p, a, j0, s);
+  }
+}
+
+// Plain shares of rows of much the same length whose neighbours hold
+// neighbouring columns (bit 2 of column_locality): long rows, where the matrix
+// stream covers the steps a workgroup takes one after the other (50000 rows, row
+// blocks / here: 401 entries FP32 k = 2 / 8 / 16 57 / 53, 73 / 69, 101 / 88 us,
+// FP64 74 / 68, 100 / 91, 147 / 147; 301 entries 47 / 48, 55 / 63, 76 / 82 and
+// 60 / 63, 83 / 84, 122 / 168; 601 entries 95 / 75, 124 / 91, 187 / 117), and
+// shorter ones where all workgroups are resident at once (8192 rows) and one
+// launch without scratch counts for more (8000 rows of 97 entries FP64 k = 2 / 8 /
+// 16: 36 / 14, 34 / 15, 31 / 24 us).
+bool band_mrhs(const Plan &p, const FwdArgs &a, hipStream_t s) {
+  const int64_t least = p.nrows <= 8192 ? 96 : 384;
+  return p.lmax > 0 && p.nnz >= least * p.nrows && p.lmax * p.nrows <= 4 * p.nnz &&
+         a.xbytes > 0 && (column_locality(p, a.colind, s) & 4) != 0;
+}
+
+void run_band(const Plan &p, FwdArgs a, int vtype, int xtype, int ytype, hipStream_t s) {
+  a.nblocks = (p.nrows + kBandRows - 1) / kBandRows;
+  a.per_xcd = (a.nblocks + kXcds - 1) / kXcds;
+  a.grid = a.per_xcd * kXcds;
+  DRX_REQUIRE(a.grid <= int64_t(0xffffffff), "too many rows for one launch");
+  if (vtype == DRX_F64 && xtype == DRX_F64 && ytype == DRX_F64)
+    launch_band_t<double, double, double, double>(p, a, s);
+  else if (vtype == DRX_F32 && xtype == DRX_F32 && ytype == DRX_F32)
+    launch_band_t<float, float, float, float>(p, a, s);
+  else if (vtype == DRX_BF16 && xtype == DRX_BF16 && ytype == DRX_F32)
+    launch_band_t<bf16, bf16, float, float>(p, a, s);
+  else if (vtype == DRX_F16 && xtype == DRX_F16 && ytype == DRX_F32)
+    launch_band_t<f16, f16, float, float>(p, a, s);
+  else if (vtype == DRX_BF16 && xtype == DRX_F32 && ytype == DRX_F32)
+    launch_band_t<bf16, float, float, float>(p, a, s);
+  else if (vtype == DRX_F16 && xtype == DRX_F32 && ytype == DRX_F32)
+    launch_band_t<f16, float, float, float>(p, a, s);
+  else
+    throw Error(DRX_ERR_UNSUPPORTED, "unsupported (vtype, xtype, ytype)");
+  DRX_HIP(hipGetLastError());
 }
 
 int mrhs_kp(int64_t k, int xtype, bool loose_local) {

@@ -246,6 +246,48 @@ def test_multi_rhs_staged_sums(orc, vdt, k):
     Ad.close()
 
 
+@pytest.mark.parametrize("vdt,xdt", [(torch.float64, torch.float64), (torch.float32, torch.float32),
+                                     (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("m,k,order", [(1, 2, "sorted"), (9, 3, "sorted"), (203, 8, "sorted"),
+                                       (203, 13, "shuffled"), (640, 5, "spread")])
+def test_multi_rhs_wide_band(orc, vdt, xdt, m, k, order):
+    """Rows of a hundred and more columns around their own: pieces of x in LDS,
+    a last group of fewer than eight rows, empty rows, columns out of order
+    within a row (read from memory) and a row that spans the whole matrix, the
+    right-hand sides in chunks with a remainder, beta, padded ldy."""
+    rng = np.random.default_rng(m + k)
+    n, hw = 5000, 700
+    rows = []
+    for i in range(m):
+        c0 = i * (n - 2 * hw) // m
+        L = 0 if i in (4, 5) else int(rng.integers(900, 1200))
+        c = np.sort(rng.choice(np.arange(c0, c0 + 2 * hw), L, replace=False))
+        if order == "shuffled" and i % 3 == 0:
+            c[1:-1] = rng.permutation(c[1:-1])
+        if order == "spread" and i % 64 == 7:
+            c[0], c[-1] = 0, n - 1
+        rows.append(c)
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in rows])]).astype(np.int64)
+    ci = np.concatenate(rows)
+    Ad = upload(rp, ci, rng.uniform(-1, 1, ci.size), (m, n))
+    vq = Ad.vals.to(vdt)
+    x = torch.as_tensor(rng.uniform(-1, 1, (k, n))).to(DEV).to(xdt)
+    ydt = torch.float64 if vdt == torch.float64 else torch.float32
+    y0 = torch.rand(k, m + 5, device=DEV, dtype=ydt)
+    y = y0.clone()
+    Ad.matvec(x, y=y, vals=vq, alpha=2.0, beta=-0.5)
+    torch.cuda.synchronize()
+    ys, absy = orc.spmv(rp, ci, vq.double().cpu().numpy(), x.double().cpu().numpy())
+    got, was = y.double().cpu().numpy(), y0.double().cpu().numpy()
+    want, den = 2.0 * ys - 0.5 * was[:, :m], 2.0 * absy + 0.5 * was[:, :m]
+    # 1200 products summed by 64 lanes and a tree, alpha and beta: at most 32
+    # roundings on the way of any product
+    u = 2.0 ** (-53 if ydt == torch.float64 else -24)
+    assert (np.abs(got[:, :m] - want) <= 40 * u * den + 1e-300).all()
+    assert np.array_equal(got[:, m:], was[:, m:])
+    Ad.close()
+
+
 def test_multi_rhs_on_panel_plan(orc):
     """A plan with column panels serves k >= 2 from the share's own arrays
     (same operand contract: the pointers the layout was built from)."""
