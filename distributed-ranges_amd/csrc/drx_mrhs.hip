@@ -172,11 +172,14 @@ void owned_free(int dev, std::initializer_list<void *> ptrs) {
   if (cur != dev) (void)hipSetDevice(cur);
 }
 
+// Fewest entries per row for which the wide-band kernel may run (band_mrhs).
+constexpr int64_t kBandLeast = 96;
+
 // Samples up to 4096 row blocks: the span between the first and the last
 // column index of each window, against its entry count (tight: at most
 // 4 n + 64) and against ncols / 16 (loose); and the columns that the eight rows
 // from the block's first on span together, against the entries they hold
-// (shared: at most half as many columns). out = {tight, loose, sampled,
+// (long rows only; shared: at most half as many columns). out = {tight, loose, sampled,
 // shared}. One workgroup, bound by the chain record, row start, column: as many
 // lanes as it can have, a sample's loads all in flight.
 template <typename TI>
@@ -199,6 +202,7 @@ __global__ __launch_bounds__(1024) void k_col_local(const BlockRec *rec, int64_t
       seen++;
       if (span <= 4 * n + 64) tight++;
       if (span <= 4 * n + 64 || span <= ncols / 16) loose++;
+      if (nnz < kBandLeast * nrows) continue;  // (no band, whatever the columns)
       int64_t at[9], c0[8], c1[8];
 #pragma unroll
       for (int q = 0; q < 9; q++) {
@@ -206,7 +210,7 @@ __global__ __launch_bounds__(1024) void k_col_local(const BlockRec *rec, int64_t
         at[q] = row_begin(rowptr, base, nrows, nnz, sent, r);
       }
 #pragma unroll
-      for (int q = 0; q < 8; q++) {  // (n >= 2, so nnz is no smaller)
+      for (int q = 0; q < 8; q++) {
         c0[q] = static_cast<int64_t>(colind[at[q] < nnz ? at[q] : nnz - 1]);
         c1[q] = static_cast<int64_t>(colind[at[q + 1] > 0 ? at[q + 1] - 1 : 0]);
       }
@@ -479,7 +483,7 @@ static void launch_band_t(const Plan &p, const FwdArgs &a, hipStream_t s) {
 // launch without scratch counts for more (8000 rows of 97 entries FP64 k = 2 / 8 /
 // 16: 36 / 14, 34 / 15, 31 / 24 us).
 bool band_mrhs(const Plan &p, const FwdArgs &a, hipStream_t s) {
-  const int64_t least = p.nrows <= 8192 ? 96 : 384;
+  const int64_t least = p.nrows <= 8192 ? kBandLeast : 4 * kBandLeast;
   return p.lmax > 0 && p.nnz >= least * p.nrows && p.lmax * p.nrows <= 4 * p.nnz &&
          a.xbytes > 0 && (column_locality(p, a.colind, s) & 4) != 0;
 }
