@@ -101,9 +101,10 @@ def headline(steps, warmup):
     layout = {"panels": npan, "panel_cols": width, "row_segments": nseg,
               "plain_csr_ms_per_step": round(plain_ms, 4),
               "plain_csr_GBps": round(B / plain_ms / 1e6, 2)}
-    # The bound that matters here: random 4-byte gathers inside one panel's x
-    # slice. drx_gather does only that (streamed indices, gathered values
-    # written out) for one panel's share of the entries.
+    # For scale: random 4-byte gathers of x from L2. drx_gather does only that
+    # (streamed indices, gathered values written out) for one panel's share of
+    # the entries. The panel layout gathers from x slices in LDS instead, which
+    # is why a step takes a fraction of the probe's time.
     per = A.nnz // npan
     g = torch.Generator(device="cuda").manual_seed(3)
     idx = torch.randint(0, width, (per,), dtype=torch.int32, device="cuda", generator=g)
@@ -121,10 +122,10 @@ def headline(steps, warmup):
 
 
 def form_panel_sweep(A, x, steps, widths=(262144, 393216, 524288, 786432, 1048576)):
-    """The headline product through column panels of each width (columns of x
-    per panel): time per step and the row segments the layout makes. Narrow
-    panels cost row-segment work; a panel whose x slice and streamed entries
-    outgrow an XCD's 4 MB L2 misses on its gathers."""
+    """The headline product through column panels of each requested width
+    (columns of x per panel): time per step and the row segments the layout
+    makes. The kernels cut x into slices that fit into LDS whatever the width
+    asked for, so the times should not differ."""
     n = A.shape[0]
     y = torch.empty(n, dtype=torch.float32, device="cuda")
     B = spmv_bytes(n, A.shape[1], A.nnz, 4, 4, 4, 4)
@@ -585,14 +586,14 @@ def main():
                    "rows": A.shape[0], "cols": A.shape[1], "nnz": A.nnz,
                    "mean_nnz_per_row": round(A.nnz / A.shape[0], 3),
                    "algorithmic_bytes_per_step": B, "parallelism": "single GPU",
-                   "layout": "CSR + column-panel plan (2 MB x slices, L2-resident gathers)",
+                   "layout": "CSR + column-panel plan (entries by x slice, slices of x staged in LDS)",
                    **layout},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": read_traffic(),
-                     "kernel": "drx::k_spmv_fwd<256,2048,kRowMap,f32,i32> (one launch per "
-                               "column panel); achieved = bytes / summed time of one step's "
-                               "launches",
+                     "kernel": "drx::k_slice_sums (segment sums from x slices in LDS) and "
+                               "drx::k_slice_rows (segments to rows); achieved = bytes / "
+                               "summed time of one step's launches",
                      "ms_per_step_kernels": round(ev_ms, 4),
                      "gather_ceiling": gather},
     }
