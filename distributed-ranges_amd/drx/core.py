@@ -164,7 +164,7 @@ class CsrMatrix:
 
     def set_panels(self, panel_cols=0, stream=None):
         """Keep a column-panel copy of the entries in the plan (see
-        drx_plan_set_panels); later matvecs run one L2-sized panel at a time."""
+        drx_plan_set_panels); later matvecs read x from slices in LDS."""
         check(lib().drx_plan_set_panels(self.plan.handle, self.vcode, _p(self.colind),
                                         _p(self.vals), int(panel_cols), _s(stream)))
         return self.panels()

@@ -288,6 +288,42 @@ def test_multi_rhs_wide_band(orc, vdt, xdt, m, k, order):
     Ad.close()
 
 
+@pytest.mark.parametrize("itype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("cut", [0, 37])
+@pytest.mark.parametrize("k", [2, 7, 16, 19])
+def test_multi_rhs_wide_band_shares(orc, itype, cut, k):
+    """The same kernel on a share cut inside a row at both ends (absolute
+    offsets, no sentinel), both index types, padded x, values that start
+    anywhere, k in one and two chunks: against the oracle, and against the
+    row-major chunks (knob mrhs 2) over the same operands."""
+    rng = np.random.default_rng(k)
+    n, L, m = 3000, 500, 150
+    cols = [np.sort(rng.choice(np.arange(i * 15, i * 15 + 700), L, replace=False))
+            for i in range(m)]
+    rp = np.arange(m + 1, dtype=np.int64) * L
+    ci, v = np.concatenate(cols), rng.uniform(-1, 1, m * L)
+    r0, r1 = (3, m - 2) if cut else (0, m)  # rows; entries [lo, hi)
+    lo, hi = int(rp[r0]) + cut, int(rp[r1]) - cut
+    rp_d = torch.as_tensor(rp[r0:r1]).to(itype).to(DEV)
+    sh = drx.CsrMatrix(rp_d, torch.as_tensor(ci).to(itype).to(DEV)[lo:hi],
+                       torch.as_tensor(v).to(DEV)[lo:hi], (r1 - r0, n), base=lo,
+                       has_sentinel=False)
+    xw = torch.as_tensor(rng.uniform(-1, 1, (k, n + 3))).to(DEV)
+    x = xw[:, :n]
+    y = sh.matvec(x)
+    with drx.tuned(mrhs=2):
+        z = sh.matvec(x)
+    torch.cuda.synchronize()
+    rps = np.clip(np.append(rp[r0:r1], hi) - lo, 0, hi - lo)
+    ys, absy = orc.spmv(rps, ci[lo:hi], v[lo:hi], x.cpu().numpy())
+    # at most 20 roundings on the way of a product in either path's trees;
+    # rows in order in the chunks' groups: at most 500 / 8 + 8
+    u = 2.0 ** -53
+    assert componentwise_err(y.cpu().numpy(), ys, absy) <= 40 * u
+    assert componentwise_err(y.cpu().numpy(), z.cpu().numpy(), absy) <= 120 * u
+    sh.close()
+
+
 def test_multi_rhs_on_panel_plan(orc):
     """A plan with column panels serves k >= 2 from the share's own arrays
     (same operand contract: the pointers the layout was built from)."""
