@@ -168,8 +168,7 @@ static void build_transpose(Transpose &t, const Plan &p, const TI *colind,
                          static_cast<const TI *>(t.perm), nnz, static_cast<TI *>(t.rowind));
       DRX_HIP(hipGetLastError());
     } catch (...) {
-      (void)hipStreamSynchronize(s);
-      for (void *q : tmp) block_free(t.device, q);
+      owned_free(t.device, tmp);
       throw;
     }
   } else {
@@ -180,8 +179,7 @@ static void build_transpose(Transpose &t, const Plan &p, const TI *colind,
                        false, false, true);
     DRX_HIP(hipStreamSynchronize(s));
   } catch (...) {
-    (void)hipStreamSynchronize(s);
-    for (void *q : tmp) block_free(t.device, q);
+    owned_free(t.device, tmp);
     throw;
   }
   for (void *q : tmp) block_free(t.device, q);

@@ -5,7 +5,7 @@
 
 #include <atomic>
 #include <cstdint>
-#include <initializer_list>
+#include <vector>
 
 namespace drx {
 
@@ -125,7 +125,9 @@ void scratch_unreserve(int dev, size_t bytes);
 void *block_alloc(size_t bytes);
 void block_free(int dev, void *p);
 // Blocks that any stream may have used: waits for the device, as hipFree does.
-void owned_free(int dev, std::initializer_list<void *> ptrs);
+// Where the runtime refuses the wait (a stream is being captured) they stay
+// aside until a later one succeeds.
+void owned_free(int dev, const std::vector<void *> &ptrs);
 
 // Row-major chunks of x for k >= 2 right-hand sides: chunk width KP and the
 // bytes of all chunks; the copy kernel.

@@ -14,12 +14,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <list>
-#include <map>
 #include <mutex>
 #include <set>
-#include <unordered_map>
+#include <vector>
 
+#include "drx_blocks.hpp"
 #include "drx_common.hpp"
 #include "drx_fwd.hpp"
 #include "drx_internal.hpp"
@@ -95,81 +94,51 @@ void scratch_unreserve(int dev, size_t bytes) {
 
 // ---------------------------------------------------------------------------
 // Blocks (block_alloc): mapping and unmapping the 0.5 GB that the plan and the
-// transpose of 20M entries take cost 14 ms beside 1.2 ms of kernels, and the
-// pool above unmaps freed memory whenever it holds more of it than is in use.
+// transpose of 20M entries take cost 9 to 14 ms (two boxes) beside 1.2 ms of
+// kernels, and the pool above unmaps freed memory whenever it holds more of it
+// than is in use.
 // ---------------------------------------------------------------------------
-struct Blocks {
-  std::mutex mu;
-  std::unordered_map<void *, size_t> size;      // every block handed out or kept
-  std::multimap<size_t, void *> kept;           // by size
-  std::list<void *> order;                      // kept ones, oldest first
-  size_t total = 0;                             // bytes kept
-  void drop(void *p) {  // a kept block goes back to the driver
-    const size_t n = size[p];
-    for (auto it = kept.lower_bound(n); it != kept.end() && it->first == n; ++it)
-      if (it->second == p) {
-        kept.erase(it);
-        break;
-      }
-    order.remove(p);
-    total -= n;
-    size.erase(p);
-    (void)hipFree(p);
+struct HipMemory {
+  static constexpr int kOutOfMemory = hipErrorOutOfMemory;
+  // (a refused call leaves no error behind for the next launch check)
+  static hipError_t cleared(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
   }
+  static int alloc(void **p, size_t bytes) { return cleared(hipMalloc(p, bytes)); }
+  static bool free(void *p) { return cleared(hipFree(p)) == hipSuccess; }
+  static bool wait() { return cleared(hipDeviceSynchronize()) == hipSuccess; }
 };
-static Blocks g_blocks[kMaxDevices];
+static BlockCache<HipMemory, kBlocksKeep> g_blocks[kMaxDevices];
+
+// Runs f with dev as the current device.
+template <typename F> static void on_device(int dev, F &&f) {
+  int cur = dev;
+  (void)hipGetDevice(&cur);
+  if (cur != dev) (void)hipSetDevice(dev);
+  f();
+  if (cur != dev) (void)hipSetDevice(cur);
+}
 
 void *block_alloc(size_t bytes) {
   int dev = 0;
   DRX_HIP(hipGetDevice(&dev));
   DRX_REQUIRE(dev >= 0 && dev < kMaxDevices, "device ordinal out of range");
-  bytes = (std::max<size_t>(bytes, 1) + 4095) & ~size_t(4095);
-  Blocks &b = g_blocks[dev];
-  std::lock_guard<std::mutex> lk(b.mu);
-  // a kept block of at most a quarter (small ones: 64 KB) more
-  const auto it = b.kept.lower_bound(bytes);
-  if (it != b.kept.end() && it->first <= bytes + std::max<size_t>(bytes / 4, 65536)) {
-    void *p = it->second;
-    b.total -= it->first;
-    b.kept.erase(it);
-    b.order.remove(p);
-    return p;
-  }
   void *p = nullptr;
-  hipError_t e = hipMalloc(&p, bytes);
-  if (e == hipErrorOutOfMemory && b.total > 0) {
-    (void)hipGetLastError();
-    while (!b.order.empty()) b.drop(b.order.front());
-    e = hipMalloc(&p, bytes);
-  }
-  DRX_HIP(e);
-  b.size[p] = bytes;
+  DRX_HIP(static_cast<hipError_t>(g_blocks[dev].take(bytes, &p)));
   return p;
 }
 
 void block_free(int dev, void *p) {
   if (p == nullptr || dev < 0 || dev >= kMaxDevices) return;
-  Blocks &b = g_blocks[dev];
-  std::lock_guard<std::mutex> lk(b.mu);
-  const auto at = b.size.find(p);
-  if (at == b.size.end()) return;
-  const size_t n = at->second;
-  b.kept.emplace(n, p);
-  b.order.push_back(p);
-  b.total += n;
-  while (b.total > kBlocksKeep) b.drop(b.order.front());
+  g_blocks[dev].give(p);
 }
 
-void owned_free(int dev, std::initializer_list<void *> ptrs) {
+void owned_free(int dev, const std::vector<void *> &ptrs) {
+  if (dev < 0 || dev >= kMaxDevices) return;
   bool any = false;
   for (void *p : ptrs) any = any || p != nullptr;
-  if (!any) return;
-  int cur = dev;
-  (void)hipGetDevice(&cur);
-  if (cur != dev) (void)hipSetDevice(dev);
-  (void)hipDeviceSynchronize();
-  for (void *p : ptrs) block_free(dev, p);
-  if (cur != dev) (void)hipSetDevice(cur);
+  if (any) on_device(dev, [&] { g_blocks[dev].retire(ptrs); });
 }
 
 // Fewest entries per row for which the wide-band kernel may run (band_mrhs).

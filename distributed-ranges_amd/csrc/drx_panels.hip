@@ -872,8 +872,7 @@ static void build_panels(Plan &p, PanelSet &ps, const TI *colind, const TV *vals
     DRX_HIP(hipGetLastError());
     DRX_HIP(hipStreamSynchronize(s));
   } catch (...) {
-    (void)hipStreamSynchronize(s);
-    for (void *q : tmp) block_free(ps.device, q);
+    owned_free(ps.device, tmp);
     throw;
   }
   for (void *q : tmp) block_free(ps.device, q);

@@ -161,6 +161,10 @@ int drx_plan_create(drx_plan *plan, int itype, const void *rowptr,
                     int64_t rowptr_base, int64_t nrows, int64_t ncols,
                     int64_t nnz, int has_sentinel, int64_t block_nnz,
                     drx_stream_t stream);
+/* Waits for the device (destroying an object while a stream is being captured
+ * invalidates that capture, as hipFree does). The memory of plans, transposes
+ * and panel layouts is kept for later ones, up to 4 GiB per device; where the
+ * wait is refused, it is not used again before a later one has succeeded. */
 int drx_plan_destroy(drx_plan plan);
 /* Number of row blocks and the block size the plan uses. */
 int drx_plan_info(drx_plan plan, int64_t *nblocks, int64_t *block_nnz);

@@ -65,6 +65,14 @@ def test_read_csr_matches_restated_reader(tmp_path):
     assert p.returncode == 1 and "out of bounds" in p.stdout
 
 
+def test_block_cache():
+    """Device memory of plans and transposes: not handed out again before a
+    wait for the device has succeeded (drx_blocks.hpp over a driver that can
+    refuse waits, frees and allocations)."""
+    p = _run("test_blocks", timeout=60)
+    assert p.returncode == 0 and "0 failures" in p.stdout
+
+
 @pytest.mark.gpu
 def test_mp_gemv_reference_tests():
     p = _run("test_mp_gemv")
