@@ -249,7 +249,7 @@ int drx_transpose_set_values(drx_transpose t, int vtype, const void *vals,
     if (tt->tvals == nullptr || tt->tvtype != vtype) {
       owned_free(tt->device, {tt->tvals});
       tt->tvals = nullptr;
-      tt->tvals = block_alloc(nnz * dtype_size(vtype));
+      tt->tvals = block_alloc(nnz * dtype_size(vtype), tt->device);
       tt->tvtype = vtype;
     }
     if (nnz == 0) return;

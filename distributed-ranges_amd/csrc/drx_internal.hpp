@@ -122,7 +122,8 @@ void scratch_unreserve(int dev, size_t bytes);
 // A block may be given back only when no work that uses it is left on the GPU,
 // so a kept block serves any stream at once. At most kBlocksKeep bytes are kept
 // per device; a failed allocation gives all of them back and tries again.
-void *block_alloc(size_t bytes);
+// (dev < 0: the current device; block_free and owned_free take the same one.)
+void *block_alloc(size_t bytes, int dev = -1);
 void block_free(int dev, void *p);
 // Blocks that any stream may have used: waits for the device, as hipFree does.
 // Where the runtime refuses the wait (a stream is being captured) they stay

@@ -111,19 +111,22 @@ struct HipMemory {
 };
 static BlockCache<HipMemory, kBlocksKeep> g_blocks[kMaxDevices];
 
-// Runs f with dev as the current device.
-template <typename F> static void on_device(int dev, F &&f) {
-  int cur = dev;
-  (void)hipGetDevice(&cur);
-  if (cur != dev) (void)hipSetDevice(dev);
-  f();
-  if (cur != dev) (void)hipSetDevice(cur);
-}
+// Makes dev the current device while it lives.
+struct OnDevice {
+  int cur, dev;
+  explicit OnDevice(int d) : cur(d), dev(d) {
+    (void)hipGetDevice(&cur);
+    if (cur != dev) (void)hipSetDevice(dev);
+  }
+  ~OnDevice() {
+    if (cur != dev) (void)hipSetDevice(cur);
+  }
+};
 
-void *block_alloc(size_t bytes) {
-  int dev = 0;
-  DRX_HIP(hipGetDevice(&dev));
+void *block_alloc(size_t bytes, int dev) {
+  if (dev < 0) DRX_HIP(hipGetDevice(&dev));
   DRX_REQUIRE(dev >= 0 && dev < kMaxDevices, "device ordinal out of range");
+  const OnDevice on(dev);
   void *p = nullptr;
   DRX_HIP(static_cast<hipError_t>(g_blocks[dev].take(bytes, &p)));
   return p;
@@ -138,7 +141,9 @@ void owned_free(int dev, const std::vector<void *> &ptrs) {
   if (dev < 0 || dev >= kMaxDevices) return;
   bool any = false;
   for (void *p : ptrs) any = any || p != nullptr;
-  if (any) on_device(dev, [&] { g_blocks[dev].retire(ptrs); });
+  if (!any) return;
+  const OnDevice on(dev);
+  g_blocks[dev].retire(ptrs);
 }
 
 // Fewest entries per row for which the wide-band kernel may run (band_mrhs).
