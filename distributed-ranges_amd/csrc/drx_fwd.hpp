@@ -890,12 +890,41 @@ __device__ __forceinline__ void load_xrow(const TX *p, TA (&xv)[KP]) {
   }
 }
 
-template <int WG, int G, int KP, typename TX, typename TY, typename TA,
+// Chains of additions per row. A lane adds its entries to CH partial sums in
+// turn, which are then added pairwise, as the lanes' sums are: the rounding
+// error is that of CH * G lanes with one sum each. It is least where a chain
+// takes 2.5 to 5 entries (a chain of m entries rounds about (m + 1) / 2 times per
+// entry, every doubling of the chains once more), whereas the gathers run best
+// with few lanes per row. RMS error against 64 bits, rows of 50 random entries,
+// FP32, in units of the last place over the root of the squared products: as
+// many lanes with one sum each 1.20, twice as many 1.10, these 1.10.
+struct MrhsLanes {
+  int g, ch;  // log2 of the lanes per row, of the partial sums per lane
+};
+template <int MOST> __device__ __forceinline__ MrhsLanes mrhs_lanes(int per_row, int gshift) {
+  // log2 of the chains that give each 2.5 to 5 entries
+  const int t = per_row * 2 / 5;
+  const int c = t < 2 ? 0 : 31 - __builtin_clz(static_cast<unsigned>(t));
+  const int fewer = MOST + (gshift > 1 ? gshift - 1 : 0);
+  const int g = c > fewer ? c - fewer : 0;
+  return {g, c - g < MOST ? c - g : MOST};
+}
+__device__ __forceinline__ float fma_acc(float v, float x, float s) { return __builtin_fmaf(v, x, s); }
+__device__ __forceinline__ double fma_acc(double v, double x, double s) { return __builtin_fma(v, x, s); }
+
+// x rows that a lane holds whole, in flight at once: eight or sixteen 16-bit
+// columns take eight or sixteen registers each as floats, and four of them cost
+// bands 1.1 (k = 8) to 1.9 (k = 16) times the time.
+template <int KP> constexpr int mrhs_inflight() { return KP >= 8 ? 2 : 4; }
+
+template <int WG, int G, int CH, int KP, typename TX, typename TY, typename TA,
           typename TI>
 __device__ __forceinline__ void reduce_rows_mrhs(
     const TA *v_s, const uint32_t *c_s, const int *rp_s, bool rows_lds,
     const FwdArgs &a, int64_t r0, int64_t e0, int64_t nr, const TX *xrc,
     int64_t j0, int kk, TA alpha, TA beta, int tid) {
+  constexpr int U = mrhs_inflight<KP>();
+  static_assert(CH <= U, "an entry in flight per chain");
   const TI *rowptr = static_cast<const TI *>(a.rowptr);
   TY *y = static_cast<TY *>(a.y);
   const int lane = tid & (G - 1);
@@ -908,29 +937,44 @@ __device__ __forceinline__ void reduce_rows_mrhs(
       s = static_cast<int>(row_begin(rowptr, a.base, a.nrows, a.nnz, a.sent, r0 + i) - e0);
       e = static_cast<int>(row_begin(rowptr, a.base, a.nrows, a.nnz, a.sent, r0 + i + 1) - e0);
     }
-    TA acc[KP];
+    TA part[CH][KP];
 #pragma unroll
-    for (int jj = 0; jj < KP; jj++) acc[jj] = 0;
+    for (int t = 0; t < CH; t++)
+#pragma unroll
+      for (int jj = 0; jj < KP; jj++) part[t][jj] = 0;
     int q = s + lane;
-    for (; q + G < e; q += 2 * G) {
-      TA x0[KP], x1[KP];
-      load_xrow<KP>(xrc + static_cast<size_t>(c_s[q]) * KP, x0);
-      load_xrow<KP>(xrc + static_cast<size_t>(c_s[q + G]) * KP, x1);
-      const TA v0 = v_s[q], v1 = v_s[q + G];
+    for (; q + (U - 1) * G < e; q += U * G) {
+      TA x[U][KP], v[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        load_xrow<KP>(xrc + static_cast<size_t>(c_s[q + u * G]) * KP, x[u]);
+        v[u] = v_s[q + u * G];
+      }
 #pragma unroll
       for (int jj = 0; jj < KP; jj++) {
-        acc[jj] += v0 * x0[jj] + v1 * x1[jj];
+#pragma unroll
+        for (int u = 0; u < U; u++) part[u % CH][jj] = fma_acc(v[u], x[u][jj], part[u % CH][jj]);
       }
     }
-    if (q < e) {
-      TA x0[KP];
-      load_xrow<KP>(xrc + static_cast<size_t>(c_s[q]) * KP, x0);
-      const TA v0 = v_s[q];
 #pragma unroll
-      for (int jj = 0; jj < KP; jj++) acc[jj] += v0 * x0[jj];
+    for (int u = 0; u < U - 1; u++) {
+      if (q < e) {
+        TA x0[KP];
+        load_xrow<KP>(xrc + static_cast<size_t>(c_s[q]) * KP, x0);
+        const TA v0 = v_s[q];
+#pragma unroll
+        for (int jj = 0; jj < KP; jj++) part[u % CH][jj] = fma_acc(v0, x0[jj], part[u % CH][jj]);
+        q += G;
+      }
     }
+    TA acc[KP];
 #pragma unroll
-    for (int jj = 0; jj < KP; jj++) acc[jj] = group_sum<G>(acc[jj]);
+    for (int jj = 0; jj < KP; jj++) {
+      acc[jj] = part[0][jj];
+      if constexpr (CH >= 2) acc[jj] += part[1][jj];
+      if constexpr (CH == 4) acc[jj] += part[2][jj] + part[3][jj];
+      acc[jj] = group_sum<G>(acc[jj]);
+    }
     const int64_t row = r0 + i;
 #pragma unroll
     for (int jj = 0; jj < KP; jj++) {
@@ -953,7 +997,7 @@ __device__ __forceinline__ void reduce_rows_mrhs(
 // and 16 values per entry in flight for FP32 k = 16) limited the batched
 // kernel to two waves per SIMD with two entries in flight per lane.
 // STAGE: the sums of row i go to yb[i * (KP + 1) + column] instead of y.
-template <int WG, int G, int KP, bool STAGE, typename TX, typename TY, typename TA,
+template <int WG, int G, int CH, int KP, bool STAGE, typename TX, typename TY, typename TA,
           typename TI>
 __device__ __forceinline__ void reduce_rows_mrhs_split(
     const TA *v_s, const uint32_t *c_s, const int *rp_s, bool rows_lds,
@@ -976,38 +1020,42 @@ __device__ __forceinline__ void reduce_rows_mrhs_split(
       s = static_cast<int>(row_begin(rowptr, a.base, a.nrows, a.nnz, a.sent, r0 + i) - e0);
       e = static_cast<int>(row_begin(rowptr, a.base, a.nrows, a.nnz, a.sent, r0 + i + 1) - e0);
     }
-    TA acc[KL];
+    TA part[CH][KL];
 #pragma unroll
-    for (int j = 0; j < KL; j++) acc[j] = 0;
+    for (int t = 0; t < CH; t++)
+#pragma unroll
+      for (int j = 0; j < KL; j++) part[t][j] = 0;
     const TX *xs = xrc + sub * KL;
     int q = s + el;
     for (; q + 3 * G < e; q += 4 * G) {
-      TA x0[KL], x1[KL], x2[KL], x3[KL];
-      load_xrow<KL>(xs + static_cast<size_t>(c_s[q]) * KP, x0);
-      load_xrow<KL>(xs + static_cast<size_t>(c_s[q + G]) * KP, x1);
-      load_xrow<KL>(xs + static_cast<size_t>(c_s[q + 2 * G]) * KP, x2);
-      load_xrow<KL>(xs + static_cast<size_t>(c_s[q + 3 * G]) * KP, x3);
-      const TA v0 = v_s[q], v1 = v_s[q + G], v2 = v_s[q + 2 * G], v3 = v_s[q + 3 * G];
+      TA x[4][KL], v[4];
 #pragma unroll
-      for (int j = 0; j < KL; j++) {
-        // (pairwise: a lane that takes more of a row's entries one after
-        // another would round more often)
-        acc[j] += (v0 * x0[j] + v1 * x1[j]) + (v2 * x2[j] + v3 * x3[j]);
+      for (int u = 0; u < 4; u++) {
+        load_xrow<KL>(xs + static_cast<size_t>(c_s[q + u * G]) * KP, x[u]);
+        v[u] = v_s[q + u * G];
       }
-    }
-    if (q < e) {
-      TA rest[KL];
 #pragma unroll
-      for (int j = 0; j < KL; j++) rest[j] = 0;
-      for (; q < e; q += G) {
+      for (int j = 0; j < KL; j++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) part[u % CH][j] = fma_acc(v[u], x[u][j], part[u % CH][j]);
+    }
+#pragma unroll
+    for (int u = 0; u < 3; u++) {
+      if (q < e) {
         TA x0[KL];
         load_xrow<KL>(xs + static_cast<size_t>(c_s[q]) * KP, x0);
         const TA v0 = v_s[q];
 #pragma unroll
-        for (int j = 0; j < KL; j++) rest[j] += v0 * x0[j];
+        for (int j = 0; j < KL; j++) part[u % CH][j] = fma_acc(v0, x0[j], part[u % CH][j]);
+        q += G;
       }
+    }
+    TA acc[KL];
 #pragma unroll
-      for (int j = 0; j < KL; j++) acc[j] += rest[j];
+    for (int j = 0; j < KL; j++) {
+      acc[j] = part[0][j];
+      if constexpr (CH >= 2) acc[j] += part[1][j];
+      if constexpr (CH == 4) acc[j] += part[2][j] + part[3][j];
     }
 #pragma unroll
     for (int o = S; o < GS; o *= 2) {
@@ -1147,19 +1195,19 @@ __device__ __forceinline__ void reduce_rows_mrhs_any(
     bool rows_lds, const FwdArgs &a, int64_t r0, int64_t e0, int64_t nr,
     const TX *xrc, int64_t j0, int kk, TA alpha, TA beta, TA *red, TA *yb, int tid) {
   if (nr <= 0) return;
-  // Few lanes per row, each with several entries in flight, use the gathers'
-  // slots best. us, thresholds as written / halved / quartered: 64 matrices of
-  // up to 200K rows of 3..64 entries, k = 16, 7408 / 5753 / 5185; band +-16, 2M
-  // rows, k = 8, FP32 399 / 261 / 224, FP64 752 / 495 / 423. gshift 1 is the
-  // default. (More entries in flight by masked or repeated ones in the last
-  // round lose: the gathers are bound by the misses that a CU's L1 keeps in
-  // flight, about 95, each 240 cycles from L2 and 900 from beyond.)
-  const int64_t avg = (n_s / nr) >> (a.gshift + 1);
   if (nr < WG / 64 && n_s / nr > 96) {
     reduce_rows_mrhs_wg<WG, KP, TX, TY, TA, TI>(v_s, c_s, rp_s, rows_lds, a, r0, e0, nr, xrc, j0,
                                                kk, alpha, beta, red, tid);
     return;
   }
+  // Few lanes per row, each with several entries in flight, use the gathers'
+  // slots best. us, lanes with about 2.5 / 5 / 10 entries each: 64 matrices of up
+  // to 200K rows of 3..64 entries, k = 16, 7408 / 5753 / 5185; band +-16, 2M rows,
+  // k = 8, FP32 399 / 261 / 224, FP64 752 / 495 / 423. (More entries in flight by
+  // masked or repeated ones in the last round lose: the gathers are bound by the
+  // misses that a CU's L1 keeps in flight, about 95, each 240 cycles from L2 and
+  // 900 from beyond.)
+  const int per_row = static_cast<int>(n_s / nr);
   constexpr int KL = 16 / static_cast<int>(sizeof(TX));
   if constexpr ((sizeof(TX) == 4 || sizeof(TX) == 8) && KP >= 2 * KL) {
     // 16-byte pieces of the x rows, S lanes per entry (G entry lanes per
@@ -1167,24 +1215,26 @@ __device__ __forceinline__ void reduce_rows_mrhs_any(
     constexpr int GMAX = 64 / (KP / KL);
     constexpr int G2 = 2 < GMAX ? 2 : GMAX, G4 = 4 < GMAX ? 4 : GMAX;
     constexpr int G8 = 8 < GMAX ? 8 : GMAX, G16 = 16 < GMAX ? 16 : GMAX;
+    const MrhsLanes w = mrhs_lanes<2>(per_row, a.gshift);
     // Sixteen sums of long rows are staged in LDS, for as many rows as fit, and
     // written column by column, consecutive rows from consecutive lanes: written
     // from the lanes that hold them they went to 16 lines per row, a third of
     // the kernel's L2 requests (the matrices above, k = 16: 5185 -> 4850 us;
     // fewer sums or shorter rows lose by the barriers).
     if constexpr (mrhs_staged<KP, TA>() > 0) {
-      if (avg > 6) {
+      if (per_row >> a.gshift > 12 && w.ch == 2) {
         constexpr int NB = mrhs_staged<KP, TA>() / (KP + 1);
         TY *y = static_cast<TY *>(a.y);
         for (int64_t i0 = 0; i0 < nr; i0 += NB) {
           const int nb = static_cast<int>(nr - i0 < NB ? nr - i0 : NB);
-#define DRX_RS(G) reduce_rows_mrhs_split<WG, G, KP, true, TX, TY, TA, TI>(v_s, c_s, rp_s + i0, rows_lds, a, r0 + i0, e0, nb, xrc, j0, kk, alpha, beta, yb, tid)
-          if (avg <= 12)
-            DRX_RS(G4);
-          else if (avg <= 24)
-            DRX_RS(G8);
-          else
-            DRX_RS(G16);
+#define DRX_RS(G) reduce_rows_mrhs_split<WG, G, 4, KP, true, TX, TY, TA, TI>(v_s, c_s, rp_s + i0, rows_lds, a, r0 + i0, e0, nb, xrc, j0, kk, alpha, beta, yb, tid)
+          switch (w.g) {
+            case 0: DRX_RS(1); break;
+            case 1: DRX_RS(G2); break;
+            case 2: DRX_RS(G4); break;
+            case 3: DRX_RS(G8); break;
+            default: DRX_RS(G16);
+          }
 #undef DRX_RS
           __syncthreads();
           for (int j = tid >> 6; j < kk; j += WG / 64) {
@@ -1200,35 +1250,39 @@ __device__ __forceinline__ void reduce_rows_mrhs_any(
         return;
       }
     }
-#define DRX_RS(G) reduce_rows_mrhs_split<WG, G, KP, false, TX, TY, TA, TI>(v_s, c_s, rp_s, rows_lds, a, r0, e0, nr, xrc, j0, kk, alpha, beta, yb, tid)
-    if (avg <= 3)
-      DRX_RS(1);
-    else if (avg <= 6)
-      DRX_RS(G2);
-    else if (avg <= 12)
-      DRX_RS(G4);
-    else if (avg <= 24)
-      DRX_RS(G8);
+#define DRX_RS(G, CH) reduce_rows_mrhs_split<WG, G, CH, KP, false, TX, TY, TA, TI>(v_s, c_s, rp_s, rows_lds, a, r0, e0, nr, xrc, j0, kk, alpha, beta, yb, tid)
+    if (w.ch == 0)
+      DRX_RS(1, 1);
+    else if (w.ch == 1)
+      DRX_RS(1, 2);
     else
-      DRX_RS(G16);
+      switch (w.g) {
+        case 0: DRX_RS(1, 4); break;
+        case 1: DRX_RS(G2, 4); break;
+        case 2: DRX_RS(G4, 4); break;
+        case 3: DRX_RS(G8, 4); break;
+        default: DRX_RS(G16, 4);
+      }
 #undef DRX_RS
     return;
   }
-#define DRX_RM(G) reduce_rows_mrhs<WG, G, KP, TX, TY, TA, TI>(v_s, c_s, rp_s, rows_lds, a, r0, e0, nr, xrc, j0, kk, alpha, beta, tid)
-  if (avg <= 3)
-    DRX_RM(1);
-  else if (avg <= 6)
-    DRX_RM(2);
-  else if (avg <= 12)
-    DRX_RM(4);
-  else if (avg <= 24)
-    DRX_RM(8);
-  else if (avg <= 48)
-    DRX_RM(16);
-  else if (avg <= 96)
-    DRX_RM(32);
+  constexpr int U = mrhs_inflight<KP>();
+  const MrhsLanes w = mrhs_lanes<(U == 4 ? 2 : 1)>(per_row, a.gshift);
+#define DRX_RM(G, CH) reduce_rows_mrhs<WG, G, CH, KP, TX, TY, TA, TI>(v_s, c_s, rp_s, rows_lds, a, r0, e0, nr, xrc, j0, kk, alpha, beta, tid)
+  if (w.ch == 0)
+    DRX_RM(1, 1);
+  else if (U == 4 && w.ch == 1)
+    DRX_RM(1, 2);
   else
-    DRX_RM(64);
+    switch (w.g) {
+      case 0: DRX_RM(1, U); break;
+      case 1: DRX_RM(2, U); break;
+      case 2: DRX_RM(4, U); break;
+      case 3: DRX_RM(8, U); break;
+      case 4: DRX_RM(16, U); break;
+      case 5: DRX_RM(32, U); break;
+      default: DRX_RM(64, U);
+    }
 #undef DRX_RM
 }
 
@@ -1331,14 +1385,15 @@ __device__ __forceinline__ void process_block_mrhs(const FwdArgs &a,
   __syncthreads();  // the next block overwrites the LDS window
 }
 
-// Waves per SIMD of the multi-RHS kernels: as many workgroups as the LDS
-// holds, at most the most that compile without spilling: 6 for sums of up
-// to 16 bytes per lane (73-78 VGPRs), 5 for wider ones taken in 16-byte
-// pieces (95), 4 for 16-bit x in wide chunks (whole chunks per lane).
+// Waves per SIMD of the multi-RHS kernels: as many workgroups as the LDS holds,
+// at most the most that compile without spilling: 5 for sums of up to 16 bytes
+// per lane and chain (four chains: 100 VGPRs), 4 for wider ones (up to 126).
+// With one wave more they spilled (batches, k = 4 and 16: 1.07 and 1.05 times
+// the time); the gathers' misses keep L1 full with either.
 template <int WG, int CAP, int KP, typename TX, typename TA> constexpr int mrhs_waves() {
   constexpr int lds = static_cast<int>(sizeof(MrhsSmem<WG, CAP, KP, TA>));
   constexpr int w = (160 * 1024) / lds * (WG / 256);
-  constexpr int most = KP * sizeof(TA) <= 16 ? 6 : (sizeof(TX) == 2 ? 4 : 5);
+  constexpr int most = KP * sizeof(TA) <= 16 ? 5 : 4;
   return w > most ? most : (w < 1 ? 1 : w);
 }
 

@@ -77,8 +77,10 @@ const char *drx_last_error(void);
  *                 average) with local columns (stencils; locality detected
  *                 once per colind pointer with one small kernel and a wait
  *                 on the stream).
- *   "mrhs_gshift" lane-group shift of the k >= 2 kernel, 0..3 (default 1: about
- *                 8 entries per lane of a row); also of new batches.
+ *   "mrhs_gshift" lane-group shift of the k >= 2 kernel, 0..3 (default 1, and 0:
+ *                 10 to 20 entries of a row per lane, in up to four partial
+ *                 sums of 2.5 to 5; 2 and 3: two and four times as many in
+ *                 four sums); also of new batches.
  *   "mrhs_kp_max" widest row-major chunk for 4-byte x: 16, 8, or 0 (default:
  *                 8 for k > 8 over loosely local columns -- stencils,
  *                 bands -- else 16; batches use 16). Fixed per call, and per

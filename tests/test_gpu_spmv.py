@@ -246,6 +246,45 @@ def test_multi_rhs_staged_sums(orc, vdt, k):
     Ad.close()
 
 
+def _chain_sums(v, x, chains):
+    """Sums of the rows of v * x (FP32, products fused) in `chains` chains of
+    additions, every chains-th entry, added pairwise."""
+    m, L = v.shape
+    part = np.zeros((m, chains), np.float32)
+    for e in range(L):
+        c = e % chains
+        part[:, c] = (v[:, e].astype(np.float64) * x[:, e] + part[:, c]).astype(np.float32)
+    while part.shape[1] > 1:
+        part = part[:, ::2] + part[:, 1::2]
+    return part[:, 0]
+
+
+@pytest.mark.parametrize("k", [4, 16])
+@pytest.mark.parametrize("L,chains", [(4, 1), (5, 2), (12, 4), (50, 16)])
+def test_multi_rhs_rounding_error(L, chains, k):
+    """The rounding error of a row's sum is that of chains of 2.5 to 5
+    additions, however many entries a lane takes: RMS over 400000 sums against
+    64 bits, at most 2 % above that of the same chains on the CPU (either RMS
+    has a standard error of about 0.2 %)."""
+    m, n = 400_000 // k, 50_000
+    rng = np.random.default_rng(L + k)
+    ci = np.sort(rng.integers(0, n, (m, L)), axis=1)
+    v = rng.uniform(-1, 1, (m, L)).astype(np.float32)
+    x = rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    Ad = upload(np.arange(m + 1) * L, ci.reshape(-1), v.reshape(-1), (m, n))
+    y = Ad.matvec(torch.as_tensor(x).to(DEV))
+    torch.cuda.synchronize()
+    y = y.cpu().numpy()
+    got = want = 0.0
+    for j in range(k):
+        p = v.astype(np.float64) * x[j][ci]
+        den = (p ** 2).sum(1)
+        got += ((y[j] - p.sum(1)) ** 2 / den).sum()
+        want += ((_chain_sums(v, x[j][ci], chains) - p.sum(1)) ** 2 / den).sum()
+    assert got <= 1.02 ** 2 * want
+    Ad.close()
+
+
 @pytest.mark.parametrize("vdt,xdt", [(torch.float64, torch.float64), (torch.float32, torch.float32),
                                      (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
 @pytest.mark.parametrize("m,k,order", [(1, 2, "sorted"), (9, 3, "sorted"), (203, 8, "sorted"),
