@@ -1451,7 +1451,7 @@ __global__ void k_x_rowmajor(const TX *x, int64_t ldx, int64_t ncols,
 void run_mrhs(const Plan &p, FwdArgs a, int mode, int vtype, int xtype,
               int ytype, hipStream_t s);
 // The same over wide bands (plain shares), reading x as it is.
-bool band_mrhs(const Plan &p, const FwdArgs &a, hipStream_t s);
+bool band_mrhs(const Plan &p, const FwdArgs &a, int xtype, hipStream_t s);
 void run_band(const Plan &p, FwdArgs a, int vtype, int xtype, int ytype, hipStream_t s);
 
 }  // namespace drx

@@ -262,7 +262,7 @@ int column_locality(const Plan &p, const void *colind, hipStream_t s) {
 // Bound by the matrix stream: 50000 rows of 2001 entries, k = 8, FP64 values and
 // 64-bit columns 315 us (5.1 TB/s; with its launch in a loop 345, the row-block
 // kernel 518; entries read again
-// in the next piece instead of kept: 390), FP32 and 32-bit columns 201 (325).
+// in the next piece instead of kept: 390), FP32 and 32-bit columns 190 (315).
 // U: FP64 2 / 4 / 8 batches 362 / 345 / 457 us, FP32 260 / 223 / 201.
 // ---------------------------------------------------------------------------
 constexpr int kBandRows = 8;                 // rows of a workgroup, two per wave
@@ -286,7 +286,19 @@ __device__ __forceinline__ void band_xcol(const TX *x, int64_t ldx, int64_t ncol
   for (int j = 0; j < KP; j++) t[j] = j < kk ? x[(j0 + j) * ldx + c] : TX{};
 }
 
-template <int KP, typename TV, typename TX, typename TY, typename TA, typename TI>
+// CH partial sums per lane, row and column, of every CH-th entry of the lane,
+// which are added at the end: W * CH chains of additions per row, as many as
+// the row-block kernel has at most (wg_row_sums), for rows that give each at
+// least 2.5 entries (see mrhs_lanes). With one, rows of 2001 entries had 1.28
+// (k <= 4) and 1.17 (k = 8) times that kernel's error; sixteen FP64 sums take one.
+template <int KP, typename TX, typename TA> constexpr int band_chains() {
+  constexpr int b = KP * static_cast<int>(sizeof(TA));
+  return b <= 16 ? 4 : (b <= 32 || (b == 64 && sizeof(TX) == 4) ? 2 : 1);
+}
+
+// Rows of fewer than 160 entries are summed by W = 32 lanes of their wave, for the
+// same reason (rows of 97: 0.6 % more error with 64 lanes than before, now less).
+template <int KP, int CH, int W, typename TV, typename TX, typename TY, typename TA, typename TI>
 __global__ __launch_bounds__(256) void k_spmv_band(FwdArgs a, int64_t j0) {
   constexpr int STRIDE = band_stride<KP, TX>(), PC = kBandLds / STRIDE / 64 * 64;
   constexpr int ALIGN = STRIDE < 16 ? STRIDE : 16;
@@ -318,25 +330,27 @@ __global__ __launch_bounds__(256) void k_spmv_band(FwdArgs a, int64_t j0) {
   int64_t at[RW], end[RW];
   uint32_t c[RW][U];
   TV w[RW][U];
-  TA acc[RW][KP];
-  // The next U * 64 entries of a row of the wave; lanes past its end are done.
+  TA acc[RW][CH][KP];
+  // The next U * W entries of a row of the wave; lanes past its end are done.
   auto load = [&](int r) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int64_t e = at[r] + u * 64 + lane;
+      const int64_t e = at[r] + u * W + lane;
       const int64_t ee = e < end[r] ? e : end[r] - 1;
       c[r][u] = col32(ld_stream(colind + ee));
       w[r][u] = ld_stream(vals + ee);
-      if (e >= end[r]) c[r][u] = kDone;
+      if (e >= end[r] || (W < 64 && lane >= W)) c[r][u] = kDone;
     }
-    at[r] += U * 64;
+    at[r] += U * W;
   };
 #pragma unroll
   for (int r = 0; r < RW; r++) {
     at[r] = row_at[wave * RW + r];
     end[r] = row_at[wave * RW + r + 1];
 #pragma unroll
-    for (int j = 0; j < KP; j++) acc[r][j] = 0;
+    for (int t = 0; t < CH; t++)
+#pragma unroll
+      for (int j = 0; j < KP; j++) acc[r][t][j] = 0;
     if (at[r] < end[r]) {
       load(r);
     } else {
@@ -373,7 +387,8 @@ __global__ __launch_bounds__(256) void k_spmv_band(FwdArgs a, int64_t j0) {
               band_xcol<KP>(x, a.ldx, a.ncols, j0, kk, c[r][u], t);
             const TA v = to_acc<TA>(w[r][u]);
 #pragma unroll
-            for (int j = 0; j < KP; j++) acc[r][j] += v * to_acc<TA>(t[j]);
+            for (int j = 0; j < KP; j++)
+              acc[r][u % CH][j] = fma_acc(v, to_acc<TA>(t[j]), acc[r][u % CH][j]);
             c[r][u] = kDone;
           }
           rest |= c[r][u] != kDone;
@@ -404,7 +419,10 @@ __global__ __launch_bounds__(256) void k_spmv_band(FwdArgs a, int64_t j0) {
   for (int r = 0; r < RW; r++) {
 #pragma unroll
     for (int j = 0; j < KP; j++) {
-      const TA sum = group_sum<64>(acc[r][j]);
+      TA sum = acc[r][0][j];
+      if constexpr (CH >= 2) sum += acc[r][1][j];
+      if constexpr (CH == 4) sum += acc[r][2][j] + acc[r][3][j];
+      sum = group_sum<64>(sum);
       if (lane == 0) ys[(wave * RW + r) * (KP + 1) + j] = sum;
     }
   }
@@ -421,13 +439,28 @@ __global__ __launch_bounds__(256) void k_spmv_band(FwdArgs a, int64_t j0) {
   }
 }
 
-template <int KP, typename TV, typename TX, typename TY, typename TA>
-static void launch_band(const Plan &p, const FwdArgs &a, int64_t j0, hipStream_t s) {
+template <int KP, int CH, int W, typename TV, typename TX, typename TY, typename TA>
+static void launch_band_ch(const Plan &p, const FwdArgs &a, int64_t j0, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(a.grid));
   if (p.itype == DRX_I32)
-    hipLaunchKernelGGL((k_spmv_band<KP, TV, TX, TY, TA, int32_t>), grid, dim3(256), 0, s, a, j0);
+    hipLaunchKernelGGL((k_spmv_band<KP, CH, W, TV, TX, TY, TA, int32_t>), grid, dim3(256), 0, s, a,
+                       j0);
   else
-    hipLaunchKernelGGL((k_spmv_band<KP, TV, TX, TY, TA, int64_t>), grid, dim3(256), 0, s, a, j0);
+    hipLaunchKernelGGL((k_spmv_band<KP, CH, W, TV, TX, TY, TA, int64_t>), grid, dim3(256), 0, s, a,
+                       j0);
+}
+
+template <int KP, typename TV, typename TX, typename TY, typename TA>
+static void launch_band(const Plan &p, const FwdArgs &a, int64_t j0, hipStream_t s) {
+  constexpr int MOST = band_chains<KP, TX, TA>();
+  if (MOST >= 4 && p.nnz >= 640 * p.nrows)
+    launch_band_ch<KP, MOST, 64, TV, TX, TY, TA>(p, a, j0, s);
+  else if (MOST >= 2 && p.nnz >= 320 * p.nrows)
+    launch_band_ch<KP, MOST < 2 ? MOST : 2, 64, TV, TX, TY, TA>(p, a, j0, s);
+  else if (p.nnz >= 160 * p.nrows)
+    launch_band_ch<KP, 1, 64, TV, TX, TY, TA>(p, a, j0, s);
+  else
+    launch_band_ch<KP, 1, 32, TV, TX, TY, TA>(p, a, j0, s);
 }
 
 template <typename TV, typename TX, typename TY, typename TA>
@@ -450,14 +483,16 @@ static void launch_band_t(const Plan &p, const FwdArgs &a, hipStream_t s) {
 // Plain shares of rows of much the same length whose neighbours hold
 // neighbouring columns (bit 2 of column_locality): long rows, where the matrix
 // stream covers the steps a workgroup takes one after the other (50000 rows, row
-// blocks / here: 401 entries FP32 k = 2 / 8 / 16 57 / 53, 73 / 69, 101 / 88 us,
-// FP64 74 / 68, 100 / 91, 147 / 147; 301 entries 47 / 48, 55 / 63, 76 / 82 and
-// 60 / 63, 83 / 84, 122 / 168; 601 entries 95 / 75, 124 / 91, 187 / 117), and
-// shorter ones where all workgroups are resident at once (8192 rows) and one
+// blocks / here: 401 entries FP32 k = 2 / 8 59 / 54, 73 / 69 us, FP64 k = 2 / 8 / 16
+// 75 / 70, 102 / 94, 154 / 156; 301 entries 47 / 48, 55 / 63 and 60 / 63, 83 / 84,
+// 122 / 168), longer ones still for more than eight FP32 right-hand sides (whose
+// sums leave three waves per SIMD: 401 entries k = 16 102 / 109, 501 167 / 122),
+// and shorter ones where all workgroups are resident at once (8192 rows) and one
 // launch without scratch counts for more (8000 rows of 97 entries FP64 k = 2 / 8 /
 // 16: 36 / 14, 34 / 15, 31 / 24 us).
-bool band_mrhs(const Plan &p, const FwdArgs &a, hipStream_t s) {
-  const int64_t least = p.nrows <= 8192 ? kBandLeast : 4 * kBandLeast;
+bool band_mrhs(const Plan &p, const FwdArgs &a, int xtype, hipStream_t s) {
+  const int64_t least =
+      p.nrows <= 8192 ? kBandLeast : (xtype == DRX_F32 && a.k > 8 ? 5 : 4) * kBandLeast;
   return p.lmax > 0 && p.nnz >= least * p.nrows && p.lmax * p.nrows <= 4 * p.nnz &&
          a.xbytes > 0 && (column_locality(p, a.colind, s) & 4) != 0;
 }

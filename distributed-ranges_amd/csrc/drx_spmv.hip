@@ -302,7 +302,7 @@ static void run_spmv_impl(const Plan &p, int vtype, const void *colind,
   const bool stencil = k <= 4 && p.nnz <= 8 * p.nrows;
   if (k >= 2 && mr != 0 &&
       (mr == 2 || !stencil || (column_locality(p, colind, s) & 1) == 0)) {
-    if (MODE == kPlain && mr == 1 && band_mrhs(p, a, s)) {
+    if (MODE == kPlain && mr == 1 && band_mrhs(p, a, xtype, s)) {
       run_band(p, a, vtype, xtype, ytype, s);
       return;
     }
