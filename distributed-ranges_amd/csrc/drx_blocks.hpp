@@ -23,12 +23,13 @@ namespace drx {
 //   int alloc(void **p, size_t bytes)  0, kOutOfMemory or another status
 //   bool free(void *p)                 false: refused, p is still allocated
 //   bool wait()                        true: all work queued before has ended
-template <typename Driver, size_t Keep> class BlockCache {
+// At most Keep bytes are kept; sizes are rounded up to a Quantum.
+template <typename Driver, size_t Keep, size_t Quantum = 4096> class BlockCache {
 public:
   // A block of at least `bytes`, or the status of the failed allocation. A
   // failed one gives all kept blocks back and tries again.
   int take(size_t bytes, void **out) {
-    bytes = (std::max<size_t>(bytes, 1) + 4095) & ~size_t(4095);
+    bytes = (std::max<size_t>(bytes, 1) + Quantum - 1) / Quantum * Quantum;
     if (find(bytes, out)) return 0;
     if (settle() && find(bytes, out)) return 0;
     void *p = nullptr;
@@ -49,14 +50,14 @@ public:
     }
   }
 
-  // Blocks that queued work may still use.
-  template <typename Ptrs> void retire(const Ptrs &ptrs) {
+  // Blocks that queued work may still use; whether the device has been waited for.
+  template <typename Ptrs> bool retire(const Ptrs &ptrs) {
     {
       std::lock_guard<std::mutex> lk(mu_);
       for (void *p : ptrs)
         if (size_.count(p)) parked_.push_back(p);
     }
-    settle();
+    return settle();
   }
 
   // Waits for the device, and keeps the blocks that were retired before; false

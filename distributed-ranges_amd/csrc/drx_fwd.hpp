@@ -50,6 +50,7 @@ struct FwdArgs {
   int64_t lmax;   // longest row of the share (-1 unknown): row-ordered round size
   const void *xr;  // k >= 2: x in row-major chunks of KP columns
   int64_t ncols;   // columns of the share (rows of one xr chunk)
+  const int *gate; // set: k_spmv_band runs where it holds 1, k_spmv_mrhs where 0
 };
 
 template <int WG, typename TA>
@@ -1403,6 +1404,7 @@ __global__ __launch_bounds__(WG)
 __attribute__((amdgpu_waves_per_eu(mrhs_waves<WG, CAP, KP, TX, TA>(), 8)))
 void k_spmv_mrhs(FwdArgs a) {
   __shared__ MrhsSmem<WG, CAP, KP, TA> sm;
+  if (a.gate != nullptr && *a.gate != 0) return;
   for (int64_t wi = blockIdx.x; wi < a.per_xcd * kXcds; wi += a.grid) {
     const int64_t blk = map_block(wi, a.per_xcd);
     if (blk >= a.nblocks) continue;
@@ -1410,10 +1412,12 @@ void k_spmv_mrhs(FwdArgs a) {
   }
 }
 
-// Row-major chunks of x (layout above); one thread per (chunk, column).
+// Row-major chunks of x (layout above); one thread per (chunk, column). Nothing
+// where `gate` is set and holds 1 (k_spmv_band reads x as it is).
 template <int KP, typename TX>
 __global__ void k_x_rowmajor(const TX *x, int64_t ldx, int64_t ncols,
-                             int64_t k, TX *xr) {
+                             int64_t k, TX *xr, const int *gate) {
+  if (gate != nullptr && *gate != 0) return;
   const int64_t nchunk = (k + KP - 1) / KP;
   const int64_t total = nchunk * ncols;
   for (int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1447,11 +1451,14 @@ __global__ void k_x_rowmajor(const TX *x, int64_t ldx, int64_t ncols,
 }
 
 // Host side (drx_mrhs.hip): copy x into row-major chunks and launch the
-// multi-RHS kernel for a plain (mode kPlain) or permuted (kPerm) share.
+// multi-RHS kernel for a plain (mode kPlain) or permuted (kPerm) share. `probe`:
+// a kernel before finds out whether the share is a wide band, and run_band's
+// kernels or these do the work.
 void run_mrhs(const Plan &p, FwdArgs a, int mode, int vtype, int xtype,
-              int ytype, hipStream_t s);
+              int ytype, bool probe, hipStream_t s);
 // The same over wide bands (plain shares), reading x as it is.
-bool band_mrhs(const Plan &p, const FwdArgs &a, int xtype, hipStream_t s);
+enum BandChoice { kBandNo = 0, kBandYes = 1, kBandProbe = 2 };
+BandChoice band_mrhs(const Plan &p, const FwdArgs &a, int xtype, hipStream_t s);
 void run_band(const Plan &p, FwdArgs a, int vtype, int xtype, int ytype, hipStream_t s);
 
 }  // namespace drx

@@ -21,6 +21,7 @@ namespace drx {
 static std::atomic<int64_t> g_block_nnz{0};
 static std::atomic<int> g_mrhs{1};
 static std::atomic<int> g_mrhs_gshift{1};
+static std::atomic<int> g_mrhs_band{1};
 static std::atomic<int> g_vec{0};
 static std::atomic<int> g_wide{1};
 int tuned_wide() { return g_wide.load(); }
@@ -28,6 +29,7 @@ static std::atomic<int64_t> g_grid_cap{0};
 
 int tuned_mrhs() { return g_mrhs.load(); }
 int tuned_mrhs_gshift() { return g_mrhs_gshift.load(); }
+int tuned_mrhs_band() { return g_mrhs_band.load(); }
 static std::atomic<int> g_mrhs_kp_max{0};
 int tuned_mrhs_kp_max() { return g_mrhs_kp_max.load(); }
 int tuned_vec() { return g_vec.load(); }
@@ -381,6 +383,9 @@ int drx_tune_set(const char *key, int64_t value) {
     } else if (std::strcmp(key, "mrhs_gshift") == 0) {
       DRX_REQUIRE(value >= 0 && value <= 3, "mrhs_gshift must be in [0, 3]");
       g_mrhs_gshift.store(static_cast<int>(value));
+    } else if (std::strcmp(key, "mrhs_band") == 0) {
+      DRX_REQUIRE(value >= 0 && value <= 2, "mrhs_band must be 0, 1 or 2");
+      g_mrhs_band.store(static_cast<int>(value));
     } else if (std::strcmp(key, "mrhs_kp_max") == 0) {
       DRX_REQUIRE(value == 0 || value == 8 || value == 16, "mrhs_kp_max must be 0, 8 or 16");
       g_mrhs_kp_max.store(static_cast<int>(value));
@@ -428,6 +433,8 @@ int drx_tune_get(const char *key, int64_t *value) {
       *value = g_mrhs.load();
     else if (std::strcmp(key, "mrhs_gshift") == 0)
       *value = g_mrhs_gshift.load();
+    else if (std::strcmp(key, "mrhs_band") == 0)
+      *value = g_mrhs_band.load();
     else if (std::strcmp(key, "vec") == 0)
       *value = g_vec.load();
     else if (std::strcmp(key, "wide") == 0)

@@ -44,13 +44,17 @@ struct Plan {
   PanelSet *panels = nullptr;  // column-panel layout (drx_plan_set_panels)
   // Cached column locality of the share for one colind pointer (k >= 2
   // path choice): -1 unknown, else bit 0 = tight (row blocks span about as
-  // many columns as entries), bit 1 = loose (within ncols / 16), bit 2 =
-  // shared (neighbouring rows hold the same columns).
+  // many columns as entries), bit 1 = loose (within ncols / 16).
   // Atomics: calls sharing the plan from several threads read and write the
   // cache without a lock. A torn read only picks the other, equally correct,
   // k >= 2 path once.
   mutable std::atomic<const void *> loc_colind{nullptr};
   mutable std::atomic<int> loc_local{-1};
+  // Host memory that probing kernels write (null: none): word 0, wide bands, the
+  // last answer -- colind pointer << 1 | band, 0 none yet --; from word 1 on the
+  // counts of column_locality. And the colind of the last band probe launched.
+  uint64_t *slot = nullptr;
+  mutable std::atomic<const void *> band_colind{nullptr};
   // Records in a caller's buffer (init_plan_in): products take no scratch
   // (k >= 2 gathers the k columns of x) and probe nothing.
   bool no_scratch = false;
@@ -83,6 +87,9 @@ int64_t default_block_nnz(int itype);
 // the k columns of x directly; lane-group shift of the row-major kernel.
 int tuned_mrhs();
 int tuned_mrhs_gshift();
+// Wide-band kernel for k >= 2: 0 never, 1 by the plan's rows and columns, 2
+// wherever it can run.
+int tuned_mrhs_band();
 int tuned_mrhs_kp_max();  // widest chunk for 4-byte x: 0 by locality, 8, 16
 // Entries per lane of the streaming loads: 0 = by type and mode, 1, or 2
 // where eligible;
@@ -128,7 +135,15 @@ void block_free(int dev, void *p);
 // Blocks that any stream may have used: waits for the device, as hipFree does.
 // Where the runtime refuses the wait (a stream is being captured) they stay
 // aside until a later one succeeds.
-void owned_free(int dev, const std::vector<void *> &ptrs);
+// True: the device has been waited for.
+bool owned_free(int dev, const std::vector<void *> &ptrs);
+// 64 bytes of pinned host memory for kernels of device dev to write, the first
+// word zeroed; null when there are none. slot_free: `waited`, no work is left
+// that writes them, else as owned_free.
+uint64_t *slot_alloc(int dev);
+void slot_free(int dev, uint64_t *slot, bool waited);
+// Fewest entries per row for which the wide-band kernel may run by itself.
+constexpr int64_t kBandLeast = 96;
 
 // Row-major chunks of x for k >= 2 right-hand sides: chunk width KP and the
 // bytes of all chunks; the copy kernel.
@@ -138,14 +153,13 @@ void owned_free(int dev, const std::vector<void *> &ptrs);
 int mrhs_kp(int64_t k, int xtype, bool loose_local = false);
 // Column locality of the share: bit 0 when most row blocks' windows span few
 // more columns than entries (banded, 2-D stencils), bit 1 when they span at
-// most ncols / 16 (3-D stencils too), bit 2 when eight neighbouring rows hold
-// each column of their span twice or more (wide bands). Measured once per
-// colind pointer (one small kernel and a wait), cached in the plan; 0 while the
-// stream is being captured.
+// most ncols / 16 (3-D stencils too). Measured once per colind pointer (one
+// small kernel and a wait), cached in the plan; 0 while the stream is being
+// captured.
 int column_locality(const Plan &p, const void *colind, hipStream_t s);
 size_t mrhs_xr_bytes(int64_t ncols, int64_t k, int kp, int xtype);
 void launch_x_rowmajor(int xtype, const void *x, int64_t ldx, int64_t ncols,
-                       int64_t k, int kp, void *xr, hipStream_t s);
+                       int64_t k, int kp, void *xr, const int *gate, hipStream_t s);
 
 // fill: measure the longest row (waits for the stream) so that blocks fill
 // their windows (block_pitch); otherwise blocks start every half window.

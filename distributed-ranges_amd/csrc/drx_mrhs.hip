@@ -137,35 +137,74 @@ void block_free(int dev, void *p) {
   g_blocks[dev].give(p);
 }
 
-void owned_free(int dev, const std::vector<void *> &ptrs) {
-  if (dev < 0 || dev >= kMaxDevices) return;
+bool owned_free(int dev, const std::vector<void *> &ptrs) {
+  if (dev < 0 || dev >= kMaxDevices) return false;
   bool any = false;
   for (void *p : ptrs) any = any || p != nullptr;
-  if (!any) return;
+  if (!any) return false;
   const OnDevice on(dev);
-  g_blocks[dev].retire(ptrs);
+  return g_blocks[dev].retire(ptrs);
 }
 
-// Fewest entries per row for which the wide-band kernel may run (band_mrhs).
-constexpr int64_t kBandLeast = 96;
+// ---------------------------------------------------------------------------
+// Slots: 64 bytes each of pinned memory, out of pieces of 64 KB that stay
+// allocated (a slot is used again by later plans).
+// ---------------------------------------------------------------------------
+struct PinnedSlots {
+  static constexpr int kOutOfMemory = -1;
+  static constexpr size_t kPiece = 65536, kSlot = 64;
+  static int alloc(void **p, size_t) {
+    static std::mutex mu;
+    static char *piece = nullptr;
+    static size_t used = kPiece;
+    std::lock_guard<std::mutex> lk(mu);
+    if (used == kPiece) {
+      void *q = nullptr;
+      const hipError_t e = HipMemory::cleared(
+          hipHostMalloc(&q, kPiece, hipHostMallocMapped | hipHostMallocCoherent));
+      if (e != hipSuccess) return e;
+      piece = static_cast<char *>(q);
+      used = 0;
+    }
+    *p = piece + used;
+    used += kSlot;
+    return 0;
+  }
+  static bool free(void *) { return false; }
+  static bool wait() { return HipMemory::wait(); }
+};
+static BlockCache<PinnedSlots, SIZE_MAX, PinnedSlots::kSlot> g_slots[kMaxDevices];
+
+uint64_t *slot_alloc(int dev) {
+  void *p = nullptr;
+  if (dev < 0 || dev >= kMaxDevices || g_slots[dev].take(PinnedSlots::kSlot, &p) != 0)
+    return nullptr;
+  *static_cast<volatile uint64_t *>(p) = 0;
+  return static_cast<uint64_t *>(p);
+}
+
+void slot_free(int dev, uint64_t *slot, bool waited) {
+  if (slot == nullptr) return;
+  if (waited) {
+    g_slots[dev].give(slot);
+    return;
+  }
+  const OnDevice on(dev);
+  g_slots[dev].retire(std::initializer_list<void *>{slot});
+}
 
 // Samples up to 4096 row blocks: the span between the first and the last
 // column index of each window, against its entry count (tight: at most
-// 4 n + 64) and against ncols / 16 (loose); and the columns that the eight rows
-// from the block's first on span together, against the entries they hold
-// (long rows only; shared: at most half as many columns). out = {tight, loose, sampled,
-// shared}. One workgroup, bound by the chain record, row start, column: as many
-// lanes as it can have, a sample's loads all in flight.
+// 4 n + 64) and against ncols / 16 (loose). out = {tight, loose, sampled}. One
+// workgroup, bound by the chain record, column.
 template <typename TI>
-__global__ __launch_bounds__(1024) void k_col_local(const BlockRec *rec, int64_t nblocks,
-                                                    int64_t ncols, const TI *colind,
-                                                    const TI *rowptr, int64_t base, int64_t nrows,
-                                                    int64_t nnz, int sent, int *out) {
-  __shared__ int cnt[4];
-  if (threadIdx.x < 4) cnt[threadIdx.x] = 0;
+__global__ __launch_bounds__(256) void k_col_local(const BlockRec *rec, int64_t nblocks,
+                                                    int64_t ncols, const TI *colind, int *out) {
+  __shared__ int cnt[3];
+  if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
   __syncthreads();
   const int64_t S = nblocks < 4096 ? nblocks : 4096;
-  int tight = 0, loose = 0, seen = 0, shared = 0;
+  int tight = 0, loose = 0, seen = 0;
   for (int64_t i = threadIdx.x; i < S; i += blockDim.x) {
     const BlockRec b = rec[i * nblocks / S];
     const int64_t n = b.es - b.e0;
@@ -176,71 +215,53 @@ __global__ __launch_bounds__(1024) void k_col_local(const BlockRec *rec, int64_t
       seen++;
       if (span <= 4 * n + 64) tight++;
       if (span <= 4 * n + 64 || span <= ncols / 16) loose++;
-      if (nnz < kBandLeast * nrows) continue;  // (no band, whatever the columns)
-      int64_t at[9], c0[8], c1[8];
-#pragma unroll
-      for (int q = 0; q < 9; q++) {
-        const int64_t r = b.r0 + q < nrows ? b.r0 + q : nrows;
-        at[q] = row_begin(rowptr, base, nrows, nnz, sent, r);
-      }
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        c0[q] = static_cast<int64_t>(colind[at[q] < nnz ? at[q] : nnz - 1]);
-        c1[q] = static_cast<int64_t>(colind[at[q + 1] > 0 ? at[q + 1] - 1 : 0]);
-      }
-      const int64_t held = at[8] - at[0];
-      int64_t first = ncols, last = 0;
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        if (at[q] >= at[q + 1]) continue;
-        first = c0[q] < first ? c0[q] : first;
-        last = c1[q] > last ? c1[q] : last;
-      }
-      if (2 * (last - first) <= held) shared++;
     }
   }
   atomicAdd(&cnt[0], tight);
   atomicAdd(&cnt[1], loose);
   atomicAdd(&cnt[2], seen);
-  atomicAdd(&cnt[3], shared);
   __syncthreads();
-  if (threadIdx.x < 4) out[threadIdx.x] = cnt[threadIdx.x];
+  if (threadIdx.x < 3) out[threadIdx.x] = cnt[threadIdx.x];
+}
+
+// The cached locality of a column array, -1 where it is not known.
+static int locality_known(const Plan &p, const void *colind) {
+  const int cached = p.loc_local.load(std::memory_order_acquire);
+  return p.loc_colind.load(std::memory_order_acquire) == colind ? cached : -1;
 }
 
 int column_locality(const Plan &p, const void *colind, hipStream_t s) {
   if (p.nnz == 0 || p.nblocks == 0 || colind == nullptr) return 0;
-  {
-    const int cached = p.loc_local.load(std::memory_order_acquire);
-    if (cached >= 0 && p.loc_colind.load(std::memory_order_acquire) == colind) return cached;
-  }
+  if (const int cached = locality_known(p, colind); cached >= 0) return cached;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   DRX_HIP(hipStreamIsCapturing(s, &st));
   if (st != hipStreamCaptureStatusNone) return 0;
-  int *d = static_cast<int *>(scratch_alloc(4 * sizeof(int), s));
-  int h[4] = {0, 0, 0, 0};
+  // (the counts straight into the plan's host memory, where it has some: scratch
+  // and a copy back take 10 us more)
+  int h[3] = {0, 0, 0};
+  int *d = p.slot ? reinterpret_cast<int *>(p.slot + 1)
+                  : static_cast<int *>(scratch_alloc(sizeof(h), s));
   try {
     if (p.itype == DRX_I32)
-      hipLaunchKernelGGL(k_col_local<int32_t>, dim3(1), dim3(1024), 0, s, p.rec, p.nblocks,
-                         p.ncols, static_cast<const int32_t *>(colind),
-                         static_cast<const int32_t *>(p.rowptr), p.base, p.nrows, p.nnz,
-                         p.has_sentinel, d);
+      hipLaunchKernelGGL(k_col_local<int32_t>, dim3(1), dim3(256), 0, s, p.rec, p.nblocks,
+                         p.ncols, static_cast<const int32_t *>(colind), d);
     else
-      hipLaunchKernelGGL(k_col_local<int64_t>, dim3(1), dim3(1024), 0, s, p.rec, p.nblocks,
-                         p.ncols, static_cast<const int64_t *>(colind),
-                         static_cast<const int64_t *>(p.rowptr), p.base, p.nrows, p.nnz,
-                         p.has_sentinel, d);
+      hipLaunchKernelGGL(k_col_local<int64_t>, dim3(1), dim3(256), 0, s, p.rec, p.nblocks,
+                         p.ncols, static_cast<const int64_t *>(colind), d);
     DRX_HIP(hipGetLastError());
-    DRX_HIP(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
+    if (!p.slot) DRX_HIP(hipMemcpyAsync(h, d, sizeof(h), hipMemcpyDeviceToHost, s));
     DRX_HIP(hipStreamSynchronize(s));
   } catch (...) {
-    scratch_free(d, s);
+    if (!p.slot) scratch_free(d, s);
     throw;
   }
-  scratch_free(d, s);
+  if (!p.slot)
+    scratch_free(d, s);
+  else
+    for (int i = 0; i < 3; i++) h[i] = static_cast<volatile int *>(d)[i];
   int loc = 0;
   if (h[2] > 0 && 10 * h[0] >= 9 * h[2]) loc |= 1;
   if (h[2] > 0 && 10 * h[1] >= 9 * h[2]) loc |= 2;
-  if (h[2] > 0 && 10 * h[3] >= 9 * h[2]) loc |= 4;
   // Invalidate, then publish pointer and value.
   p.loc_local.store(-1, std::memory_order_release);
   p.loc_colind.store(colind, std::memory_order_release);
@@ -310,6 +331,7 @@ __global__ __launch_bounds__(256) void k_spmv_band(FwdArgs a, int64_t j0) {
   __shared__ TA ys[kBandRows * (KP + 1)];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (a.gate != nullptr && *a.gate == 0) return;
   const int64_t blk = map_block(blockIdx.x, a.per_xcd);
   if (blk >= a.nblocks) return;  // the whole workgroup
   const int64_t r0 = blk * kBandRows;
@@ -480,8 +502,87 @@ static void launch_band_t(const Plan &p, const FwdArgs &a, hipStream_t s) {
   }
 }
 
+// Whether eight neighbouring rows hold the columns that they span at least
+// twice, for nine in ten of up to 128 groups of rows: *gate, and with colind's
+// address the plan's slot. One workgroup, eight lanes per group, all loads of
+// a lane in two steps. The answer steers the kernels that follow it on the
+// stream (first call on a column array: either these or the row blocks run,
+// the others leave at once), so the host does not wait for it; later calls find
+// it in the slot. (With a host wait, as one workgroup over 4096 samples, the first
+// product of 8000 rows of 97..400 entries took 75..110 us instead of 37..40.)
+constexpr int kBandGroups = 128;
+template <typename TI>
+__global__ __launch_bounds__(8 * kBandGroups) void k_band_probe(const TI *rowptr, int64_t base,
+                                                                int64_t nrows, int64_t nnz,
+                                                                int sent, const TI *colind,
+                                                                int *gate, uint64_t *slot) {
+  __shared__ int cnt[2];
+  if (threadIdx.x < 2) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int64_t groups = (nrows + 7) / 8, S = groups < kBandGroups ? groups : kBandGroups;
+  const int64_t i = threadIdx.x / 8;
+  const int64_t r = i < S ? i * groups / S * 8 + threadIdx.x % 8 : nrows;
+  int64_t at = 0, end = 0;
+  if (r < nrows) {
+    at = row_begin(rowptr, base, nrows, nnz, sent, r);
+    end = row_begin(rowptr, base, nrows, nnz, sent, r + 1);
+  }
+  int64_t first = INT64_MAX, last = 0, held = 0;
+  if (at < end) {
+    first = static_cast<int64_t>(colind[at]);
+    last = static_cast<int64_t>(colind[end - 1]);
+    held = end - at;
+  }
+#pragma unroll
+  for (int o = 1; o < 8; o *= 2) {
+    const int64_t f = __shfl_xor(first, o, 64), l = __shfl_xor(last, o, 64);
+    first = f < first ? f : first;
+    last = l > last ? l : last;
+    held += __shfl_xor(held, o, 64);
+  }
+  if (threadIdx.x % 8 == 0 && held > 0) {
+    atomicAdd(&cnt[0], 1);
+    if (2 * (last - first) <= held) atomicAdd(&cnt[1], 1);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const int band = cnt[0] > 0 && 10 * cnt[1] >= 9 * cnt[0];
+    if (gate != nullptr) *gate = band;
+    __hip_atomic_store(slot, (reinterpret_cast<uint64_t>(colind) << 1) | band, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
+static void launch_band_probe(const Plan &p, const FwdArgs &a, int *gate, hipStream_t s) {
+  p.band_colind.store(a.colind, std::memory_order_relaxed);
+  if (p.itype == DRX_I32)
+    hipLaunchKernelGGL(k_band_probe<int32_t>, dim3(1), dim3(8 * kBandGroups), 0, s,
+                       static_cast<const int32_t *>(p.rowptr), p.base, p.nrows, p.nnz,
+                       p.has_sentinel, static_cast<const int32_t *>(a.colind), gate, p.slot);
+  else
+    hipLaunchKernelGGL(k_band_probe<int64_t>, dim3(1), dim3(8 * kBandGroups), 0, s,
+                       static_cast<const int64_t *>(p.rowptr), p.base, p.nrows, p.nnz,
+                       p.has_sentinel, static_cast<const int64_t *>(a.colind), gate, p.slot);
+  DRX_HIP(hipGetLastError());
+}
+
+// What the plan's slot says of a column array: kBandProbe, nothing.
+static BandChoice band_known(const Plan &p, const void *colind) {
+  const uint64_t v = __atomic_load_n(p.slot, __ATOMIC_RELAXED);
+  if (v == 0 || v >> 1 != reinterpret_cast<uint64_t>(colind)) return kBandProbe;
+  return v & 1 ? kBandYes : kBandNo;
+}
+
+// Whether run_mrhs takes its chunk width from the columns' locality: 8-wide
+// chunks for k > 8 when the columns are loosely local (measured on the 3-D
+// Laplacian 128^3 FP32, k = 16: 2293 vs 1982 GB/s, while a matrix of random
+// columns runs half as fast with them: 323 vs 618 GB/s).
+static bool mrhs_asks_locality(int64_t k, int xtype) {
+  return k > 8 && dtype_size(xtype) == 4 && tuned_mrhs_kp_max() == 0;
+}
+
 // Plain shares of rows of much the same length whose neighbours hold
-// neighbouring columns (bit 2 of column_locality): long rows, where the matrix
+// neighbouring columns (k_band_probe): long rows, where the matrix
 // stream covers the steps a workgroup takes one after the other (50000 rows, row
 // blocks / here: 401 entries FP32 k = 2 / 8 59 / 54, 73 / 69 us, FP64 k = 2 / 8 / 16
 // 75 / 70, 102 / 94, 154 / 156; 301 entries 47 / 48, 55 / 63 and 60 / 63, 83 / 84,
@@ -490,11 +591,29 @@ static void launch_band_t(const Plan &p, const FwdArgs &a, hipStream_t s) {
 // and shorter ones where all workgroups are resident at once (8192 rows) and one
 // launch without scratch counts for more (8000 rows of 97 entries FP64 k = 2 / 8 /
 // 16: 36 / 14, 34 / 15, 31 / 24 us).
-bool band_mrhs(const Plan &p, const FwdArgs &a, int xtype, hipStream_t s) {
+BandChoice band_mrhs(const Plan &p, const FwdArgs &a, int xtype, hipStream_t s) {
+  const int knob = tuned_mrhs_band();
+  if (knob == 0 || a.xbytes == 0) return kBandNo;
+  if (knob == 2) return kBandYes;
   const int64_t least =
       p.nrows <= 8192 ? kBandLeast : (xtype == DRX_F32 && a.k > 8 ? 5 : 4) * kBandLeast;
-  return p.lmax > 0 && p.nnz >= least * p.nrows && p.lmax * p.nrows <= 4 * p.nnz &&
-         a.xbytes > 0 && (column_locality(p, a.colind, s) & 4) != 0;
+  if (p.slot == nullptr || p.nnz < least * p.nrows || p.lmax * p.nrows > 4 * p.nnz)
+    return kBandNo;
+  const BandChoice known = band_known(p, a.colind);
+  if (known != kBandProbe) return known;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  DRX_HIP(hipStreamIsCapturing(s, &st));
+  // A capture asks only where a probe was launched before (whose answer may be
+  // on its way), so that what it records does not hang on timing.
+  if (st != hipStreamCaptureStatusNone)
+    return p.band_colind.load(std::memory_order_relaxed) == a.colind ? kBandProbe : kBandNo;
+  if (mrhs_asks_locality(a.k, xtype) && locality_known(p, a.colind) < 0) {
+    // the chunk width hangs on a probe that the host waits for: one wait
+    launch_band_probe(p, a, nullptr, s);
+    (void)column_locality(p, a.colind, s);
+    return band_known(p, a.colind);
+  }
+  return kBandProbe;
 }
 
 void run_band(const Plan &p, FwdArgs a, int vtype, int xtype, int ytype, hipStream_t s) {
@@ -536,13 +655,13 @@ size_t mrhs_xr_bytes(int64_t ncols, int64_t k, int kp, int xtype) {
 // x -> xr on stream s (only the element size matters: the zero padding is
 // all-zero bits, +0 in every floating type).
 void launch_x_rowmajor(int xtype, const void *x, int64_t ldx, int64_t ncols,
-                       int64_t k, int kp, void *xr, hipStream_t s) {
+                       int64_t k, int kp, void *xr, const int *gate, hipStream_t s) {
   const int64_t total = ((k + kp - 1) / kp) * ncols;
   if (total == 0) return;
   const dim3 g(static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 1 << 16)));
 #define DRX_XR(KP, T)                                                          \
   hipLaunchKernelGGL((k_x_rowmajor<KP, T>), g, dim3(256), 0, s,                \
-                     static_cast<const T *>(x), ldx, ncols, k, static_cast<T *>(xr))
+                     static_cast<const T *>(x), ldx, ncols, k, static_cast<T *>(xr), gate)
 #define DRX_XR_T(T)                                                            \
   do {                                                                         \
     if (kp == 2)                                                               \
@@ -608,18 +727,22 @@ static void launch_mrhs_t(const Plan &p, const FwdArgs &a, int mode, int kp,
 }
 
 void run_mrhs(const Plan &p, FwdArgs a, int mode, int vtype, int xtype,
-              int ytype, hipStream_t s) {
+              int ytype, bool probe, hipStream_t s) {
   DRX_REQUIRE(mode == kPlain || mode == kPerm, "bad mode for k >= 2");
-  // one chunk width for the copy and the kernel (the knob may change);
-  // 8-wide chunks for k > 8 when the columns are loosely local (measured on
-  // the 3-D Laplacian 128^3 FP32, k = 16: 2293 vs 1982 GB/s, while a matrix
-  // of random columns runs half as fast with them: 323 vs 618 GB/s)
-  const bool loose = a.k > 8 && dtype_size(xtype) == 4 && tuned_mrhs_kp_max() == 0 &&
-                     (column_locality(p, a.colind, s) & 2) != 0;
+  // one chunk width for the copy and the kernel (the knob may change)
+  const bool loose =
+      mrhs_asks_locality(a.k, xtype) && (column_locality(p, a.colind, s) & 2) != 0;
   const int kp = mrhs_kp(a.k, xtype, loose);
-  void *xr = scratch_alloc(mrhs_xr_bytes(p.ncols, a.k, kp, xtype), s);
+  const size_t xr_bytes = (mrhs_xr_bytes(p.ncols, a.k, kp, xtype) + 255) & ~size_t(255);
+  void *xr = scratch_alloc(xr_bytes + (probe ? 256 : 0), s);
   try {
-    launch_x_rowmajor(xtype, a.x, a.ldx, p.ncols, a.k, kp, xr, s);
+    if (probe) {
+      int *gate = reinterpret_cast<int *>(static_cast<char *>(xr) + xr_bytes);
+      launch_band_probe(p, a, gate, s);
+      a.gate = gate;
+      run_band(p, a, vtype, xtype, ytype, s);
+    }
+    launch_x_rowmajor(xtype, a.x, a.ldx, p.ncols, a.k, kp, xr, a.gate, s);
     a.xr = xr;
     a.ncols = p.ncols;
     a.gshift = tuned_mrhs_gshift();

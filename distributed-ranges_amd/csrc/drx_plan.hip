@@ -238,6 +238,7 @@ Plan *make_plan(int itype, const void *rowptr, int64_t base, int64_t nrows,
       p->rec_mem = block_alloc(static_cast<size_t>(most) * sizeof(BlockRec));
       const int64_t lmax = analyse(*p, validate, s);
       if (fill) p->lmax = lmax;
+      if (fill && nnz > 0) p->slot = slot_alloc(p->device);
     } else {
       DRX_HIP(hipMallocAsync(&p->rec_mem,
                              static_cast<size_t>(records_needed(nnz, p->block_nnz)) *
@@ -277,7 +278,7 @@ void free_plan(Plan *p, hipStream_t s) {
   if (!p) return;
   if (p->panels) free_panels(p->panels);
   if (!p->owns_async)
-    owned_free(p->device, {p->rec_mem});
+    slot_free(p->device, p->slot, owned_free(p->device, {p->rec_mem}));
   else if (p->rec_mem)
     (void)hipFreeAsync(p->rec_mem, s);
   delete p;

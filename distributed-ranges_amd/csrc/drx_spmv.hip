@@ -300,13 +300,15 @@ static void run_spmv_impl(const Plan &p, int vtype, const void *colind,
   // entries per row, is faster through chunks at every k).
   const int mr = p.no_scratch ? 0 : tuned_mrhs();
   const bool stencil = k <= 4 && p.nnz <= 8 * p.nrows;
+  const BandChoice band =
+      MODE == kPlain && k >= 2 && mr == 1 ? band_mrhs(p, a, xtype, s) : kBandNo;
+  if (band == kBandYes) {
+    run_band(p, a, vtype, xtype, ytype, s);
+    return;
+  }
   if (k >= 2 && mr != 0 &&
       (mr == 2 || !stencil || (column_locality(p, colind, s) & 1) == 0)) {
-    if (MODE == kPlain && mr == 1 && band_mrhs(p, a, xtype, s)) {
-      run_band(p, a, vtype, xtype, ytype, s);
-      return;
-    }
-    run_mrhs(p, a, MODE, vtype, xtype, ytype, s);
+    run_mrhs(p, a, MODE, vtype, xtype, ytype, band == kBandProbe, s);
     return;
   }
   // Staging each block's x window in LDS (one right-hand side) only when

@@ -73,10 +73,19 @@ const char *drx_last_error(void);
  *                 stream (scratch from a per-device pool the library keeps)
  *                 and gathers one contiguous vector per entry; 0 gathers the
  *                 k columns of x directly (no scratch); 1 (default) chunks
- *                 except for k <= 4 over short rows (<= 8 entries on
- *                 average) with local columns (stencils; locality detected
- *                 once per colind pointer with one small kernel and a wait
- *                 on the stream).
+ *                 except for wide bands ("mrhs_band") and for k <= 4 over
+ *                 short rows (<= 8 entries on average) with local columns
+ *                 (stencils; locality detected once per colind pointer with
+ *                 one small kernel and a wait on the stream).
+ *   "mrhs_band"   k >= 2 of plain shares with "mrhs" 1: the wide-band kernel,
+ *                 which copies the columns that eight rows span into LDS
+ *                 piece by piece. 1 (default) for rows of much the same
+ *                 length, at least 384 entries on average (480 for k > 8 in
+ *                 FP32; 96 for shares of at most 8192 rows), whose neighbours
+ *                 hold neighbouring columns. That is found out on the GPU by
+ *                 the first call on a colind pointer, without a wait; under
+ *                 capture such a call takes the chunks. 2 wherever it can run
+ *                 (x below 4 GiB), 0 never.
  *   "mrhs_gshift" lane-group shift of the k >= 2 kernel, 0..3 (default 1, and 0:
  *                 10 to 20 entries of a row per lane, in up to four partial
  *                 sums of 2.5 to 5; 2 and 3: two and four times as many in

@@ -351,6 +351,148 @@ def test_multi_rhs_wide_band(orc, vdt, xdt, m, k, order):
     Ad.close()
 
 
+@pytest.mark.parametrize("vdt,xdt", [(torch.float64, torch.float64), (torch.float32, torch.float32),
+                                     (torch.bfloat16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("m,k,kind", [(1, 2, "band"), (9, 3, "span"), (203, 8, "shuffled"),
+                                      (640, 5, "span"), (650, 16, "short"), (75, 13, "far"),
+                                      (75, 2, "far"), (16, 19, "long")])
+def test_wide_band_kernel_forms(orc, vdt, xdt, m, k, kind):
+    """The wide-band kernel itself (knob mrhs_band 2) over everything that it
+    accepts: one row, last groups of fewer than eight rows, empty rows, columns
+    out of order within a row, a row in every other group that spans the whole
+    matrix (other rows' entries wait in registers over many pieces), rows too
+    few and far apart for pieces (x from memory), rows summed by 32 lanes and
+    rows in four partial sums; infinite and NaN x reach the rows that hold their
+    columns and no others."""
+    rng = np.random.default_rng(m + k)
+    n, hw = (200_000, 100_000) if kind == "far" else (20_000, 1500)
+    lo, hi = {"short": (60, 150), "far": (0, 4), "long": (2000, 2900)}.get(kind, (300, 700))
+    rows = []
+    for i in range(m):
+        c0 = i * (n - 2 * hw) // m
+        L = 0 if i in (4, 5) else int(rng.integers(lo, hi))
+        c = np.sort(rng.choice(np.arange(c0, c0 + 2 * hw), L, replace=False))
+        if kind == "shuffled" and i % 3 == 0:
+            c[1:-1] = rng.permutation(c[1:-1])
+        if kind == "span" and i % 16 == 7:
+            c[0], c[-1] = 0, n - 1
+        rows.append(c)
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in rows])]).astype(np.int64)
+    ci = np.concatenate(rows).astype(np.int64)
+    Ad = upload(rp, ci, rng.uniform(-1, 1, ci.size), (m, n))
+    vq = Ad.vals.to(vdt)
+    x = torch.as_tensor(rng.uniform(-1, 1, (k, n))).to(DEV).to(xdt)
+    ydt = torch.float64 if vdt == torch.float64 else torch.float32
+    y0 = torch.rand(k, m + 5, device=DEV, dtype=ydt)
+    y = y0.clone()
+    with drx.tuned(mrhs_band=2):
+        Ad.matvec(x, y=y, vals=vq, alpha=2.0, beta=-0.5)
+        torch.cuda.synchronize()
+        ys, absy = orc.spmv(rp, ci, vq.double().cpu().numpy(), x.double().cpu().numpy())
+        got, was = y.double().cpu().numpy(), y0.double().cpu().numpy()
+        want, den = 2.0 * ys - 0.5 * was[:, :m], 2.0 * absy + 0.5 * was[:, :m]
+        # at least 32 lanes add a row's products (fused), then two levels of
+        # partial sums and six of lanes; alpha, beta and their sum
+        u = 2.0 ** (-53 if ydt == torch.float64 else -24)
+        assert (np.abs(got[:, :m] - want) <= (hi / 32 + 14) * u * den + 1e-300).all()
+        assert np.array_equal(got[:, m:], was[:, m:])
+        cs = [int(ci[0]), int(ci[ci.size // 2])]
+        x[0, cs[0]], x[k - 1, cs[1]] = float("inf"), float("nan")
+        z = Ad.matvec(x, y=y0.clone(), vals=vq, alpha=2.0, beta=-0.5).double().cpu().numpy()
+    for j, c in ((0, cs[0]), (k - 1, cs[1])):
+        hit = np.unique(np.repeat(np.arange(m), np.diff(rp))[ci == c])
+        assert np.array_equal(np.flatnonzero(~np.isfinite(z[j])), hit)
+        rest = np.setdiff1d(np.arange(m), hit)
+        assert np.array_equal(z[j][rest], got[j][rest])
+    if k > 2:
+        assert np.array_equal(z[1:k - 1], got[1:k - 1])
+    Ad.close()
+
+
+def test_wide_band_choice():
+    """A band takes the wide-band kernel and random columns the row blocks, from
+    the first call on and bit for bit the same in later ones, whichever stream
+    and column array the plan's calls alternate between; a capture takes the
+    row blocks where no call came before it, and else what those calls take."""
+    m, L, k = 4000, 400, 4
+    rng = np.random.default_rng(3)
+    rp = torch.arange(m + 1, dtype=torch.int32, device=DEV) * L
+    band = torch.as_tensor((np.arange(m)[:, None] + np.arange(L)).astype(np.int32).reshape(-1))
+    rand = torch.as_tensor(np.sort(rng.integers(0, m + L, (m, L)), axis=1).astype(np.int32).reshape(-1))
+    v = torch.as_tensor(rng.uniform(-1, 1, m * L).astype(np.float32)).to(DEV)
+    x = torch.as_tensor(rng.uniform(-1, 1, (k, m + L)).astype(np.float32)).to(DEV)
+
+    def mk(ci):
+        return drx.CsrMatrix(rp, ci.to(DEV), v, (m, m + L))
+
+    want, other = {}, {}
+    for name, ci in (("band", band), ("rand", rand)):
+        A = mk(ci)
+        with drx.tuned(mrhs_band=2):
+            a = A.matvec(x)
+        with drx.tuned(mrhs_band=0):
+            b = A.matvec(x)
+        assert not torch.equal(a, b)
+        want[name], other[name] = (a, b) if name == "band" else (b, a)
+        for _ in range(3):  # the first call asks, later ones know
+            assert torch.equal(A.matvec(x), want[name])
+            torch.cuda.synchronize()
+        A.close()
+    # one plan, two column arrays in turn, on two streams at once
+    A = mk(band)
+    other_ci, first_ci = rand.to(DEV), A.colind
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    out = []
+    torch.cuda.synchronize()
+    for i in range(12):
+        A.colind = (first_ci, other_ci)[i % 2]
+        with torch.cuda.stream(streams[i % 2]):
+            out.append(A.matvec(x))
+    torch.cuda.synchronize()
+    for i, y in enumerate(out):
+        assert torch.equal(y, want[("band", "rand")[i % 2]])
+    A.colind = first_ci
+    A.close()
+    for before in (False, True):
+        A = mk(band)
+        y = torch.empty(k, m, device=DEV)
+        if before:
+            A.matvec(x)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            A.matvec(x, y=y)
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            eager = A.matvec(x)
+            torch.cuda.synchronize()
+            assert torch.equal(y, want["band"] if before else other["band"])
+            assert torch.equal(eager, want["band"])
+        del g
+        A.close()
+
+
+def test_first_product_of_long_rows_does_not_wait():
+    """The first product of several right-hand sides on a column array returns
+    while the stream is still busy."""
+    m, L = 3000, 400
+    rp = torch.arange(m + 1, dtype=torch.int32, device=DEV) * L
+    ci = (torch.arange(m, device=DEV)[:, None] + torch.arange(L, device=DEV)).int().reshape(-1)
+    x = torch.rand(4, m + L, device=DEV)
+    drx.CsrMatrix(rp, ci, torch.rand(m * L, device=DEV), (m, m + L)).matvec(x)  # (loads the kernels)
+    A = drx.CsrMatrix(rp, ci.clone(), torch.rand(m * L, device=DEV), (m, m + L))
+    y = torch.empty(4, m, device=DEV)
+    torch.cuda.synchronize()
+    busy = torch.cuda.Event()
+    torch.cuda._sleep(100_000_000)
+    busy.record()
+    A.matvec(x, y=y)
+    assert not busy.query()
+    torch.cuda.synchronize()
+    A.close()
+
+
 @pytest.mark.parametrize("itype", [torch.int32, torch.int64])
 @pytest.mark.parametrize("cut", [0, 37])
 @pytest.mark.parametrize("k", [2, 7, 16, 19])
