@@ -318,9 +318,7 @@ __global__ void __launch_bounds__(64 * WM * WN)
     __syncthreads();
   }
 
-  // Epilogue: element v of the lane holds D[Mfma<T>::row(g, v)][r] of each
-  // MFMA tile. beta == 0 does not read C (so C may hold anything, NaN
-  // included), as in BLAS.
+  // A part of a tile: its sums, to the workspace.
   if (part.slot >= 0) {
     T *p = ws + part.slot * (BM * BN);
 #pragma unroll
@@ -738,6 +736,14 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
 // four-wave workgroup per CU, 0.45 of the rate of three), and the cut tiles'
 // sums are written and read once more.
 constexpr int64_t kLeastStages = 4;
+// A product with cut tiles takes at least kCutLeast: two launches and a
+// workspace from the pool take the host 29..33 us, a single launch 18 (one call
+// after another; the model overstates tiles this small). Tiles across column n
+// take their last stage with checks, kEdge more. us per call before cuts / all
+// that the model without these two cut / now: FP32 512 x 512 x 128 22 / 33 / 21,
+// x 224 29 / 33 / 28, x 400 42 / 33 / 33, 500 x 499 x 200 47 / 32 / 32; FP64
+// 512 x 512 x 96 27 / 30 / 27, x 160 36 / 30 / 30.
+constexpr double kCutLeast = 45.0, kEdge = 12.0;
 struct GemmCost {
   int waves;     // per SIMD and workgroup
   int resident;  // workgroups per CU
@@ -751,7 +757,7 @@ inline double gemm_time_us(int64_t units, int64_t parts, double tile_us, int64_t
   return static_cast<double>(per_cu) / static_cast<double>(parts) * tile_us / kEff[waves];
 }
 inline GemmGrid gemm_grid(int64_t m, int64_t n, int64_t k, int bm, int bn, int bk, size_t esz,
-                          int64_t cus, const GemmCost &c, double *cost_us = nullptr) {
+                          int64_t cus, const GemmCost &c) {
   GemmGrid g{};
   g.tiles_m = (m + bm - 1) / bm;
   g.tiles_n = (n + bn - 1) / bn;
@@ -760,18 +766,18 @@ inline GemmGrid gemm_grid(int64_t m, int64_t n, int64_t k, int bm, int bn, int b
   const double tile_us = 2e-6 * bm * bn * static_cast<double>(nk * bk) / c.rate;
   g.main = tiles;
   g.parts = 1;
-  double best = gemm_time_us(tiles, 1, tile_us, cus, c);
+  double best = gemm_time_us(tiles, 1, tile_us, cus, c) + (n % bn != 0 ? kEdge : 0.0);
   const double before = static_cast<double>(whole) / static_cast<double>(cus) * tile_us;
   for (int64_t p = 2; rest > 0 && p <= std::min<int64_t>(64, nk / kLeastStages); p++) {
     const double bytes = 2.0 * static_cast<double>(rest * p) * bm * bn * static_cast<double>(esz);
-    const double t = before + gemm_time_us(rest * p, p, tile_us, cus, c) + 6.0 + bytes / 4e6;
+    const double t = std::max(
+        kCutLeast, before + gemm_time_us(rest * p, p, tile_us, cus, c) + 6.0 + bytes / 4e6);
     if (t < best) {
       best = t;
       g.main = whole;
       g.parts = static_cast<int>(p);
     }
   }
-  if (cost_us) *cost_us = best;
   g.main_xcd = (g.main + kXcds - 1) / kXcds;
   g.tail_xcd = ((tiles - g.main) * g.parts + kXcds - 1) / kXcds;
   DRX_REQUIRE((g.main_xcd + g.tail_xcd) * kXcds <= int64_t(0xffffffff),

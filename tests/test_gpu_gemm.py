@@ -8,6 +8,8 @@ Small-integer inputs, whose every partial sum is exact in the working type,
 must match the oracle bit for bit; they pin the MFMA operand and result
 layouts independently of rounding.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -201,3 +203,29 @@ def test_gemm_in_parts_captured():
         other = drx.gemm(-a, b)
         torch.cuda.synchronize()
         assert torch.equal(c, eager) and torch.equal(other, -c)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("m,n,k,cut", [(96, 96, 96, False), (512, 512, 96, False),
+                                       (256, 256, 128, False), (1024, 1024, 128, False),
+                                       (203, 295, 4502, True), (1000, 1000, 1000, True)])
+def test_gemm_small_products_take_one_launch(dtype, m, n, k, cut):
+    """Products that one launch serves as fast as two launches and a workspace
+    are recorded as one graph node; products worth cutting as several."""
+    hip = ctypes.CDLL([ln.split()[-1] for ln in open("/proc/self/maps") if "libamdhip64" in ln][0])
+    a = torch.randn(m, k, device=DEV, dtype=dtype)
+    b = torch.randn(k, n, device=DEV, dtype=dtype)
+    c = drx.gemm(a, b)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        drx.gemm(a, b, c, beta=0.0)
+    nodes = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(nodes)) == 0
+    assert (nodes.value > 1) == cut
+    g.instantiate()
+    for _ in range(3):
+        c.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, drx.gemm(a, b))
