@@ -756,6 +756,12 @@ inline double gemm_time_us(int64_t units, int64_t parts, double tile_us, int64_t
   const int64_t waves = std::min<int64_t>(4, std::min<int64_t>(per_cu, c.resident) * c.waves);
   return static_cast<double>(per_cu) / static_cast<double>(parts) * tile_us / kEff[waves];
 }
+inline void fill_grid(GemmGrid &g) {
+  g.main_xcd = (g.main + kXcds - 1) / kXcds;
+  g.tail_xcd = ((g.tiles_m * g.tiles_n - g.main) * g.parts + kXcds - 1) / kXcds;
+  DRX_REQUIRE((g.main_xcd + g.tail_xcd) * kXcds <= int64_t(0xffffffff),
+              "product too large for one launch");
+}
 inline GemmGrid gemm_grid(int64_t m, int64_t n, int64_t k, int bm, int bn, int bk, size_t esz,
                           int64_t cus, const GemmCost &c) {
   GemmGrid g{};
@@ -778,10 +784,14 @@ inline GemmGrid gemm_grid(int64_t m, int64_t n, int64_t k, int bm, int bn, int b
       g.parts = static_cast<int>(p);
     }
   }
-  g.main_xcd = (g.main + kXcds - 1) / kXcds;
-  g.tail_xcd = ((tiles - g.main) * g.parts + kXcds - 1) / kXcds;
-  DRX_REQUIRE((g.main_xcd + g.tail_xcd) * kXcds <= int64_t(0xffffffff),
-              "product too large for one launch");
+  fill_grid(g);
+  return g;
+}
+// The same product without cut tiles.
+inline GemmGrid whole_grid(GemmGrid g) {
+  g.main = g.tiles_m * g.tiles_n;
+  g.parts = 1;
+  fill_grid(g);
   return g;
 }
 
@@ -807,15 +817,23 @@ inline int gemm_cus() {
 template <typename T, int BM, int BN, int BK, typename Launch>
 void launch_tiles(int64_t m, int64_t n, int64_t k, T alpha, T beta, T *c, int64_t ldc,
                   const GemmCost &cost, hipStream_t s, Launch &&kernel) {
-  const GemmGrid g = gemm_grid(m, n, k, BM, BN, BK, sizeof(T), gemm_cus(), cost);
+  GemmGrid g = gemm_grid(m, n, k, BM, BN, BK, sizeof(T), gemm_cus(), cost);
+  int64_t cut = g.tiles_m * g.tiles_n - g.main;
+  T *ws = nullptr;
+  if (cut > 0) {
+    ws = static_cast<T *>(
+        scratch_try(static_cast<size_t>(cut) * g.parts * BM * BN * sizeof(T), s));
+    if (ws == nullptr) {  // no memory: all tiles whole
+      g = whole_grid(g);
+      cut = 0;
+    }
+  }
   const dim3 grid(static_cast<unsigned>((g.main_xcd + g.tail_xcd) * kXcds));
-  const int64_t cut = g.tiles_m * g.tiles_n - g.main;
   if (cut == 0) {
-    kernel(grid, g, static_cast<T *>(nullptr));
+    kernel(grid, g, ws);
     DRX_HIP(hipGetLastError());
     return;
   }
-  T *ws = static_cast<T *>(scratch_alloc(static_cast<size_t>(cut) * g.parts * BM * BN * sizeof(T), s));
   try {
     kernel(grid, g, ws);
     const int64_t blocks = std::min<int64_t>(cut * (BM * BN / 256), 8192);

@@ -22,6 +22,7 @@ static std::atomic<int64_t> g_block_nnz{0};
 static std::atomic<int> g_mrhs{1};
 static std::atomic<int> g_mrhs_gshift{1};
 static std::atomic<int> g_mrhs_band{1};
+static std::atomic<int64_t> g_scratch_max{0};
 static std::atomic<int> g_vec{0};
 static std::atomic<int> g_wide{1};
 int tuned_wide() { return g_wide.load(); }
@@ -30,6 +31,7 @@ static std::atomic<int64_t> g_grid_cap{0};
 int tuned_mrhs() { return g_mrhs.load(); }
 int tuned_mrhs_gshift() { return g_mrhs_gshift.load(); }
 int tuned_mrhs_band() { return g_mrhs_band.load(); }
+int64_t tuned_scratch_max() { return g_scratch_max.load(); }
 static std::atomic<int> g_mrhs_kp_max{0};
 int tuned_mrhs_kp_max() { return g_mrhs_kp_max.load(); }
 int tuned_vec() { return g_vec.load(); }
@@ -386,6 +388,9 @@ int drx_tune_set(const char *key, int64_t value) {
     } else if (std::strcmp(key, "mrhs_band") == 0) {
       DRX_REQUIRE(value >= 0 && value <= 2, "mrhs_band must be 0, 1 or 2");
       g_mrhs_band.store(static_cast<int>(value));
+    } else if (std::strcmp(key, "scratch_max") == 0) {
+      DRX_REQUIRE(value >= 0, "scratch_max must not be negative");
+      g_scratch_max.store(value);
     } else if (std::strcmp(key, "mrhs_kp_max") == 0) {
       DRX_REQUIRE(value == 0 || value == 8 || value == 16, "mrhs_kp_max must be 0, 8 or 16");
       g_mrhs_kp_max.store(static_cast<int>(value));
@@ -433,6 +438,8 @@ int drx_tune_get(const char *key, int64_t *value) {
       *value = g_mrhs.load();
     else if (std::strcmp(key, "mrhs_gshift") == 0)
       *value = g_mrhs_gshift.load();
+    else if (std::strcmp(key, "scratch_max") == 0)
+      *value = g_scratch_max.load();
     else if (std::strcmp(key, "mrhs_band") == 0)
       *value = g_mrhs_band.load();
     else if (std::strcmp(key, "vec") == 0)

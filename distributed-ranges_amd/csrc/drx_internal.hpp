@@ -118,6 +118,10 @@ int tuned_rowgather();
 // Stream-ordered scratch from the library's per-device pool, which keeps up to
 // kPoolKeep bytes (and the reserves below) of unused memory.
 void *scratch_alloc(size_t bytes, hipStream_t s);
+// The same for a product that has another way without: null where there is no
+// memory, or more than the knob scratch_max allows is asked for.
+void *scratch_try(size_t bytes, hipStream_t s);
+int64_t tuned_scratch_max();
 void scratch_free(void *p, hipStream_t s);
 // An object whose products take `bytes` of scratch at once: scratch_reserve
 // brings the pool to that size (so that its first product does not pay for
@@ -132,6 +136,9 @@ void scratch_unreserve(int dev, size_t bytes);
 // (dev < 0: the current device; block_free and owned_free take the same one.)
 void *block_alloc(size_t bytes, int dev = -1);
 void block_free(int dev, void *p);
+size_t blocks_kept(int dev);  // bytes kept for reuse
+// Gives all memory that nothing uses on the current device back to the driver.
+void release_memory();
 // Blocks that any stream may have used: waits for the device, as hipFree does.
 // Where the runtime refuses the wait (a stream is being captured) they stay
 // aside until a later one succeeds.
@@ -184,7 +191,8 @@ void run_spmv(const Plan &p, int vtype, const void *colind, const void *vals,
               int64_t ldy, int64_t k, double alpha, double beta,
               hipStream_t s);
 
-void run_spmv_panels(const Plan &p, int vtype, const void *colind,
+// The product over slices; false: no memory for its segment sums, nothing done.
+bool run_spmv_panels(const Plan &p, int vtype, const void *colind,
                      const void *vals, int xtype, const void *x, int64_t ldx,
                      int ytype, void *y, int64_t ldy, int64_t k, double alpha,
                      double beta, hipStream_t s);

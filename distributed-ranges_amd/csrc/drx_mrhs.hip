@@ -38,6 +38,8 @@ static std::mutex g_pool_mu;
 static hipMemPool_t g_pools[kMaxDevices];
 static std::multiset<size_t> g_reserved[kMaxDevices];
 
+static bool blocks_release(int dev);  // gives the kept blocks back; whether any
+
 static hipMemPool_t pool_for(int dev) {
   std::lock_guard<std::mutex> lk(g_pool_mu);
   DRX_REQUIRE(dev >= 0 && dev < kMaxDevices, "device ordinal out of range");
@@ -56,12 +58,38 @@ static hipMemPool_t pool_for(int dev) {
   return g_pools[dev];
 }
 
-void *scratch_alloc(size_t bytes, hipStream_t s) {
+// null: out of memory (a limit of the caller's choice, or the device's).
+static void *pool_alloc(size_t bytes, hipStream_t s) {
   int dev = 0;
   DRX_HIP(hipGetDevice(&dev));
+  const hipMemPool_t pool = pool_for(dev);
+  bytes = std::max<size_t>(bytes, 256);
   void *p = nullptr;
-  DRX_HIP(hipMallocFromPoolAsync(&p, std::max<size_t>(bytes, 256), pool_for(dev), s));
+  hipError_t e = hipMallocFromPoolAsync(&p, bytes, pool, s);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    // blocks that nobody uses go back to the driver first (not under capture,
+    // where this allocation takes no memory yet)
+    if (blocks_release(dev)) e = hipMallocFromPoolAsync(&p, bytes, pool, s);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  DRX_HIP(e);
   return p;
+}
+
+void *scratch_alloc(size_t bytes, hipStream_t s) {
+  void *p = pool_alloc(bytes, s);
+  if (p == nullptr) throw Error(DRX_ERR_NOMEM, "no device memory for a product's scratch");
+  return p;
+}
+
+void *scratch_try(size_t bytes, hipStream_t s) {
+  const int64_t most = tuned_scratch_max();
+  if (most > 0 && bytes > static_cast<size_t>(most)) return nullptr;
+  return pool_alloc(bytes, s);
 }
 
 void scratch_free(void *p, hipStream_t s) {
@@ -130,6 +158,18 @@ void *block_alloc(size_t bytes, int dev) {
   void *p = nullptr;
   DRX_HIP(static_cast<hipError_t>(g_blocks[dev].take(bytes, &p)));
   return p;
+}
+
+static bool blocks_release(int dev) { return g_blocks[dev].release(); }
+size_t blocks_kept(int dev) { return g_blocks[dev].kept(); }
+
+void release_memory() {
+  int dev = 0;
+  DRX_HIP(hipGetDevice(&dev));
+  DRX_REQUIRE(dev >= 0 && dev < kMaxDevices, "device ordinal out of range");
+  (void)blocks_release(dev);
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  if (g_pools[dev]) (void)HipMemory::cleared(hipMemPoolTrimTo(g_pools[dev], 0));
 }
 
 void block_free(int dev, void *p) {

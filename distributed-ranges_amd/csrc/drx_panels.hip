@@ -465,8 +465,9 @@ void check_panel_operands(const Plan &p, int vtype, const void *colind,
               "from: pass those pointers (drx_plan_update_values re-packs new values)");
 }
 
+// false: no memory for the sums (nothing is launched then).
 template <typename TV, typename TX, typename TA>
-static void run_slices(const Plan &p, const PanelSet &ps, const TX *x, int64_t ldx, TA *y,
+static bool run_slices(const Plan &p, const PanelSet &ps, const TX *x, int64_t ldx, TA *y,
                        int64_t ldy, int64_t k, double alpha, double beta, hipStream_t s) {
   SliceArgs a{};
   a.pcol = ps.pcol;
@@ -489,7 +490,8 @@ static void run_slices(const Plan &p, const PanelSet &ps, const TX *x, int64_t l
   // in the type that the sums have, as the other products take them
   b.alpha = static_cast<double>(static_cast<TA>(alpha));
   b.beta = static_cast<double>(static_cast<TA>(beta));
-  void *sums = scratch_alloc(ps.scratch, s);
+  void *sums = scratch_try(static_cast<size_t>(ps.nseg) * sizeof(TA), s);
+  if (sums == nullptr) return false;
   try {
     a.sums = sums;
     b.sums = sums;
@@ -511,9 +513,10 @@ static void run_slices(const Plan &p, const PanelSet &ps, const TX *x, int64_t l
     throw;
   }
   scratch_free(sums, s);
+  return true;
 }
 
-void run_spmv_panels(const Plan &p, int vtype, const void *colind,
+bool run_spmv_panels(const Plan &p, int vtype, const void *colind,
                      const void *vals, int xtype, const void *x, int64_t ldx,
                      int ytype, void *y, int64_t ldy, int64_t k, double alpha,
                      double beta, hipStream_t s) {
@@ -523,10 +526,10 @@ void run_spmv_panels(const Plan &p, int vtype, const void *colind,
   DRX_REQUIRE(k == 1 || (ldx >= p.ncols && ldy >= p.nrows), "ldx/ldy too small");
   DRX_REQUIRE(static_cast<uint64_t>(p.ncols) * dtype_size(xtype) < (uint64_t(1) << 32),
               "the panel layout needs ncols * sizeof(x) < 4 GiB");
-  if (p.nrows == 0) return;
+  if (p.nrows == 0) return true;
   DRX_REQUIRE(ytype == DRX_F64 || ytype == DRX_F32, "unsupported ytype");
   if (p.nnz == 0) {
-    if (beta == 1.0) return;
+    if (beta == 1.0) return true;
     if (ytype == DRX_F64)
       hipLaunchKernelGGL(k_scale_y<double>, grid_of(p.nrows * k), dim3(256), 0, s,
                          static_cast<double *>(y), p.nrows, ldy, k, beta);
@@ -534,26 +537,25 @@ void run_spmv_panels(const Plan &p, int vtype, const void *colind,
       hipLaunchKernelGGL(k_scale_y<float>, grid_of(p.nrows * k), dim3(256), 0, s,
                          static_cast<float *>(y), p.nrows, ldy, k, beta);
     DRX_HIP(hipGetLastError());
-    return;
+    return true;
   }
   DRX_REQUIRE(x != nullptr, "colind/vals/x is null");
 #define DRX_RS(TV, TX, TA)                                                     \
-  run_slices<TV, TX, TA>(p, ps, static_cast<const TX *>(x), ldx,               \
+  return run_slices<TV, TX, TA>(p, ps, static_cast<const TX *>(x), ldx,               \
                          static_cast<TA *>(y), ldy, k, alpha, beta, s)
   if (vtype == DRX_F64 && xtype == DRX_F64 && ytype == DRX_F64)
     DRX_RS(double, double, double);
-  else if (vtype == DRX_F32 && xtype == DRX_F32 && ytype == DRX_F32)
+  if (vtype == DRX_F32 && xtype == DRX_F32 && ytype == DRX_F32)
     DRX_RS(float, float, float);
-  else if (vtype == DRX_BF16 && xtype == DRX_BF16 && ytype == DRX_F32)
+  if (vtype == DRX_BF16 && xtype == DRX_BF16 && ytype == DRX_F32)
     DRX_RS(bf16, bf16, float);
-  else if (vtype == DRX_F16 && xtype == DRX_F16 && ytype == DRX_F32)
+  if (vtype == DRX_F16 && xtype == DRX_F16 && ytype == DRX_F32)
     DRX_RS(f16, f16, float);
-  else if (vtype == DRX_BF16 && xtype == DRX_F32 && ytype == DRX_F32)
+  if (vtype == DRX_BF16 && xtype == DRX_F32 && ytype == DRX_F32)
     DRX_RS(bf16, float, float);
-  else if (vtype == DRX_F16 && xtype == DRX_F32 && ytype == DRX_F32)
+  if (vtype == DRX_F16 && xtype == DRX_F32 && ytype == DRX_F32)
     DRX_RS(f16, float, float);
-  else
-    throw Error(DRX_ERR_UNSUPPORTED, "unsupported (vtype, xtype, ytype)");
+  throw Error(DRX_ERR_UNSUPPORTED, "unsupported (vtype, xtype, ytype)");
 #undef DRX_RS
 }
 

@@ -366,14 +366,14 @@ void run_spmv(const Plan &p, int vtype, const void *colind, const void *vals,
               int64_t ldy, int64_t k, double alpha, double beta,
               hipStream_t s) {
   // Column panels serve k = 1 (one column after another where row-major
-  // chunks of x are off); with k >= 2 the product runs over the share's own
-  // arrays.
-  if (p.panels && (k == 1 || tuned_mrhs() == 0)) {
-    run_spmv_panels(p, vtype, colind, vals, xtype, x, ldx, ytype, y, ldy, k,
-                    alpha, beta, s);
-    return;
+  // chunks of x are off); with k >= 2, and where there is no memory for the
+  // segment sums, the product runs over the share's own arrays.
+  if (p.panels) {
+    check_panel_operands(p, vtype, colind, vals);
+    if ((k == 1 || tuned_mrhs() == 0) &&
+        run_spmv_panels(p, vtype, colind, vals, xtype, x, ldx, ytype, y, ldy, k, alpha, beta, s))
+      return;
   }
-  if (p.panels) check_panel_operands(p, vtype, colind, vals);
   run_spmv_impl<kPlain>(p, vtype, colind, vals, nullptr, xtype, x,
                         ldx, ytype, y, ldy, k, alpha, beta, s);
 }

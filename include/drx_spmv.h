@@ -86,6 +86,11 @@ const char *drx_last_error(void);
  *                 the first call on a colind pointer, without a wait; under
  *                 capture such a call takes the chunks. 2 wherever it can run
  *                 (x below 4 GiB), 0 never.
+ *   "scratch_max" most bytes of scratch for a product that has a way without:
+ *                 segment sums of column panels (else the share's own arrays
+ *                 are used), parts of dense tiles (else they stay whole). 0
+ *                 (default): no limit. The same ways are taken where the
+ *                 device has no memory left.
  *   "mrhs_gshift" lane-group shift of the k >= 2 kernel, 0..3 (default 1, and 0:
  *                 10 to 20 entries of a row per lane, in up to four partial
  *                 sums of 2.5 to 5; 2 and 3: two and four times as many in
@@ -177,6 +182,11 @@ int drx_plan_create(drx_plan *plan, int itype, const void *rowptr,
  * and panel layouts is kept for later ones, up to 4 GiB per device; where the
  * wait is refused, it is not used again before a later one has succeeded. */
 int drx_plan_destroy(drx_plan plan);
+/* Gives the memory that the library keeps on the current device for reuse, and
+ * that nothing uses, back to the driver: that of destroyed objects (up to 4 GiB)
+ * and the scratch pool's (up to 8 GiB and the largest panel layout's sums). The
+ * library does so itself when one of its allocations fails. */
+int drx_release_memory(void);
 /* Number of row blocks and the block size the plan uses. */
 int drx_plan_info(drx_plan plan, int64_t *nblocks, int64_t *block_nnz);
 

@@ -854,6 +854,52 @@ def test_panel_slices_captured(orc):
     A.close()
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_products_without_memory_for_scratch(orc, dtype):
+    """Where there is no memory for segment sums or parts of dense tiles (a
+    limit of one byte stands for it), the products take the share's own arrays
+    and whole tiles."""
+    rng = np.random.default_rng(31)
+    rp, ci = _sliced_rows(rng, 131075)
+    m = rp.size - 1
+    wide = np.float64 if dtype == torch.float64 else np.float32
+    A = upload(rp, ci, rng.uniform(-1, 1, ci.size).astype(wide), (m, 131075))
+    x = torch.as_tensor(rng.uniform(-1, 1, 131075).astype(wide)).to(DEV)
+    y0 = torch.rand(m, dtype=dtype, device=DEV)
+    plain = A.matvec(x, y=y0.clone(), alpha=2.0, beta=0.5)
+    A.set_panels()
+    a = torch.randn(203, 4502, dtype=dtype, device=DEV)
+    b = torch.randn(4502, 295, dtype=dtype, device=DEV)
+    cut = drx.gemm(a, b)
+    with drx.tuned(scratch_max=1):
+        assert torch.equal(A.matvec(x, y=y0.clone(), alpha=2.0, beta=0.5), plain)
+        whole = drx.gemm(a, b)
+    ref, absref = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    u = 2.0 ** (-53 if dtype == torch.float64 else -24)
+    for c in (cut, whole):
+        assert float(((c.double() - ref).abs() / absref).max()) <= 2 * 4504 * u
+    assert not torch.equal(cut, whole)
+    A.close()
+
+
+def test_memory_of_closed_matrices_is_given_back():
+    """The memory of a closed matrix is kept for the next one, and given back
+    on request."""
+    drx.release_memory()
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    A = drx.gen.uniform_rows_csr(400_000, 400_000, 10, 60, seed=3)
+    A.transpose()
+    A.close()
+    del A
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    kept = before - torch.cuda.mem_get_info()[0]
+    drx.release_memory()
+    left = before - torch.cuda.mem_get_info()[0]
+    assert kept > 100 << 20 and left < 16 << 20
+
+
 @pytest.mark.parametrize("vdt", [torch.float64, torch.float32])
 def test_panel_slices_sparse_rows(orc, vdt):
     """So few entries over 25M rows and 4M columns that the table of row
