@@ -161,16 +161,6 @@ void *block_alloc(size_t bytes, int dev) {
 }
 
 static bool blocks_release(int dev) { return g_blocks[dev].release(); }
-size_t blocks_kept(int dev) { return g_blocks[dev].kept(); }
-
-void release_memory() {
-  int dev = 0;
-  DRX_HIP(hipGetDevice(&dev));
-  DRX_REQUIRE(dev >= 0 && dev < kMaxDevices, "device ordinal out of range");
-  (void)blocks_release(dev);
-  std::lock_guard<std::mutex> lk(g_pool_mu);
-  if (g_pools[dev]) (void)HipMemory::cleared(hipMemPoolTrimTo(g_pools[dev], 0));
-}
 
 void block_free(int dev, void *p) {
   if (p == nullptr || dev < 0 || dev >= kMaxDevices) return;

@@ -315,10 +315,6 @@ int drx_plan_destroy(drx_plan plan) {
   });
 }
 
-int drx_release_memory(void) {
-  return guarded([] { release_memory(); });
-}
-
 int drx_plan_info(drx_plan plan, int64_t *nblocks, int64_t *block_nnz) {
   return guarded([&] {
     DRX_REQUIRE(plan != nullptr, "plan is null");

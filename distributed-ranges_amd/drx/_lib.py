@@ -42,7 +42,6 @@ SIGNATURES = {
     "drx_plan_create": (c_int, [ctypes.POINTER(c_vp), c_int, c_vp, c_i64, c_i64,
                                 c_i64, c_i64, c_int, c_i64, c_vp]),
     "drx_plan_destroy": (c_int, [c_vp]),
-    "drx_release_memory": (c_int, []),
     "drx_plan_info": (c_int, [c_vp, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64)]),
     "drx_plan_set_panels": (c_int, [c_vp, c_int, c_vp, c_vp, c_i64, c_vp]),
     "drx_plan_update_values": (c_int, [c_vp, c_vp, c_vp]),
@@ -153,12 +152,6 @@ def tune_get(key):
 def tune_set(key, value):
     """Set a process-wide tuning knob (drx_tune_set)."""
     check(lib().drx_tune_set(key.encode(), int(value)))
-
-
-def release_memory():
-    """Give the device memory that the library keeps for reuse, and that
-    nothing uses, back to the driver (drx_release_memory)."""
-    check(lib().drx_release_memory())
 
 
 class tuned:

@@ -179,14 +179,10 @@ int drx_plan_create(drx_plan *plan, int itype, const void *rowptr,
                     drx_stream_t stream);
 /* Waits for the device (destroying an object while a stream is being captured
  * invalidates that capture, as hipFree does). The memory of plans, transposes
- * and panel layouts is kept for later ones, up to 4 GiB per device; where the
- * wait is refused, it is not used again before a later one has succeeded. */
+ * and panel layouts is kept for later ones, up to 4 GiB per device, and given
+ * back when one of the library's allocations fails; where the wait is refused,
+ * it is not used again before a later one has succeeded. */
 int drx_plan_destroy(drx_plan plan);
-/* Gives the memory that the library keeps on the current device for reuse, and
- * that nothing uses, back to the driver: that of destroyed objects (up to 4 GiB)
- * and the scratch pool's (up to 8 GiB and the largest panel layout's sums). The
- * library does so itself when one of its allocations fails. */
-int drx_release_memory(void);
 /* Number of row blocks and the block size the plan uses. */
 int drx_plan_info(drx_plan plan, int64_t *nblocks, int64_t *block_nnz);
 
