@@ -136,6 +136,7 @@ void scratch_unreserve(int dev, size_t bytes);
 // (dev < 0: the current device; block_free and owned_free take the same one.)
 void *block_alloc(size_t bytes, int dev = -1);
 void block_free(int dev, void *p);
+size_t blocks_kept(int dev);  // bytes kept for reuse
 // Blocks that any stream may have used: waits for the device, as hipFree does.
 // Where the runtime refuses the wait (a stream is being captured) they stay
 // aside until a later one succeeds.

@@ -161,6 +161,7 @@ void *block_alloc(size_t bytes, int dev) {
 }
 
 static bool blocks_release(int dev) { return g_blocks[dev].release(); }
+size_t blocks_kept(int dev) { return g_blocks[dev].kept(); }
 
 void block_free(int dev, void *p) {
   if (p == nullptr || dev < 0 || dev >= kMaxDevices) return;

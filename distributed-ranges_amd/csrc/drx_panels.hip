@@ -880,6 +880,44 @@ static void build_panels(Plan &p, PanelSet &ps, const TI *colind, const TV *vals
   for (void *q : tmp) block_free(ps.device, q);
 }
 
+// Slices of panels of `width` columns over ncols columns: groups, and how many
+// slices hold columns (the last panel's may be fewer).
+static void cut_slices(PanelSet &ps, int64_t ncols) {
+  const int64_t slice = ps.vtype == DRX_F64 ? slice_cols<double>() : slice_cols<float>();
+  if (ps.width <= slice) {  // whole panels share a slice
+    ps.group = ps.sw = slice / ps.width * ps.width;
+    ps.spg = 1;
+  } else {  // a panel is cut into equal slices
+    ps.group = ps.width;
+    ps.spg = (ps.width + slice - 1) / slice;
+    ps.sw = (ps.width + ps.spg - 1) / ps.spg;
+  }
+  const int64_t full = ncols / ps.group;
+  ps.ns = std::max<int64_t>(1, full * ps.spg + (ncols - full * ps.group + ps.sw - 1) / ps.sw);
+}
+
+// Whether products are faster over slices than over the share's own arrays.
+// Below some 8M entries the slice kernels' own steps (33 us however few entries)
+// outweigh the gathers, and where a wave's rows hold only a few entries of a
+// slice k_slice_rows reads mostly empty ranges. us per product, random columns,
+// n x n and fewer rows, own arrays / slices:
+//   FP32 n = 600K, 12 and 16 entries per row 46 / 48, 85 / 53; 1.2M, 5 and 8: 43 /
+//   53, 64 / 58; 4M, 4: 236 / 99; 30M, 2 (1.4 entries per wave and slice), 3 (2.1)
+//   and 4 (2.8): 1147 / 1527, 1148 / 1112, 1217 / 893
+//   FP64 n = 1.2M, 5 and 8: 75 / 93, 115 / 103; 12M, 6 (4.2) and 8 (5.6): 1150 /
+//   1196, 1147 / 989; 30M, 2 (0.6) and 16 (4.5): 1212 / 8411, 1147 / 1256
+//   BF16 n = 2M, 3 and 4: 41 / 51, 59 / 54; 30M, 3 (2.1) and 4 (2.8): 1079 / 1088,
+//   1123 / 867
+static bool slices_pay(int vtype, int64_t nnz, int64_t nrows, int64_t ns) {
+  const int64_t rows = vtype == DRX_F64 ? rows_per_wave<double>() : rows_per_wave<float>();
+  const double cells = static_cast<double>((nrows + rows - 1) / rows) * static_cast<double>(ns);
+  return nnz >= 8000000 && static_cast<double>(nnz) >= (vtype == DRX_F64 ? 5.0 : 2.5) * cells;
+}
+
+static int64_t default_width(int vtype) {
+  return std::max<int64_t>(4096, (int64_t(2) << 20) / static_cast<int64_t>(dtype_size(vtype)));
+}
+
 // Builds the panel layout of p (drx_plan_set_panels).
 static void set_panels(Plan &p, int vtype, const void *colind, const void *vals,
                      int64_t panel_cols, hipStream_t s) {
@@ -891,24 +929,11 @@ static void set_panels(Plan &p, int vtype, const void *colind, const void *vals,
   ps->vtype = vtype;
   ps->src_colind = colind;
   ps->src_vals = vals;
-  ps->width = panel_cols > 0 ? panel_cols
-                             : std::max<int64_t>(4096, (int64_t(2) << 20) /
-                                                           static_cast<int64_t>(dtype_size(vtype)));
+  ps->width = panel_cols > 0 ? panel_cols : default_width(vtype);
   ps->npanels = std::max<int64_t>(1, (p.ncols + ps->width - 1) / ps->width);
   try {
     DRX_REQUIRE(ps->npanels <= (int64_t(1) << 20), "too many panels");
-    const int64_t slice = vtype == DRX_F64 ? slice_cols<double>() : slice_cols<float>();
-    if (ps->width <= slice) {  // whole panels share a slice
-      ps->group = ps->sw = slice / ps->width * ps->width;
-      ps->spg = 1;
-    } else {  // a panel is cut into equal slices
-      ps->group = ps->width;
-      ps->spg = (ps->width + slice - 1) / slice;
-      ps->sw = (ps->width + ps->spg - 1) / ps->spg;
-    }
-    // slices that hold columns (the last panel's may be fewer)
-    const int64_t full = p.ncols / ps->group;
-    ps->ns = std::max<int64_t>(1, full * ps->spg + (p.ncols - full * ps->group + ps->sw - 1) / ps->sw);
+    cut_slices(*ps, p.ncols);
     if (p.nnz > 0) {
       int cus = 0;
       DRX_HIP(hipGetDevice(&ps->device));
@@ -978,14 +1003,22 @@ static bool panels_pay(const Plan &p, int vtype, const void *colind, hipStream_t
   if (tuned_auto_panels() == 0) return false;
   if (p.panels != nullptr || p.nnz == 0 || p.nnz > INT32_MAX) return false;
   if (p.ncols * sx <= (int64_t(4) << 20)) return false;          // x fits one XCD's L2
-  if (p.nnz < 4 * p.nrows) return false;                         // y updates would dominate
+  if (p.nnz < 4 * p.nrows) return false;  // too few gathers for a copy of the entries
   if (static_cast<uint64_t>(p.ncols) * sx >= (uint64_t(1) << 32)) return false;
-  // device memory for the copy (entries, permutation, segments, build
-  // scratch): about 4 index arrays and 1 value array of nnz, with a margin
+  PanelSet shape;
+  shape.vtype = vtype;
+  shape.width = default_width(vtype);
+  cut_slices(shape, p.ncols);
+  if (!slices_pay(vtype, p.nnz, p.nrows, shape.ns)) return false;
+  // device memory for the most that building holds at once, with columns so
+  // scattered that every entry is a segment: positions, sorted slices,
+  // permutation, copies, flags, segment numbers, rows and first entries (34
+  // bytes per entry beside the value with 32-bit indices)
   const int64_t si = p.itype == DRX_I32 ? 4 : 8;
   size_t free_b = 0, total_b = 0;
   DRX_HIP(hipMemGetInfo(&free_b, &total_b));
-  if (static_cast<double>(free_b) < 1.25 * static_cast<double>(p.nnz) * (4 * si + sx + 8))
+  free_b += blocks_kept(p.device);
+  if (static_cast<double>(free_b) < 1.1 * static_cast<double>(p.nnz) * (3 * si + 22 + sx))
     return false;
   unsigned long long *d = static_cast<unsigned long long *>(
       scratch_alloc(2 * sizeof(unsigned long long), s));
@@ -1041,7 +1074,12 @@ int drx_plan_auto_panels(drx_plan plan, int vtype, const void *colind,
     DRX_HIP(hipStreamIsCapturing(s, &cs));
     DRX_REQUIRE(cs == hipStreamCaptureStatusNone, "the stream is being captured");
     if (!panels_pay(p, vtype, colind, s)) return;
-    set_panels(p, vtype, colind, vals, 0, s);
+    try {
+      set_panels(p, vtype, colind, vals, 0, s);
+    } catch (const Error &e) {
+      if (e.status != DRX_ERR_NOMEM) throw;
+      return;  // (another user of the device was faster)
+    }
     if (built) *built = 1;
   });
 }

@@ -209,10 +209,12 @@ int drx_plan_panels(drx_plan plan, int64_t *npanels, int64_t *panel_cols,
 /* Builds the panel layout (as drx_plan_set_panels with panel_cols = 0) when
  * it pays, and reports it in *built (1, else 0; may be NULL). It pays when
  * x of vtype exceeds 4 MiB (one XCD's L2), the share averages at least 4
- * entries per row, its columns scatter (fewer than half of the entries
+ * entries per row, holds at least 8M entries, of which the rows of a wave (640;
+ * FP64 512) have on average at least 2.5 (FP64: 5) in a slice, its columns scatter (fewer than half of the entries
  * sampled from up to 2048 row blocks lie within 1 MiB of x of their block's
  * middle column; one small kernel), the share holds at most 2^31 - 1
- * entries and the device has memory for the copy. Synchronizes the stream;
+ * entries and the device has memory for the copy (not built either where that
+ * runs out meanwhile). Synchronizes the stream;
  * refuses a stream under capture. Knob "auto_panels" 0 turns it off. Called
  * by the host interface's share and tile setup (the seams of
  * csr_row_distribution::init, csr_row_distribution.hpp:205-318,

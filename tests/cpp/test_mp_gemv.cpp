@@ -301,4 +301,16 @@ TEST(SparseMatrix, BandShareKeepsPlainCsr) {
   dr::destroy_csr_matrix_view(csr);
 }
 
+// Scattered columns, but too few entries for the panel layout's own steps (4.6M
+// over 1.2M columns): plain CSR, which is the faster one there.
+TEST(SparseMatrix, SmallScatteredShareKeepsPlainCsr) {
+  auto csr = zipf_host(150000, 1200000, 256, 79);
+  EXPECT_TRUE(csr.size() < 8000000);
+  mp::run_ranks(1, [&] {
+    mp::distributed_sparse_matrix<float, int> e(csr, 0);
+    EXPECT_TRUE(e.matrix_distribution().panels() == 0);
+  });
+  dr::destroy_csr_matrix_view(csr);
+}
+
 int main(int argc, char **argv) { return harness::run_all(argc > 1 ? argv[1] : nullptr); }
