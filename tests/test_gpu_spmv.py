@@ -246,6 +246,33 @@ def test_multi_rhs_staged_sums(orc, vdt, k):
     Ad.close()
 
 
+@pytest.mark.parametrize("k", [9, 16])
+@pytest.mark.parametrize("gshift,block_nnz,least", [(0, 4096, 14), (1, 4096, 28), (0, 2048, 13)])
+def test_multi_rhs_staged_sums_in_passes(orc, gshift, block_nnz, least, k):
+    """Blocks of more rows than have their sums staged at once (120), with a row
+    offset in their second and third pass; the last block has fewer."""
+    rng = np.random.default_rng(block_nnz + k)
+    n = 5000
+    lens = rng.integers(least, least + 3, 2000)
+    rp = np.concatenate([[0], np.cumsum(lens)])
+    ci = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens])
+    v = rng.uniform(-1, 1, ci.size).astype(np.float32)
+    m = lens.size
+    A = upload(rp, ci, v, (m, n), block_nnz=block_nnz)
+    x = rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    y0 = rng.uniform(-1, 1, (k, m + 3)).astype(np.float32)
+    y = torch.as_tensor(y0).to(DEV)
+    with drx.tuned(mrhs_gshift=gshift):
+        A.matvec(torch.as_tensor(x).to(DEV), y=y, alpha=2.0, beta=-0.5)
+    got = y.double().cpu().numpy()
+    ys, absy = orc.spmv(rp, ci, v.astype(np.float64), x.astype(np.float64))
+    want, den = 2.0 * ys - 0.5 * y0[:, :m], 2.0 * absy + 0.5 * np.abs(y0[:, :m])
+    # a product and at most least + 2 additions, then alpha, beta and their sum
+    assert (np.abs(got[:, :m] - want) <= (least + 6) * 2.0 ** -24 * den).all()
+    assert np.array_equal(y.cpu().numpy()[:, m:], y0[:, m:])
+    A.close()
+
+
 def _chain_sums(v, x, chains):
     """Sums of the rows of v * x (FP32, products fused) in `chains` chains of
     additions, every chains-th entry, added pairwise."""
