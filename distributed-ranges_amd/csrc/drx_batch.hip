@@ -18,8 +18,8 @@
 // created.
 //
 // Tunables: block_nnz (entries per block, i.e. rows per workgroup), gshift
-// (the lane-group thresholds: a block of mean row length L uses G lanes per
-// row chosen from L >> gshift), wg_per_cu (persistent grid size). The
+// (the lane-group thresholds: k = 1, a block of mean row length L uses G lanes
+// per row chosen from L >> gshift; k >= 2, see mrhs_lanes), wg_per_cu (persistent grid size). The
 // autotuner times every combination on the batch itself.
 #include <hip/hip_runtime.h>
 
@@ -526,7 +526,6 @@ int drx_batch_create(drx_batch *out, int64_t nitems, const drx_batch_item *items
       b->ytype = ytype;
       b->k = k;
       b->mrhs = k >= 2 && tuned_mrhs() != 0;
-      b->gshift = b->mrhs ? tuned_mrhs_gshift() : 0;
       b->kp = b->mrhs ? mrhs_kp(k, xtype, tuned_mrhs_kp_max() == 8) : 0;
       b->alpha = alpha;
       b->beta = beta;

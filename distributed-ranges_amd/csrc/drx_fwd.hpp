@@ -899,12 +899,16 @@ __device__ __forceinline__ void load_xrow(const TX *p, TA (&xv)[KP]) {
 // with few lanes per row. RMS error against 64 bits, rows of 50 random entries,
 // FP32, in units of the last place over the root of the squared products: as
 // many lanes with one sum each 1.20, twice as many 1.10, these 1.10.
+// Batches ask for more chains (gshift 0): their blocks tend to mix row lengths, and
+// the longer rows, whose chains are longer than the mean row's, make most of the
+// error (relative error of all outputs, 24 matrices of rows of 3..64 entries, k = 16:
+// 6.55e-8 with 2.5 to 5 entries, 6.45e-8 so; 1726 / 1761 us, one sum per lane 2704).
 struct MrhsLanes {
   int g, ch;  // log2 of the lanes per row, of the partial sums per lane
 };
 template <int MOST> __device__ __forceinline__ MrhsLanes mrhs_lanes(int per_row, int gshift) {
-  // log2 of the chains that give each 2.5 to 5 entries
-  const int t = per_row * 2 / 5;
+  // log2 of the chains that give each 2.5 to 5 entries (gshift 0: 1.6 to 3.1)
+  const int t = gshift > 0 ? per_row * 2 / 5 : per_row * 16 / 25;
   const int c = t < 2 ? 0 : 31 - __builtin_clz(static_cast<unsigned>(t));
   const int fewer = MOST + (gshift > 1 ? gshift - 1 : 0);
   const int g = c > fewer ? c - fewer : 0;

@@ -91,10 +91,10 @@ const char *drx_last_error(void);
  *                 are used), parts of dense tiles (else they stay whole). 0
  *                 (default): no limit. The same ways are taken where the
  *                 device has no memory left.
- *   "mrhs_gshift" lane-group shift of the k >= 2 kernel, 0..3 (default 1, and 0:
- *                 10 to 20 entries of a row per lane, in up to four partial
- *                 sums of 2.5 to 5; 2 and 3: two and four times as many in
- *                 four sums); also of new batches.
+ *   "mrhs_gshift" lane-group shift of the k >= 2 kernel, 0..3 (default 1: 10 to
+ *                 20 entries of a row per lane, in up to four partial sums of
+ *                 2.5 to 5; 2 and 3: two and four times as many in four sums;
+ *                 0: 1.6 to 3.1 entries per sum, which batches start with).
  *   "mrhs_kp_max" widest row-major chunk for 4-byte x: 16, 8, or 0 (default:
  *                 8 for k > 8 over loosely local columns -- stencils,
  *                 bands -- else 16; batches use 16). Fixed per call, and per

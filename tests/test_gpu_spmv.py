@@ -312,6 +312,34 @@ def test_multi_rhs_rounding_error(L, chains, k):
     Ad.close()
 
 
+@pytest.mark.parametrize("k", [4, 16])
+def test_batch_rounding_error(k):
+    """A batch of rows of 3..64 entries: blocks of 26 to 49 entries per row take
+    16 chains. RMS over 320000 sums, at most 0.8 % above that of the same chains
+    on the CPU (8 chains: 1.2 to 1.4 %; standard errors of about 0.2 %)."""
+    m, n, L = 320_000 // k, 50_000, 64
+    rng = np.random.default_rng(k)
+    lens = rng.integers(3, 65, m)
+    held = np.arange(L)[None, :] < lens[:, None]
+    ci = rng.integers(0, n, (m, L))
+    v = np.where(held, rng.uniform(-1, 1, (m, L)), 0).astype(np.float32)
+    x = rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    A = upload(np.concatenate([[0], np.cumsum(lens)]), ci[held], v[held], (m, n))
+    y = torch.empty(k, m, device=DEV)
+    b = drx.Batch(forward=[(A, torch.as_tensor(x).to(DEV), y)], k=k)
+    b.run()
+    torch.cuda.synchronize()
+    y = y.cpu().numpy()
+    got = want = 0.0
+    for j in range(k):
+        p = v.astype(np.float64) * x[j][ci]
+        got += ((y[j] - p.sum(1)) ** 2).sum()
+        want += ((_chain_sums(v, x[j][ci], 16) - p.sum(1)) ** 2).sum()
+    assert got <= 1.008 ** 2 * want
+    b.close()
+    A.close()
+
+
 @pytest.mark.parametrize("k,chains", [(4, 256), (8, 128), (16, 128)])
 def test_wide_band_rounding_error(k, chains):
     """The same over a wide band (1201 columns around the diagonal): as many
