@@ -739,11 +739,15 @@ constexpr int64_t kLeastStages = 4;
 // A product with cut tiles takes at least kCutLeast: two launches and a
 // workspace from the pool take the host 29..33 us, a single launch 18 (one call
 // after another; the model overstates tiles this small). Tiles across column n
-// take their last stage with checks, kEdge more. us per call before cuts / all
-// that the model without these two cut / now: FP32 512 x 512 x 128 22 / 33 / 21,
-// x 224 29 / 33 / 28, x 400 42 / 33 / 33, 500 x 499 x 200 47 / 32 / 32; FP64
-// 512 x 512 x 96 27 / 30 / 27, x 160 36 / 30 / 30.
-constexpr double kCutLeast = 45.0, kEdge = 12.0;
+// take their last stage with checks, kEdge more. us per call, one after another,
+// before cuts / all that the model without these two cut / now: FP32 512 x 512 x 128
+// 22 / 34 / 21, x 224 29 / 33 / 28, x 400 42 / 32 / 32, 500 x 499 x 200 47 / 32 / 34;
+// FP64 512 x 512 x 96 27 / 33 / 27, x 160 36 / 33 / 30. Over 15 sizes and 15 k no
+// call is slower than before cuts by more than 3 % (kCutLeast 45: FP64 128 x 128 x
+// 160 36 us where cut tiles take 29). Single calls that are waited for, whose time
+// on the GPU counts too, would gain from cutting earlier: 41.5 us whatever k, against
+// 45 for 512 x 512 x 96 FP64 and 39 for x 128 FP32 in one launch.
+constexpr double kCutLeast = 40.0, kEdge = 12.0;
 struct GemmCost {
   int waves;     // per SIMD and workgroup
   int resident;  // workgroups per CU
@@ -772,17 +776,23 @@ inline GemmGrid gemm_grid(int64_t m, int64_t n, int64_t k, int bm, int bn, int b
   const double tile_us = 2e-6 * bm * bn * static_cast<double>(nk * bk) / c.rate;
   g.main = tiles;
   g.parts = 1;
-  double best = gemm_time_us(tiles, 1, tile_us, cus, c) + (n % bn != 0 ? kEdge : 0.0);
+  const double uncut = gemm_time_us(tiles, 1, tile_us, cus, c) + (n % bn != 0 ? kEdge : 0.0);
   const double before = static_cast<double>(whole) / static_cast<double>(cus) * tile_us;
+  // the best number of parts first, then whether to cut at all: kCutLeast says
+  // nothing about the parts
+  double best = 0;
+  int parts = 1;
   for (int64_t p = 2; rest > 0 && p <= std::min<int64_t>(64, nk / kLeastStages); p++) {
     const double bytes = 2.0 * static_cast<double>(rest * p) * bm * bn * static_cast<double>(esz);
-    const double t = std::max(
-        kCutLeast, before + gemm_time_us(rest * p, p, tile_us, cus, c) + 6.0 + bytes / 4e6);
-    if (t < best) {
+    const double t = before + gemm_time_us(rest * p, p, tile_us, cus, c) + 6.0 + bytes / 4e6;
+    if (parts == 1 || t < best) {
       best = t;
-      g.main = whole;
-      g.parts = static_cast<int>(p);
+      parts = static_cast<int>(p);
     }
+  }
+  if (parts > 1 && std::max(kCutLeast, best) < uncut) {
+    g.main = whole;
+    g.parts = parts;
   }
   fill_grid(g);
   return g;

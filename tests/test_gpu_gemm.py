@@ -247,3 +247,20 @@ def test_gemm_small_products_stay_whole(dtype, m, n, k, cut):
     with drx.tuned(scratch_max=1):
         whole = drx.gemm(a, b)
     assert torch.equal(c, whole) != cut
+
+
+@pytest.mark.parametrize("m,n,k,parts", [(157, 232, 1147, 17), (300, 200, 2000, 31)])
+def test_gemm_small_products_take_the_best_parts(m, n, k, parts):
+    """Few tiles of long k are cut into many parts (about as many as there are
+    16-deep stages over four). A chain of s steps of four k rounds s / 2 times
+    as much as one addition, and adding p parts p / 2 times: against whole
+    tiles the RMS error is the root of (k / 4p + p) / (k / 4), 0.34 and 0.30
+    here, and 0.5 with four parts."""
+    a = torch.randn(m, k, device=DEV)
+    b = torch.randn(k, n, device=DEV)
+    ref = a.double() @ b.double()
+    cut = drx.gemm(a, b)
+    with drx.tuned(scratch_max=1):
+        whole = drx.gemm(a, b)
+    ratio = float((cut.double() - ref).norm() / (whole.double() - ref).norm())
+    assert ratio <= 1.2 * ((k / 4 / parts + parts) / (k / 4)) ** 0.5
