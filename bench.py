@@ -115,33 +115,10 @@ def headline(steps, warmup):
     torch.cuda.empty_cache()
     gather = {"G_gathers_per_s": round(per / g_ms / 1e6, 1),
               "ms_per_step": round(g_ms * npan, 4),
-              "kernel_frac_of_gather_ceiling": round(g_ms * npan / ev_ms, 4),
+              "times_the_step": round(g_ms * npan / ev_ms, 4),
               "probe": "drx_gather: %d random int32 indices into %d floats (one panel's x "
                        "slice), x %d panels" % (per, width, npan)}
     return A, x, y, B, wall_ms, ev_ms, layout, gather
-
-
-def form_panel_sweep(A, x, steps, widths=(262144, 393216, 524288, 786432, 1048576)):
-    """The headline product through column panels of each requested width
-    (columns of x per panel): time per step and the row segments the layout
-    makes. The kernels cut x into slices that fit into LDS whatever the width
-    asked for, so the times should not differ."""
-    n = A.shape[0]
-    y = torch.empty(n, dtype=torch.float32, device="cuda")
-    B = spmv_bytes(n, A.shape[1], A.nnz, 4, 4, 4, 4)
-    out = []
-    for w in widths:
-        M = drx.CsrMatrix(A.rowptr, A.colind, A.vals, A.shape)
-        npan, width, nseg = M.set_panels(w)
-        _, ms = time_launches(lambda: M.matvec(x, y=y), steps, 2)
-        out.append({"panel_cols": width, "MB_of_x": round(width * 4 / 2**20, 3),
-                    "panels": npan, "row_segments": nseg, "ms_per_step": round(ms, 4),
-                    "GBps": round(B / ms / 1e6, 1)})
-        log("panel sweep: %s" % out[-1])
-        M.close()
-        del M
-        torch.cuda.empty_cache()
-    return out
 
 
 def host_cpu_info():
@@ -540,7 +517,7 @@ def main():
     ap.add_argument("--steps", type=int, default=20)
     ap.add_argument("--warmup", type=int, default=5)
     ap.add_argument("--forms", default="all",
-                    help="all | none | comma list (panel_sweep runs only when listed)")
+                    help="all | none | comma list")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--cpu-seconds", type=float, default=10.0)
     ap.add_argument("--xstage", type=int, default=None,
@@ -595,7 +572,7 @@ def main():
                                "drx::k_slice_rows (segments to rows); achieved = bytes / "
                                "summed time of one step's launches",
                      "ms_per_step_kernels": round(ev_ms, 4),
-                     "gather_ceiling": gather},
+                     "l2_gathers": gather},
     }
     log("stream ceiling ...")
     result["roofline"]["stream_ceiling"] = stream_ceiling()
@@ -612,9 +589,6 @@ def main():
     if "lowprec" in want:
         log("form lowprec ...")
         forms["lowprec"] = form_lowprec(steps_f, zipf=(A, x))
-    if "panel_sweep" in want:
-        log("form panel_sweep ...")
-        forms["panel_sweep"] = form_panel_sweep(A, x, steps_f)
     del A
     torch.cuda.empty_cache()
     if "laplacian2d_f64" in want:
